@@ -398,6 +398,51 @@ struct Cells {
 
 int nbits_for(int64_t n_cells) { return nbits_for_cells(n_cells); }
 
+// Cells of the step, energy and virial kernels: numbered with the last axis
+// fastest, so that a stencil column is one run of the sorted particles.  Any
+// numbering gives the same candidates in the same order.
+template <class Real>
+GridPT<Real> column_grid(GridPT<Real> g, int dim) {
+  g.strides[dim - 1] = 1;
+  for (int a = dim - 2; a >= 0; --a) g.strides[a] = g.strides[a + 1] * g.dims[a + 1];
+  return g;
+}
+
+template <class Real>
+struct Columns {
+  int32_t* perm;
+  int32_t* skeys;
+  int32_t* starts;  // n_cells + 1: first sorted slot of each cell
+  Real4<Real>* spos;
+};
+
+// Hash + sort + cell starts + sorted (x, r) of `pos` on the column grid g.
+template <class Real>
+int build_columns(jdem_ctx* ctx, const Real* pos, const Real* rad, int64_t n, int dim, const DomPT<Real>& dom,
+                  const GridPT<Real>& g, Columns<Real>* out) {
+  const size_t nn = (size_t)(n > 0 ? n : 1);
+  ENSURE(ctx, ctx->wKeys, 4 * nn);
+  ENSURE(ctx, ctx->cstart, 4 * ((size_t)g.n_cells + 1));
+  ENSURE(ctx, ctx->spos, sizeof(Real4<Real>) * nn);
+  uint32_t* hk = (uint32_t*)ctx->wKeys.p;
+  HIPCHK(ctx, launch_hash(pos, n, dim, dom, g, hk, ctx->stream));
+  uint32_t* sk = nullptr;
+  int32_t* perm = nullptr;
+  int32_t* cs = (int32_t*)ctx->cstart.p;
+  if (use_cell_sort_sparse(n, g.n_cells)) {
+    HIPCHK(ctx, cell_sort_pairs(ctx, hk, n, g.n_cells, &sk, &perm, cs, ctx->stream));
+  } else {
+    HIPCHK(ctx, radix_sort_pairs(ctx, hk, n, nbits_for(g.n_cells), &sk, &perm, ctx->stream));
+    HIPCHK(ctx, ws_launch_cell_starts(sk, n, g.n_cells, cs, ctx->stream));
+  }
+  HIPCHK(ctx, launch_gather_spos(perm, pos, rad, n, dim, (Real4<Real>*)ctx->spos.p, ctx->stream));
+  out->perm = perm;
+  out->skeys = (int32_t*)sk;
+  out->starts = cs;
+  out->spos = (Real4<Real>*)ctx->spos.p;
+  return JDEM_OK;
+}
+
 // Hash + sort + cell ranges + sorted (x, r) of `pos` (cell_list.py:37-87);
 // in float64 the kernels read the partners' own arrays and no (x, r) copy
 // is made.
@@ -1411,14 +1456,13 @@ int reject_clumps(jdem_ctx* ctx, const jdem_state& s, const char* what) {
 // Fill the source fields of `a` for the collider (building cells if needed).
 int prepare_source(jdem_ctx* ctx, jdem_system* sys, StepArgs& a, const float* pos) {
   if (sys->collider_kind == JDEM_COLLIDER_CELL_LIST) {
-    Cells c;
-    a.grid = grid_of(sys->grid);
-    int rc = build_cells(ctx, pos, sys->state.rad, sys->state.n, sys->state.dim, a.dom, a.grid, &c);
+    Columns<float> c;
+    a.grid = column_grid(grid_of(sys->grid), sys->state.dim);
+    int rc = build_columns(ctx, pos, sys->state.rad, sys->state.n, sys->state.dim, a.dom, a.grid, &c);
     if (rc) return rc;
     a.perm = c.perm;
     a.skeys = c.skeys;
-    a.cstart = c.cstart;
-    a.cend = c.cend;
+    a.cstart = c.starts;
     a.spos = c.spos;
   }
   return JDEM_OK;
@@ -2699,15 +2743,14 @@ int nl_check_and_rebuild64(jdem_ctx* ctx, jdem_system_f64* sys) {
 
 int prepare_source64(jdem_ctx* ctx, const jdem_system_f64* sys, StepArgs64& a, const double* pos) {
   if (sys->collider_kind == JDEM_COLLIDER_CELL_LIST) {
-    Cells c;
-    a.grid = grid_of(sys->grid);
-    int rc = build_cells(ctx, pos, sys->state.rad, sys->state.n, sys->state.dim, a.dom, a.grid, &c);
+    Columns<double> c;
+    a.grid = column_grid(grid_of(sys->grid), sys->state.dim);
+    int rc = build_columns(ctx, pos, sys->state.rad, sys->state.n, sys->state.dim, a.dom, a.grid, &c);
     if (rc) return rc;
     a.perm = c.perm;
     a.skeys = c.skeys;
-    a.cstart = c.cstart;
-    a.cend = c.cend;
-    a.spos = nullptr;
+    a.cstart = c.starts;
+    a.spos = c.spos;
   }
   return JDEM_OK;
 }

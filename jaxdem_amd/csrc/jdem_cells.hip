@@ -711,24 +711,34 @@ hipError_t launch_cell_ranges(const uint32_t* skeys, int64_t n, int32_t* cstart,
 }
 
 // Sorted copy (x, y, z, r) of the particles: contiguous candidate reads.
+template <class Real>
 __global__ void __launch_bounds__(kBlock) k_gather_spos(const int32_t* __restrict__ perm,
-                                                         const float* __restrict__ pos, const float* __restrict__ rad,
-                                                         int64_t n, int dim, float4* __restrict__ spos) {
+                                                         const Real* __restrict__ pos, const Real* __restrict__ rad,
+                                                         int64_t n, int dim, Real4<Real>* __restrict__ spos) {
   int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const int64_t i = perm[s];
-  float4 v;
+  Real4<Real> v;
   v.x = pos[dim * i];
   v.y = pos[dim * i + 1];
-  v.z = (dim == 3) ? pos[dim * i + 2] : 0.0f;
+  v.z = (dim == 3) ? pos[dim * i + 2] : Real(0);
   v.w = rad[i];
   spos[s] = v;
 }
+template <class Real>
+hipError_t gather_spos_run(const int32_t* perm, const Real* pos, const Real* rad, int64_t n, int dim,
+                           Real4<Real>* spos, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_gather_spos<Real>), dim3(nblocks(n)), dim3(kBlock), 0, s, perm, pos, rad, n, dim, spos);
+  return hipGetLastError();
+}
 hipError_t launch_gather_spos(const int32_t* perm, const float* pos, const float* rad, int64_t n, int dim,
                               float4* spos, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gather_spos, dim3(nblocks(n)), dim3(kBlock), 0, s, perm, pos, rad, n, dim, spos);
-  return hipGetLastError();
+  return gather_spos_run(perm, pos, rad, n, dim, spos, s);
+}
+hipError_t launch_gather_spos(const int32_t* perm, const double* pos, const double* rad, int64_t n, int dim,
+                              Double4* spos, hipStream_t s) {
+  return gather_spos_run(perm, pos, rad, n, dim, spos, s);
 }
 
 // ---------------------------------------------------------------------------

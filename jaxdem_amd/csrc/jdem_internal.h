@@ -32,6 +32,21 @@ struct GridPT {
 };
 using GridP = GridPT<float>;
 
+// Four scalars of one cell-sorted particle, (x, y, z, r).
+struct alignas(16) Double4 {
+  double x, y, z, w;
+};
+template <class Real>
+struct Real4Of {
+  using T = float4;
+};
+template <>
+struct Real4Of<double> {
+  using T = Double4;
+};
+template <class Real>
+using Real4 = typename Real4Of<Real>::T;
+
 // One grow-only device allocation of the context.
 struct Buf {
   void* p = nullptr;
@@ -151,13 +166,16 @@ struct StepArgsT {
   Real dt;
   int lin;
   int rot;
-  // cell-list source
+  // cell-list source: cells numbered with the last axis fastest, so a stencil
+  // column is one run of cstart (n_cells + 1 entries); sorted (x, r)
   const int32_t* perm;
   const int32_t* skeys;
   const int32_t* cstart;
-  const int32_t* cend;
-  const float4* spos;  // float only: sorted (x, r)
+  const Real4<Real>* spos;
   GridPT<Real> grid;
+  // particles of one wavefront of a cell-list or naive traversal (a multiple
+  // of the particles it walks at once, at most 64)
+  int pw;
   // neighbour-list source
   const int32_t* nl;
   int M;
@@ -200,7 +218,9 @@ using DomP64 = DomPT<double>;
 using GridP64 = GridPT<double>;
 using LawP64 = LawPT<double>;
 
-enum Src { SRC_NAIVE = 1, SRC_CELLS = 2, SRC_NLIST = 3 };
+// SRC_CELLS_LANE: the cell list walked by one lane per particle, chosen by
+// launch_step for large systems
+enum Src { SRC_NAIVE = 1, SRC_CELLS = 2, SRC_NLIST = 3, SRC_CELLS_LANE = 4 };
 
 // launchers (jdem_step.hip)
 hipError_t launch_step(const StepArgs& a, int dim, int law, int src, hipStream_t s);
@@ -287,10 +307,16 @@ inline int nbits_for_cells(int64_t n_cells) {
 int noalloc_init(int device);
 // whether cell_sort_pairs is the cheaper sort for n keys below n_cells
 inline bool use_cell_sort(int64_t n, int64_t n_cells) { return n > 0 && n_cells <= 4 * n + 65536; }
+// The same question where memory may be allocated: a cell costs 12 bytes of
+// traffic, the radix sort five launches per eight key bits, so the
+// counting sort stays ahead on grids far sparser than the particles.
+inline bool use_cell_sort_sparse(int64_t n, int64_t n_cells) { return n > 0 && n_cells <= 32 * n + (1 << 20); }
 hipError_t launch_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 hipError_t launch_cell_ranges(const uint32_t* skeys, int64_t n, int32_t* cstart, int32_t* cend, hipStream_t s);
 hipError_t launch_gather_spos(const int32_t* perm, const float* pos, const float* rad, int64_t n, int dim,
                               float4* spos, hipStream_t s);
+hipError_t launch_gather_spos(const int32_t* perm, const double* pos, const double* rad, int64_t n, int dim,
+                              Double4* spos, hipStream_t s);
 template <class Real = float>
 struct NLBuildT {
   int64_t n;
@@ -485,6 +511,46 @@ hipError_t ws_launch_place(const RB& r, const uint32_t* sk, int32_t* starts, hip
 __device__ inline unsigned xcd_tile(unsigned w, unsigned nw) {
   const unsigned q = nw / 8u, r = nw % 8u, x = w % 8u, l = w / 8u;
   return (x < r ? x * (q + 1u) : r * (q + 1u) + (x - r) * q) + l;
+}
+
+// Cells of the stencil along one axis, in stencil order: the offsets
+// -sr..hi (hi = min(sr, dims - sr - 1) on a periodic axis, which drops the
+// offsets that would revisit a cell) give at most two runs of consecutive
+// cells, [r0a, r0b] then [r1a, r1b] (empty when a > b).
+JD void stencil_runs(bool per, int c, int sr, int dims, int& r0a, int& r0b, int& r1a, int& r1b) {
+  if (per) {
+    const int cnt = sr + min(sr, dims - sr - 1) + 1;  // in [1, dims]
+    int start = (c - sr) % dims;
+    if (start < 0) start += dims;
+    const int last = start + cnt - 1;
+    r0a = start;
+    r0b = min(last, dims - 1);
+    r1a = 0;
+    r1b = last - dims;
+  } else {
+    r0a = max(c - sr, 0);
+    r0b = min(c + sr, dims - 1);
+    r1a = 0;
+    r1b = -1;
+  }
+}
+
+// Offsets along a slow axis; returns the cell or -1 when it is off the grid.
+JD int stencil_cell(bool per, int c, int o, int dims) {
+  int x = c + o;
+  if (per) {
+    x %= dims;
+    if (x < 0) x += dims;
+    return x;
+  }
+  return (x < 0 || x >= dims) ? -1 : x;
+}
+
+// orders the LDS traffic of one wave around an exchange between its lanes
+JD void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 struct WS {

@@ -266,16 +266,25 @@ __global__ void __launch_bounds__(kBlock) k_seg_ids(const int64_t* __restrict__ 
 
 // Dense cell starts: starts[h] = first sorted slot with key >= h, for h in
 // [0, n_cells]; an empty cell gets the start of the next occupied one, so
-// consecutive cells h1..h2 hold the slots [starts[h1], starts[h2 + 1]).
-// Thread s (0 <= s <= n) writes the cells in (sk[s-1], sk[s]], the gap
-// before slot s, so every cell is written once.
+// consecutive cells h1..h2 hold the slots [starts[h1], starts[h2 + 1]).  One
+// search per cell: a wavefront's cells follow the same path through the keys,
+// and a long run of empty cells (a lattice coarser than the grid, spheres in
+// one corner of their box) costs no more than any other.  Filled by the
+// thread of the slot behind it, the empty planes of a lattice on cells of
+// half its spacing took 1.4 ms at 150 k spheres.
 __global__ void __launch_bounds__(kBlock) k_cell_starts(const uint32_t* __restrict__ sk, int64_t n, int64_t n_cells,
                                                          int32_t* __restrict__ starts) {
-  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s > n) return;
-  const int64_t lo = (s == 0) ? 0 : (int64_t)sk[s - 1] + 1;
-  const int64_t hi = (s == n) ? n_cells : (int64_t)sk[s];
-  for (int64_t h = lo; h <= hi; ++h) starts[h] = (int32_t)s;
+  const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (h > n_cells) return;
+  int64_t lo = 0, hi = n;  // the first slot with key >= h lies in [lo, hi]
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if ((int64_t)sk[mid] < h)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  starts[h] = (int32_t)lo;
 }
 
 // new work slot b' takes old slot src = wpos[new_orig[b']]; inv[src] = b'
@@ -531,39 +540,6 @@ JD bool bonded_o(const int32_t* bond_id, int bond_w, int64_t i, int32_t j) {
   for (int w = 0; w < bond_w; ++w)
     if (bond_id[i * bond_w + w] == j) return true;
   return false;
-}
-
-// Cells of the stencil along one axis, in stencil order: the offsets
-// -sr..hi (hi = min(sr, dims - sr - 1) on a periodic axis, which drops the
-// offsets that would revisit a cell) give at most two runs of consecutive
-// cells, [r0a, r0b] then [r1a, r1b] (empty when a > b).
-JD void stencil_runs(bool per, int c, int sr, int dims, int& r0a, int& r0b, int& r1a, int& r1b) {
-  if (per) {
-    const int cnt = sr + min(sr, dims - sr - 1) + 1;  // in [1, dims]
-    int start = (c - sr) % dims;
-    if (start < 0) start += dims;
-    const int last = start + cnt - 1;
-    r0a = start;
-    r0b = min(last, dims - 1);
-    r1a = 0;
-    r1b = last - dims;
-  } else {
-    r0a = max(c - sr, 0);
-    r0b = min(c + sr, dims - 1);
-    r1a = 0;
-    r1b = -1;
-  }
-}
-
-// Offsets along a slow axis; returns the cell or -1 when it is off the grid.
-JD int stencil_cell(bool per, int c, int o, int dims) {
-  int x = c + o;
-  if (per) {
-    x %= dims;
-    if (x < 0) x += dims;
-    return x;
-  }
-  return (x < 0 || x >= dims) ? -1 : x;
 }
 
 // Number of set bits of the live words (w0..w3) below slot s.
@@ -968,13 +944,6 @@ constexpr int kPairCap = 128;
 // pass 1 keeps the partner index of a lane's first kStash marked slots in LDS,
 // so the pair evaluation need not reload it from the list
 constexpr int kStash = 4;
-
-// orders the LDS traffic of one wave around the exchange of pair results
-JD void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // MW = 64-slot words of a row the kernel handles (1 when M <= 64, else 4):
 // the per-lane slot masks then take 2 * MW registers
@@ -1534,7 +1503,7 @@ hipError_t ws_launch_seg_init_flags(int n_seg, const int32_t* n_build, int32_t* 
   return hipGetLastError();
 }
 hipError_t ws_launch_cell_starts(const uint32_t* skeys, int64_t n, int64_t n_cells, int32_t* starts, hipStream_t s) {
-  hipLaunchKernelGGL(k_cell_starts, dim3(nblocks(n + 1)), dim3(kBlock), 0, s, skeys, n, n_cells, starts);
+  hipLaunchKernelGGL(k_cell_starts, dim3(nblocks(n_cells + 1)), dim3(kBlock), 0, s, skeys, n, n_cells, starts);
   return hipGetLastError();
 }
 hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s) {
