@@ -22,7 +22,7 @@ std::vector<Buf*> jdem_ctx::bufs() {
                            &cstart,  &cend,   &spos,     &nl_new,  &xi_new,  &live_new, &flags,  &red,
                            &nl_copy, &xi_copy, &live_copy, &wF,     &wT,      &wOld,     &wWpos, &wSrc,
                            &wInv,    &wKeys,  &fireV,    &fireDev, &segp,  &segid, &segflag, &wXiRank,
-                           &route,   &ccnt,   &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl, &pvaux};
+                           &route,   &ccnt,   &cscnt,  &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl, &pvaux};
   for (int k = 0; k < 2; ++k)
     for (Buf* b : {&wP[k], &wV[k], &wW[k], &wQ[k], &wI[k], &wOrig[k], &wNl[k], &wXi[k], &wLive[k]}) all.push_back(b);
   return all;
@@ -425,21 +425,27 @@ int build_columns(jdem_ctx* ctx, const Real* pos, const Real* rad, int64_t n, in
   ENSURE(ctx, ctx->cstart, 4 * ((size_t)g.n_cells + 1));
   ENSURE(ctx, ctx->spos, sizeof(Real4<Real>) * nn);
   uint32_t* hk = (uint32_t*)ctx->wKeys.p;
-  HIPCHK(ctx, launch_hash(pos, n, dim, dom, g, hk, ctx->stream));
+  int32_t* cs = (int32_t*)ctx->cstart.p;
+  Real4<Real>* spos = (Real4<Real>*)ctx->spos.p;
   uint32_t* sk = nullptr;
   int32_t* perm = nullptr;
-  int32_t* cs = (int32_t*)ctx->cstart.p;
   if (use_cell_sort_sparse(n, g.n_cells)) {
-    HIPCHK(ctx, cell_sort_pairs(ctx, hk, n, g.n_cells, &sk, &perm, cs, ctx->stream));
+    CellSort srt;
+    HIPCHK(ctx, cell_sort_begin(ctx, n, g.n_cells, &srt, ctx->stream));
+    HIPCHK(ctx, launch_hash(pos, n, dim, dom, g, hk, ctx->stream, &srt));
+    HIPCHK(ctx, cell_sort_end(ctx, srt, hk, n, g.n_cells, cs, pos, rad, dim, spos, ctx->stream));
+    sk = srt.sk;
+    perm = srt.perm;
   } else {
+    HIPCHK(ctx, launch_hash(pos, n, dim, dom, g, hk, ctx->stream));
     HIPCHK(ctx, radix_sort_pairs(ctx, hk, n, nbits_for(g.n_cells), &sk, &perm, ctx->stream));
     HIPCHK(ctx, ws_launch_cell_starts(sk, n, g.n_cells, cs, ctx->stream));
+    HIPCHK(ctx, launch_gather_spos(perm, pos, rad, n, dim, spos, ctx->stream));
   }
-  HIPCHK(ctx, launch_gather_spos(perm, pos, rad, n, dim, (Real4<Real>*)ctx->spos.p, ctx->stream));
   out->perm = perm;
   out->skeys = (int32_t*)sk;
   out->starts = cs;
-  out->spos = (Real4<Real>*)ctx->spos.p;
+  out->spos = spos;
   return JDEM_OK;
 }
 
@@ -745,13 +751,18 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
   if (R) {
     HIPCHK(ctx, hipMemcpyAsync(ctx->wOrig[0].p, R->orig.p, ni, hipMemcpyDeviceToDevice, st));
   } else if (!naive2 && !sg) {
-    HIPCHK(ctx, launch_hash(s.pos, N, D, dom, g, (uint32_t*)ctx->wKeys.p, st));
     uint32_t* sk = nullptr;
     int32_t* perm = nullptr;
-    if (use_cell_sort(N, g.n_cells))
-      HIPCHK(ctx, cell_sort_pairs(ctx, (uint32_t*)ctx->wKeys.p, N, g.n_cells, &sk, &perm, I32(ctx->cstart), st));
-    else
+    if (use_cell_sort_sparse(N, g.n_cells)) {
+      CellSort srt;
+      HIPCHK(ctx, cell_sort_begin(ctx, N, g.n_cells, &srt, st));
+      HIPCHK(ctx, launch_hash(s.pos, N, D, dom, g, (uint32_t*)ctx->wKeys.p, st, &srt));
+      HIPCHK(ctx, cell_sort_end(ctx, srt, (uint32_t*)ctx->wKeys.p, N, g.n_cells, I32(ctx->cstart), st));
+      perm = srt.perm;
+    } else {
+      HIPCHK(ctx, launch_hash(s.pos, N, D, dom, g, (uint32_t*)ctx->wKeys.p, st));
       HIPCHK(ctx, radix_sort_pairs(ctx, (uint32_t*)ctx->wKeys.p, N, nbits_for(g.n_cells), &sk, &perm, st));
+    }
     HIPCHK(ctx, hipMemcpyAsync(ctx->wOrig[0].p, perm, ni, hipMemcpyDeviceToDevice, st));
   } else {
     HIPCHK(ctx, ws_launch_iota(I32(ctx->wOrig[0]), N, st));
@@ -950,15 +961,20 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
     int32_t* inv = I32(ctx->wInv);
     uint32_t* sk = nullptr;
     if (!naive2) {
-      HIPCHK(ctx, ws_launch_hash(F4(ctx->wP[cur]), I32(ctx->wOrig[set]), N, D, dom, g, (uint32_t*)ctx->wKeys.p,
-                                 I32(ctx->wWpos), st));
       int32_t* new_orig = nullptr;
       // the counting sort also writes the cell starts
-      const bool counted = use_cell_sort(N, n_cells);
-      if (counted)
-        HIPCHK(ctx, cell_sort_pairs(ctx, (uint32_t*)ctx->wKeys.p, N, n_cells, &sk, &new_orig, I32(ctx->cstart), st));
-      else
+      const bool counted = use_cell_sort_sparse(N, n_cells);
+      CellSort srt;
+      if (counted) HIPCHK(ctx, cell_sort_begin(ctx, N, n_cells, &srt, st));
+      HIPCHK(ctx, ws_launch_hash(F4(ctx->wP[cur]), I32(ctx->wOrig[set]), N, D, dom, g, (uint32_t*)ctx->wKeys.p,
+                                 I32(ctx->wWpos), st, counted ? &srt : nullptr));
+      if (counted) {
+        HIPCHK(ctx, cell_sort_end(ctx, srt, (uint32_t*)ctx->wKeys.p, N, n_cells, I32(ctx->cstart), st));
+        sk = srt.sk;
+        new_orig = srt.perm;
+      } else {
         HIPCHK(ctx, radix_sort_pairs(ctx, (uint32_t*)ctx->wKeys.p, N, nbits_for(n_cells), &sk, &new_orig, st));
+      }
       HIPCHK(ctx, ws_launch_permute(N, new_orig, I32(ctx->wWpos), F4(ctx->wP[cur]), F4(ctx->wV[cur]),
                                     F4(ctx->wW[cur]), F4(ctx->wQ[set]), F4(ctx->wI[set]), F4(ctx->wP[1 - cur]),
                                     F4(ctx->wV[1 - cur]), F4(ctx->wW[1 - cur]), F4(ctx->wQ[1 - set]),

@@ -34,41 +34,44 @@ JD int cell_coord(Real x, int a, const DomPT<Real>& dom, const GridPT<Real>& g) 
 
 template <int D, bool PER, class Real>
 __global__ void __launch_bounds__(kBlock) k_hash(const Real* __restrict__ pos, int64_t n, DomPT<Real> dom,
-                                                  GridPT<Real> g, uint32_t* __restrict__ keys) {
+                                                  GridPT<Real> g, uint32_t* __restrict__ keys,
+                                                  int32_t* __restrict__ cnt, int32_t* __restrict__ arr) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   int h = 0;
 #pragma unroll
   for (int a = 0; a < D; ++a) h += cell_coord<PER>(pos[D * i + a], a, dom, g) * g.strides[a];
   keys[i] = (uint32_t)h;
+  if (cnt) arr[i] = atomicAdd(&cnt[h], 1);  // the count pass of the counting sort
 }
 
 template <class Real>
 hipError_t hash_run(const Real* pos, int64_t n, int dim, const DomPT<Real>& dom, const GridPT<Real>& g,
-                    uint32_t* keys, hipStream_t s) {
+                    uint32_t* keys, hipStream_t s, const CellSort* cs) {
   if (n == 0) return hipSuccess;
   dim3 grd(nblocks(n)), blk(kBlock);
   bool per = g.periodic != 0;
+  int32_t *cnt = cs ? cs->cnt : nullptr, *arr = cs ? cs->arr : nullptr;
   if (dim == 3) {
     if (per)
-      hipLaunchKernelGGL((k_hash<3, true, Real>), grd, blk, 0, s, pos, n, dom, g, keys);
+      hipLaunchKernelGGL((k_hash<3, true, Real>), grd, blk, 0, s, pos, n, dom, g, keys, cnt, arr);
     else
-      hipLaunchKernelGGL((k_hash<3, false, Real>), grd, blk, 0, s, pos, n, dom, g, keys);
+      hipLaunchKernelGGL((k_hash<3, false, Real>), grd, blk, 0, s, pos, n, dom, g, keys, cnt, arr);
   } else {
     if (per)
-      hipLaunchKernelGGL((k_hash<2, true, Real>), grd, blk, 0, s, pos, n, dom, g, keys);
+      hipLaunchKernelGGL((k_hash<2, true, Real>), grd, blk, 0, s, pos, n, dom, g, keys, cnt, arr);
     else
-      hipLaunchKernelGGL((k_hash<2, false, Real>), grd, blk, 0, s, pos, n, dom, g, keys);
+      hipLaunchKernelGGL((k_hash<2, false, Real>), grd, blk, 0, s, pos, n, dom, g, keys, cnt, arr);
   }
   return hipGetLastError();
 }
 hipError_t launch_hash(const float* pos, int64_t n, int dim, const DomP& dom, const GridP& g, uint32_t* keys,
-                       hipStream_t s) {
-  return hash_run(pos, n, dim, dom, g, keys, s);
+                       hipStream_t s, const CellSort* cs) {
+  return hash_run(pos, n, dim, dom, g, keys, s, cs);
 }
 hipError_t launch_hash(const double* pos, int64_t n, int dim, const DomP64& dom, const GridP64& g, uint32_t* keys,
-                       hipStream_t s) {
-  return hash_run(pos, n, dim, dom, g, keys, s);
+                       hipStream_t s, const CellSort* cs) {
+  return hash_run(pos, n, dim, dom, g, keys, s, cs);
 }
 
 // ---------------------------------------------------------------------------
@@ -360,56 +363,129 @@ hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, i
 }
 
 // ---------------------------------------------------------------------------
-// counting sort by cell.  Placement through atomic cursors puts a cell's ids
-// in arbitrary order inside the cell's range; the rank pass then writes each
-// id at its cell start + the number of smaller ids in the cell, which is the
-// order of a stable sort of (key, id).  Cells hold a few particles, so the
-// rank pass reads a handful of ids per element.
+// counting sort by cell.  The count pass keeps each element's arrival number
+// in its cell (the value its atomic returns), so placement needs no second
+// atomic; arrival order is arbitrary, and the rank pass then writes each id at
+// its cell start + the number of smaller ids in the cell, which is the order
+// of a stable sort of (key, id).  Cells hold a few particles, so the rank pass
+// reads a handful of ids per element.
+//
+// Below ~10^5 particles the sort is bounded by its launches (4-6 us each, one
+// after the other), so the passes are few: the caller's key kernel counts too,
+// the scan adds up the totals of the chunks before its own instead of a pass
+// over the totals, it clears the counts for the next sort, and the rank pass
+// gathers the sorted (x, r).  Five launches with the key kernel where there
+// were ten (45 -> 25 us of a 100 k-particle cell-list step).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_cs_zero(int32_t* __restrict__ cnt, int32_t* __restrict__ cur,
-                                                     int64_t n_cells, const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c > n_cells) return;
-  cnt[c] = 0;
-  if (c < n_cells) cur[c] = 0;
-}
-
 __global__ void __launch_bounds__(kBlock) k_cs_count(const uint32_t* __restrict__ keys, int64_t n,
-                                                      int32_t* __restrict__ cnt, const int32_t* __restrict__ gate) {
+                                                      int32_t* __restrict__ cnt, int32_t* __restrict__ arr,
+                                                      const int32_t* __restrict__ gate) {
   if (gate && *gate == 0) return;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  atomicAdd(&cnt[keys[i]], 1);
+  arr[i] = atomicAdd(&cnt[keys[i]], 1);
+}
+
+// starts[c] = number of elements in the cells before c, c in [0, n_cells];
+// cnt is cleared.  sums holds each chunk's total, or (scanned) the sum of the
+// chunks before it.
+__global__ void __launch_bounds__(kBlock) k_cs_scan(int32_t* __restrict__ cnt, int64_t n_cells,
+                                                     const uint32_t* __restrict__ sums, int scanned,
+                                                     int32_t* __restrict__ starts, const int32_t* __restrict__ gate) {
+  if (gate && *gate == 0) return;
+  __shared__ uint32_t tile[SC_CHUNK];
+  __shared__ uint32_t tsum[kBlock];
+  const int tid = threadIdx.x;
+  const int64_t base = (int64_t)blockIdx.x * SC_CHUNK;
+  uint32_t before = 0;
+  if (scanned) {
+    before = sums[blockIdx.x];
+  } else {
+    for (int64_t c = tid; c < (int64_t)blockIdx.x; c += kBlock) before += sums[c];
+    tsum[tid] = before;
+    __syncthreads();
+    for (int off = kBlock / 2; off > 0; off >>= 1) {
+      if (tid < off) tsum[tid] += tsum[tid + off];
+      __syncthreads();
+    }
+    before = tsum[0];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int it = 0; it < SC_ITEMS; ++it) {
+    const int64_t k = base + (int64_t)it * kBlock + tid;
+    uint32_t v = 0;
+    if (k < n_cells) {
+      v = (uint32_t)cnt[k];
+      cnt[k] = 0;
+    }
+    tile[it * kBlock + tid] = v;
+  }
+  __syncthreads();
+  // thread t scans its contiguous run tile[t*SC_ITEMS .. +SC_ITEMS)
+  uint32_t s = 0;
+#pragma unroll
+  for (int it = 0; it < SC_ITEMS; ++it) s += tile[tid * SC_ITEMS + it];
+  tsum[tid] = s;
+  __syncthreads();
+  for (int off = 1; off < kBlock; off <<= 1) {
+    const uint32_t v = (tid >= off) ? tsum[tid - off] : 0u;
+    __syncthreads();
+    tsum[tid] += v;
+    __syncthreads();
+  }
+  uint32_t run = before + ((tid == 0) ? 0u : tsum[tid - 1]);
+#pragma unroll
+  for (int it = 0; it < SC_ITEMS; ++it) {
+    const uint32_t v = tile[tid * SC_ITEMS + it];
+    tile[tid * SC_ITEMS + it] = run;
+    run += v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < SC_ITEMS; ++it) {
+    const int64_t k = base + (int64_t)it * kBlock + tid;
+    if (k <= n_cells) starts[k] = (int32_t)tile[it * kBlock + tid];
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) k_cs_place(const uint32_t* __restrict__ keys, int64_t n,
-                                                      const int32_t* __restrict__ starts, int32_t* __restrict__ cur,
-                                                      uint32_t* __restrict__ tkey, int32_t* __restrict__ tid,
+                                                      const int32_t* __restrict__ starts,
+                                                      const int32_t* __restrict__ arr, uint2* __restrict__ pairs,
                                                       const int32_t* __restrict__ gate) {
   if (gate && *gate == 0) return;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t k = keys[i];
-  const int32_t slot = starts[k] + atomicAdd(&cur[k], 1);
-  tkey[slot] = k;
-  tid[slot] = (int32_t)i;
+  pairs[starts[k] + arr[i]] = make_uint2(k, (uint32_t)i);
 }
 
-__global__ void __launch_bounds__(kBlock) k_cs_rank(const uint32_t* __restrict__ tkey, const int32_t* __restrict__ tid,
-                                                     int64_t n, const int32_t* __restrict__ starts,
-                                                     uint32_t* __restrict__ sk, int32_t* __restrict__ perm,
+// sorted keys and ids and, with spos, the sorted (x, r)
+template <class Real>
+__global__ void __launch_bounds__(kBlock) k_cs_rank(const uint2* __restrict__ pairs, int64_t n,
+                                                     const int32_t* __restrict__ starts, uint32_t* __restrict__ sk,
+                                                     int32_t* __restrict__ perm, const Real* __restrict__ pos,
+                                                     const Real* __restrict__ rad, int dim,
+                                                     Real4<Real>* __restrict__ spos,
                                                      const int32_t* __restrict__ gate) {
   if (gate && *gate == 0) return;
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const uint32_t k = tkey[j];
-  const int32_t id = tid[j];
-  const int32_t s = starts[k], e = starts[k + 1];
-  int32_t r = 0;
-  for (int32_t m = s; m < e; ++m) r += tid[m] < id ? 1 : 0;
-  sk[s + r] = k;
-  perm[s + r] = id;
+  const uint2 me = pairs[j];
+  const int32_t s = starts[me.x], e = starts[me.x + 1];
+  int32_t r = s;
+  for (int32_t m = s; m < e; ++m) r += pairs[m].y < me.y ? 1 : 0;
+  sk[r] = me.x;
+  perm[r] = (int32_t)me.y;
+  if (spos) {
+    const int64_t i = me.y;
+    Real4<Real> v;
+    v.x = pos[dim * i];
+    v.y = pos[dim * i + 1];
+    v.z = (dim == 3) ? pos[dim * i + 2] : Real(0);
+    v.w = rad[i];
+    spos[r] = v;
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) k_cs_ends(const int32_t* __restrict__ starts, int64_t n_cells,
@@ -428,35 +504,49 @@ size_t cell_sort_sum_words(int64_t n_cells) {
   return (size_t)((total + SC_CHUNK - 1) / SC_CHUNK) + 1;
 }
 
+// Chunk totals that a scan block adds up itself; with more chunks a pass over
+// the totals comes first (a block reads them all).
+constexpr int kScanDirect = 1024;
+
+// The passes after the count: scan, placement, rank (+ gather).
+template <class Real>
+hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells, int32_t* starts,
+                     const Real* pos, const Real* rad, int dim, Real4<Real>* spos, hipStream_t s,
+                     const int32_t* gate) {
+  const int nchunks = (int)((n_cells + 1 + SC_CHUNK - 1) / SC_CHUNK);
+  if (nchunks > 1)
+    hipLaunchKernelGGL(k_scan_totals, dim3(nchunks), dim3(kBlock), 0, s, (const uint32_t*)cs.cnt, n_cells, cs.sums,
+                       gate);
+  const bool scanned = nchunks > kScanDirect;
+  if (scanned) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, cs.sums, nchunks, gate);
+  hipLaunchKernelGGL(k_cs_scan, dim3(nchunks), dim3(kBlock), 0, s, cs.cnt, n_cells, cs.sums, scanned ? 1 : 0, starts,
+                     gate);
+  if (n > 0) {
+    hipLaunchKernelGGL(k_cs_place, dim3(nblocks(n)), dim3(kBlock), 0, s, keys, n, starts, cs.arr, cs.pairs, gate);
+    hipLaunchKernelGGL((k_cs_rank<Real>), dim3(nblocks(n)), dim3(kBlock), 0, s, cs.pairs, n, starts, cs.sk, cs.perm,
+                       pos, rad, dim, spos, gate);
+  }
+  return hipGetLastError();
+}
+
 // keys_in may be sb.k1: it is read only before the rank pass writes the
-// sorted keys there.
+// sorted keys there.  sb.k0 holds 2 n words, sb.v1 the arrival numbers until
+// the rank pass writes the ids there.
 hipError_t cell_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
                           int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate) {
-  const int64_t total = n_cells + 1;
-  const int nchunks = (int)((total + SC_CHUNK - 1) / SC_CHUNK);
-  uint32_t* tkey = sb.k0;
-  int32_t* tid = sb.v0;
-  uint32_t* sk = sb.k1;
-  int32_t* perm = sb.v1;
-  int32_t* cur = sb.cur;
-  hipLaunchKernelGGL(k_cs_zero, dim3(nblocks(total)), dim3(kBlock), 0, s, starts, cur, n_cells, gate);
-  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, starts, gate);
-  uint32_t* cnt = (uint32_t*)starts;  // counts are non-negative: scan them as uint32
-  if (nchunks <= 1) {
-    hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, cnt, total, gate);
-  } else {
-    uint32_t* sums = sb.hist;
-    hipLaunchKernelGGL(k_scan_totals, dim3(nchunks), dim3(kBlock), 0, s, cnt, total, sums, gate);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nchunks, gate);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nchunks), dim3(kBlock), 0, s, cnt, total, sums, gate);
-  }
-  if (n > 0) {
-    hipLaunchKernelGGL(k_cs_place, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, starts, cur, tkey, tid, gate);
-    hipLaunchKernelGGL(k_cs_rank, dim3(nblocks(n)), dim3(kBlock), 0, s, tkey, tid, n, starts, sk, perm, gate);
-  }
-  *keys_out = sk;
-  *vals_out = perm;
-  return hipGetLastError();
+  CellSort cs;
+  cs.cnt = sb.cur;
+  cs.arr = sb.v1;
+  cs.pairs = (uint2*)sb.k0;
+  cs.sums = sb.hist;
+  cs.sk = sb.k1;
+  cs.perm = sb.v1;
+  hipError_t e = launch_fill_i32(cs.cnt, n_cells, 0, s);
+  if (e != hipSuccess) return e;
+  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr, gate);
+  *keys_out = cs.sk;
+  *vals_out = cs.perm;
+  return cs_finish<float>(cs, keys_in, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s, gate);
 }
 
 // ---- counting sort with device-side counts (batch rebuilds) --------------
@@ -654,22 +744,61 @@ hipError_t cell_sort_dev(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int6
   return hipGetLastError();
 }
 
-hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
-                           int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate) {
-  const size_t nn = (size_t)(n > 0 ? n : 1);
-  if (!ensure(ctx, ctx->keys[0], sizeof(uint32_t) * nn) || !ensure(ctx, ctx->keys[1], sizeof(uint32_t) * nn) ||
+hipError_t cell_sort_begin(jdem_ctx* ctx, int64_t n, int64_t n_cells, CellSort* cs, hipStream_t s) {
+  const size_t nn = (size_t)(n > 0 ? n : 1), nc = (size_t)(n_cells > 0 ? n_cells : 1);
+  if (ctx->cscnt.bytes < sizeof(int32_t) * nc) ctx->cscnt_clear = false;  // a new buffer comes uncleared
+  if (!ensure(ctx, ctx->keys[0], sizeof(uint2) * nn) || !ensure(ctx, ctx->keys[1], sizeof(uint32_t) * nn) ||
       !ensure(ctx, ctx->vals[0], sizeof(int32_t) * nn) || !ensure(ctx, ctx->vals[1], sizeof(int32_t) * nn) ||
-      !ensure(ctx, ctx->ccur, sizeof(int32_t) * (size_t)(n_cells > 0 ? n_cells : 1)) ||
+      !ensure(ctx, ctx->cscnt, sizeof(int32_t) * nc) ||
       !ensure(ctx, ctx->hist, sizeof(uint32_t) * cell_sort_sum_words(n_cells)))
     return hipErrorOutOfMemory;
-  SortBufs sb;
-  sb.k0 = (uint32_t*)ctx->keys[0].p;
-  sb.k1 = (uint32_t*)ctx->keys[1].p;
-  sb.v0 = (int32_t*)ctx->vals[0].p;
-  sb.v1 = (int32_t*)ctx->vals[1].p;
-  sb.hist = (uint32_t*)ctx->hist.p;
-  sb.cur = (int32_t*)ctx->ccur.p;
-  return cell_sort_bufs(sb, keys_in, n, n_cells, keys_out, vals_out, starts, s, gate);
+  cs->cnt = (int32_t*)ctx->cscnt.p;
+  cs->arr = (int32_t*)ctx->vals[0].p;
+  cs->pairs = (uint2*)ctx->keys[0].p;
+  cs->sums = (uint32_t*)ctx->hist.p;
+  cs->sk = (uint32_t*)ctx->keys[1].p;
+  cs->perm = (int32_t*)ctx->vals[1].p;
+  // the scan of every sort leaves the counts clear; a sort that was not
+  // finished does not
+  if (!ctx->cscnt_clear) {
+    const hipError_t e = launch_fill_i32(cs->cnt, (int64_t)(ctx->cscnt.bytes / sizeof(int32_t)), 0, s);
+    if (e != hipSuccess) return e;
+  }
+  ctx->cscnt_clear = false;
+  return hipSuccess;
+}
+
+template <class Real>
+hipError_t cell_sort_end_run(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                             int32_t* starts, const Real* pos, const Real* rad, int dim, Real4<Real>* spos,
+                             hipStream_t s, const int32_t* gate) {
+  const hipError_t e = cs_finish<Real>(cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, gate);
+  ctx->cscnt_clear = e == hipSuccess;
+  return e;
+}
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, hipStream_t s, const int32_t* gate) {
+  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s, gate);
+}
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, const float* pos, const float* rad, int dim, float4* spos, hipStream_t s) {
+  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, nullptr);
+}
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, const double* pos, const double* rad, int dim, Double4* spos,
+                         hipStream_t s) {
+  return cell_sort_end_run<double>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, nullptr);
+}
+
+hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
+                           int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate) {
+  CellSort cs;
+  const hipError_t e = cell_sort_begin(ctx, n, n_cells, &cs, s);
+  if (e != hipSuccess) return e;
+  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr, gate);
+  *keys_out = cs.sk;
+  *vals_out = cs.perm;
+  return cell_sort_end(ctx, cs, keys_in, n, n_cells, starts, s, gate);
 }
 
 // ---------------------------------------------------------------------------

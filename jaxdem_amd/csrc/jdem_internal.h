@@ -62,7 +62,9 @@ struct jdem_ctx {
   // scratch, grown on demand and reused across calls
   jdem::Buf pos2, vel2, ang2;          // ping-pong kinematics
   jdem::Buf keys[2], vals[2], hist;    // radix sort
-  jdem::Buf ccur;                      // counting sort: per-cell cursors
+  jdem::Buf ccur;                      // batch counting sort: per-cell cursors
+  jdem::Buf cscnt;                     // counting sort: per-cell counts, left clear by every finished sort
+  bool cscnt_clear = false;
   jdem::Buf cstart, cend, spos;        // cell tables, sorted (x, r)
   jdem::Buf nl_new, xi_new, live_new;  // neighbour-list rebuild
   jdem::Buf flags;                     // small device words
@@ -243,12 +245,25 @@ hipError_t launch_clump_reflect(const StepArgs64& a, int dim, hipStream_t s);
 inline int refl_scratch_words(int dim) { return 8 * dim + 2 + (dim == 3 ? 3 : 1); }
 
 // launchers (jdem_cells.hip)
+// Buffers of one counting sort by cell: per-cell counts, each element's
+// arrival number in its cell, (key, id) by arrival, scan totals; sorted keys
+// and ids.
+struct CellSort {
+  int32_t* cnt;
+  int32_t* arr;
+  uint2* pairs;
+  uint32_t* sums;
+  uint32_t* sk;
+  int32_t* perm;
+};
+// With cs, the key kernel is the sort's count pass too.
 hipError_t launch_hash(const float* pos, int64_t n, int dim, const DomP& dom, const GridP& g, uint32_t* keys,
-                       hipStream_t s);
+                       hipStream_t s, const CellSort* cs = nullptr);
 hipError_t launch_hash(const double* pos, int64_t n, int dim, const DomP64& dom, const GridP64& g, uint32_t* keys,
-                       hipStream_t s);
-// Buffers of a sort: key and value ping-pong arrays of n entries, a
-// histogram / scan-sum array and (counting sort) per-cell cursors.
+                       hipStream_t s, const CellSort* cs = nullptr);
+// Buffers of a sort: key and value ping-pong arrays of n entries (the
+// counting sort takes k0 and v0 as one array of 2 n words at k0), a histogram
+// / scan-sum array and (counting sort) per-cell counts.
 struct SortBufs {
   uint32_t* k0;
   uint32_t* k1;
@@ -275,10 +290,22 @@ hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, i
                             const int32_t* gate = nullptr);
 // The same result as radix_sort_pairs for keys < n_cells, by counting:
 // per-cell counts, their exclusive scan (written to starts[0..n_cells],
-// starts[n_cells] = n), placement through per-cell cursors, then each
-// element's rank among its cell's ids.  Cost grows with n + n_cells.
-// With gate, every kernel of the sort returns at once while *gate == 0 (a
-// device word), leaving the previous sort's outputs in place.
+// starts[n_cells] = n), placement by arrival number, then each element's rank
+// among its cell's ids.  Cost grows with n + n_cells.  With gate, every kernel
+// of the sort returns at once while *gate == 0 (a device word), leaving the
+// previous sort's outputs in place.
+// cell_sort_begin hands out the buffers (counts clear); a kernel of the caller
+// then writes each key, adds 1 to its cell's count and keeps the value the
+// atomic returned; cell_sort_end runs the remaining passes on those keys (and,
+// with spos, gathers the sorted (x, r)).
+hipError_t cell_sort_begin(jdem_ctx* ctx, int64_t n, int64_t n_cells, CellSort* cs, hipStream_t s);
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, const float* pos, const float* rad, int dim, float4* spos, hipStream_t s);
+hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
+                         int32_t* starts, const double* pos, const double* rad, int dim, Double4* spos,
+                         hipStream_t s);
 hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
                            int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
 // The counting sort with both counts on the device: the first *n_dev of
@@ -629,7 +656,7 @@ hipError_t ws_launch_inverse(const int32_t* orig, int64_t n, int32_t* wpos, hipS
 hipError_t ws_launch_iota(int32_t* p, int64_t n, hipStream_t s);
 hipError_t ws_launch_copy4(float4* d, const float4* src, int64_t n, hipStream_t s);
 hipError_t ws_launch_hash(const float4* P4, const int32_t* orig, int64_t n, int dim, const DomP& dom, const GridP& g,
-                          uint32_t* keys, int32_t* wpos, hipStream_t s);
+                          uint32_t* keys, int32_t* wpos, hipStream_t s, const CellSort* cs = nullptr);
 // seg[b] = system of particle b for the ranges offsets[0..n_seg]
 hipError_t ws_launch_seg_ids(const int64_t* offsets, int n_seg, int64_t n, int32_t* seg, hipStream_t s);
 hipError_t ws_launch_permute(int64_t n, const int32_t* new_orig, const int32_t* wpos, const float4* P,

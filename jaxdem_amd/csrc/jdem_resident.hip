@@ -230,11 +230,13 @@ JD uint32_t wkey(const int* c, const GridP& g) {
   return (uint32_t)(c[0] * g.dims[1] + c[1]);
 }
 
-// keys[orig[b]] = work cell key of P4[b]; wpos[orig[b]] = b
+// keys[orig[b]] = work cell key of P4[b]; wpos[orig[b]] = b; with cnt, the
+// element's arrival number in its cell
 template <int D, bool PER>
 __global__ void __launch_bounds__(kBlock) k_hash_work(const float4* __restrict__ P4, const int32_t* __restrict__ orig,
                                                        int64_t n, DomP dom, GridP g, uint32_t* __restrict__ keys,
-                                                       int32_t* __restrict__ wpos) {
+                                                       int32_t* __restrict__ wpos, int32_t* __restrict__ cnt,
+                                                       int32_t* __restrict__ arr) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= n) return;
   const float4 p = P4[b];
@@ -243,8 +245,10 @@ __global__ void __launch_bounds__(kBlock) k_hash_work(const float4* __restrict__
 #pragma unroll
   for (int a = 0; a < D; ++a) c[a] = ccoord<PER>(x[a], a, dom, g);
   const int32_t i = orig[b];
-  keys[i] = wkey<D>(c, g);
+  const uint32_t k = wkey<D>(c, g);
+  keys[i] = k;
   wpos[i] = (int32_t)b;
+  if (cnt) arr[i] = atomicAdd(&cnt[k], 1);  // the count pass of the counting sort
 }
 
 // seg[b] = the system whose particle range [offsets[s], offsets[s + 1])
@@ -1439,19 +1443,20 @@ hipError_t ws_launch_copy4(float4* d, const float4* src, int64_t n, hipStream_t 
   return hipGetLastError();
 }
 hipError_t ws_launch_hash(const float4* P4, const int32_t* orig, int64_t n, int dim, const DomP& dom, const GridP& g,
-                          uint32_t* keys, int32_t* wpos, hipStream_t s) {
+                          uint32_t* keys, int32_t* wpos, hipStream_t s, const CellSort* cs) {
   dim3 gr(nblocks(n)), b(kBlock);
   const bool per = g.periodic != 0;
+  int32_t *cnt = cs ? cs->cnt : nullptr, *arr = cs ? cs->arr : nullptr;
   if (dim == 3) {
     if (per)
-      hipLaunchKernelGGL((k_hash_work<3, true>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos);
+      hipLaunchKernelGGL((k_hash_work<3, true>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos, cnt, arr);
     else
-      hipLaunchKernelGGL((k_hash_work<3, false>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos);
+      hipLaunchKernelGGL((k_hash_work<3, false>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos, cnt, arr);
   } else {
     if (per)
-      hipLaunchKernelGGL((k_hash_work<2, true>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos);
+      hipLaunchKernelGGL((k_hash_work<2, true>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos, cnt, arr);
     else
-      hipLaunchKernelGGL((k_hash_work<2, false>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos);
+      hipLaunchKernelGGL((k_hash_work<2, false>), gr, b, 0, s, P4, orig, n, dom, g, keys, wpos, cnt, arr);
   }
   return hipGetLastError();
 }
