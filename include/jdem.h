@@ -511,6 +511,16 @@ typedef struct jdem_precise {
  * sum over pairs r_ij (x) F_ij of the final configuration. */
 int jdem_precise_minimize(jdem_ctx* ctx, jdem_precise* p, const jdem_fire* fire, int64_t max_steps, double pe_tol,
                           double pe_diff_tol, double force_tol, jdem_minimize_stats* stats, double* virial);
+/* float64 positions (N, D) on the device <-> integer cell + float32 offset.
+ * box_edge, cell_edge (dim doubles: dims * cell_edge and cell + cell_lo),
+ * cell_hi (dim floats: cell) and dims are host arrays.  Import wraps a
+ * position into the box and rounds its offset once, kept in [0, cell). */
+int jdem_precise_import(jdem_ctx* ctx, const double* pos, int64_t n, int32_t dim, const double* box_edge,
+                        const double* cell_edge, const float* cell_hi, const int32_t* dims, int32_t* cidx,
+                        float* off);
+int jdem_precise_export(jdem_ctx* ctx, const int32_t* cidx, const float* off, int64_t n, int32_t dim,
+                        const double* box_edge, const double* cell_edge, const float* cell_hi, const int32_t* dims,
+                        double* pos);
 
 /* ---- (f) the plain step in float64 -------------------------------------------
  *

@@ -378,6 +378,12 @@ SIGNATURES = {
         [c_void_p, POINTER(JdemPrecise), POINTER(JdemFire), c_int64, c_double, c_double, c_double,
          POINTER(JdemMinimizeStats), c_void_p],
     ),
+    "jdem_precise_import": (
+        c_int, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
+    "jdem_precise_export": (
+        c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
     "jdem_resident_release": (c_int, [c_void_p, c_void_p]),
     "jdem_resident_export": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "jdem_ctx_trim": (c_int, [c_void_p]),

@@ -22,7 +22,7 @@ std::vector<Buf*> jdem_ctx::bufs() {
                            &cstart,  &cend,   &spos,     &nl_new,  &xi_new,  &live_new, &flags,  &red,
                            &nl_copy, &xi_copy, &live_copy, &wF,     &wT,      &wOld,     &wWpos, &wSrc,
                            &wInv,    &wKeys,  &fireV,    &fireDev, &segp,  &segid, &segflag, &wXiRank,
-                           &route,   &ccnt,   &cscnt,  &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl, &pvaux};
+                           &route,   &ccnt,   &cscnt,  &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl};
   for (int k = 0; k < 2; ++k)
     for (Buf* b : {&wP[k], &wV[k], &wW[k], &wQ[k], &wI[k], &wOrig[k], &wNl[k], &wXi[k], &wLive[k]}) all.push_back(b);
   return all;
@@ -2075,53 +2075,13 @@ int jdem_precise_minimize(jdem_ctx* ctx, jdem_precise* p, const jdem_fire* fire,
   if (max_steps < 0) return fail(ctx, JDEM_EINVAL, "max_steps < 0");
   (void)hipSetDevice(ctx->device);
   hipStream_t st = ctx->stream;
-  const int A = D == 3 ? 3 : 1;
-  const size_t Nn = (size_t)std::max<int64_t>(N, 1);
-  const int nparts = std::max(1u, nblocks(N));
-  // scratch: FIRE velocities and zero torque / fixed / rotation velocities,
-  // per-sphere energies and virials, cell keys and starts
-  ENSURE(ctx, ctx->fireV, 4 * Nn * (D + 2 * A) + Nn);
-  ENSURE(ctx, ctx->fireDev, sizeof(FireDev) + 8 * (size_t)nparts + 64 + sizeof(PrecStop));
-  ENSURE(ctx, ctx->red, 8 * (Nn * (1 + D * D) + 256 * D * D + D * D + 8));
-  ENSURE(ctx, ctx->wKeys, 4 * Nn);
-  ENSURE(ctx, ctx->cstart, 4 * ((size_t)n_cells + 1));
-  ENSURE(ctx, ctx->spos, 16 * Nn);
-  float* vpos = (float*)ctx->fireV.p;
-  float* vrot = vpos + Nn * D;
-  float* zt = vrot + Nn * A;
-  uint8_t* zfix = (uint8_t*)(zt + Nn * A);
-  HIPCHK(ctx, hipMemsetAsync(ctx->fireV.p, 0, 4 * Nn * (D + 2 * A) + Nn, st));
-  FireArgs f;
-  std::memset(&f, 0, sizeof(f));
-  f.n = N;
-  f.dim = D;
-  f.p.dt0 = (float)fire->dt;
-  f.p.alpha_init = (float)fire->alpha_init;
-  f.p.f_inc = (float)fire->f_inc;
-  f.p.f_dec = (float)fire->f_dec;
-  f.p.f_alpha = (float)fire->f_alpha;
-  f.p.dt_max = (float)(fire->dt * fire->dt_max_scale);
-  f.p.dt_min = (float)(fire->dt * fire->dt_min_scale);
-  f.p.n_min = fire->n_min;
-  f.p.n_bad_max = fire->n_bad_max;
-  f.st = (FireDev*)ctx->fireDev.p;
-  f.part = (double*)((char*)ctx->fireDev.p + sizeof(FireDev));
-  f.nparts = nparts;
-  f.force = p->force;
-  f.torque = zt;
-  f.fixed = zfix;
-  f.vel_pos = vpos;
-  f.vel_rot = vrot;
-  int32_t* moved = (int32_t*)((char*)ctx->fireDev.p + sizeof(FireDev) + 8 * (size_t)nparts);
-  FireDev h0;
-  std::memset(&h0, 0, sizeof(h0));
-  h0.dt = (float)fire->dt;
-  h0.alpha = (float)fire->alpha_init;
-  HIPCHK(ctx, hipMemcpyAsync(f.st, &h0, sizeof(h0), hipMemcpyHostToDevice, st));
-  double* per = (double*)ctx->red.p;
-  double* wper = per + Nn;
-  double* part = wper + Nn * D * D;
-  double* out = part + 256 * D * D;
+  if (N == 0) {
+    if (virial)
+      for (int q = 0; q < D * D; ++q) virial[q] = 0.0;
+    if (stats) std::memset(stats, 0, sizeof(*stats));
+    return JDEM_OK;
+  }
+  const size_t Nn = (size_t)N;
   PrecArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = N;
@@ -2134,27 +2094,14 @@ int jdem_precise_minimize(jdem_ctx* ctx, jdem_precise* p, const jdem_fire* fire,
   a.cidx = p->cidx;
   a.off = p->off;
   a.rad = p->rad;
-  a.k = p->k;
-  a.keys = (uint32_t*)ctx->wKeys.p;
-  a.starts = (int32_t*)ctx->cstart.p;
-  a.sp = (float4*)ctx->spos.p;
   a.force = p->force;
-  a.e_out = per;
-  a.w_out = nullptr;
-  a.moved = moved;
-  a.gmax_bits = &f.st->max_grad_bits;
-  // With the counting sort the re-sort is decided on the device: its kernels
-  // run only while a sphere has changed cell, so a step needs no host read
-  // of the flag.  The radix fallback keeps the host-side decision.
-  const bool gated = use_cell_sort(N, n_cells);
-  a.gated = gated ? 1 : 0;
-  // The Verlet list (with the counting sort only): pairs within r_i + r_j +
-  // skin; a partner is at most 1 + ceil(skin / h) cells away on an axis
-  // when h >= 2 r_max, so skin <= h keeps the build stencil at half-width
-  // 2 (cell differences in one byte of the entry), which must not wrap onto
-  // itself; slots take the entry's low 24 bits.
-  int32_t* vovf = nullptr;
-  if (gated && N > 0 && N < (int64_t)1 << 24 && p->skin > 0.0f && p->max_neighbors > 0) {
+  a.k = p->k;
+  // The Verlet list: pairs within r_i + r_j + skin; a partner is at most 1 +
+  // ceil(skin / h) cells away on an axis when h >= 2 r_max, so skin <= h
+  // keeps the build stencil at half-width 2 (cell differences in one byte of
+  // the entry), which must not wrap onto itself; slots take the entry's low
+  // 24 bits.  Grids much sparser than the spheres keep the stencil.
+  if (use_cell_sort(N, n_cells) && N < (int64_t)1 << 24 && p->skin > 0.0f && p->max_neighbors > 0) {
     float hmin = p->cell[0];
     for (int q = 1; q < D; ++q) hmin = std::min(hmin, p->cell[q]);
     const int sr = 1 + (int)std::ceil(p->skin / hmin);
@@ -2162,179 +2109,173 @@ int jdem_precise_minimize(jdem_ctx* ctx, jdem_precise* p, const jdem_fire* fire,
     for (int q = 0; q < D; ++q) fits = fits && p->dims[q] >= 2 * sr + 1;
     if (fits) {
       ENSURE(ctx, ctx->pvl, 4 * Nn * (size_t)p->max_neighbors);
-      ENSURE(ctx, ctx->pvaux, 4 * Nn * (size_t)D + 64);
+      ENSURE(ctx, ctx->wOld, 16 * Nn);
       a.vl = (int32_t*)ctx->pvl.p;
       a.vm = p->max_neighbors;
       a.vsr = sr;
       a.vcut = p->skin;
       a.vtrig = 0.25f * p->skin * p->skin;
-      a.boff = (float*)ctx->pvaux.p;
-      vovf = (int32_t*)(a.boff + D * Nn);
-      a.vovf = vovf;
-      HIPCHK(ctx, launch_fill_i32(vovf, 1, 0, st));
+      a.B = (float4*)ctx->wOld.p;
     }
   }
-  auto list_overflow = [&]() -> int {
-    int32_t ov = 0;
-    if (!vovf) return JDEM_OK;
-    HIPCHK(ctx, hipMemcpyAsync(&ov, vovf, sizeof(ov), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    return ov ? fail(ctx, JDEM_EINVAL, "a neighbour row exceeds max_neighbors") : JDEM_OK;
+  a.nparts = (int)prec_parts(N, a.vl != nullptr);
+  // optimiser scalars, then the stopping state and the device words
+  struct Dev {
+    FireDev fire;
+    PrecStop ps;
+    int32_t cur, moved, vovf;
+    unsigned rmax_bits;
   };
-  bool sorted = false;
-  double pe = 0.0, gmax = 0.0;
-  auto eval = [&](bool with_virial) -> int {
-    if ((gated || !sorted) && N > 0) {  // the cell list, rebuilt when a sphere changed cell
-      HIPCHK(ctx, launch_prec_keys(a, st));
-      uint32_t* sk = nullptr;
-      int32_t* perm = nullptr;
-      if (gated) {
-        HIPCHK(ctx, cell_sort_pairs(ctx, a.keys, N, n_cells, &sk, &perm, (int32_t*)ctx->cstart.p, st, moved));
-      } else {
-        HIPCHK(ctx, radix_sort_pairs(ctx, a.keys, N, nbits_for(n_cells), &sk, &perm, st));
-        HIPCHK(ctx, ws_launch_cell_starts(sk, N, n_cells, (int32_t*)ctx->cstart.p, st));
-      }
-      a.perm = perm;
-      sorted = true;
-    }
-    a.w_out = with_virial ? wper : nullptr;
-    HIPCHK(ctx, launch_prec_gather(a, st));
-    if (a.vl) HIPCHK(ctx, launch_prec_vbuild(a, st));
+  ENSURE(ctx, ctx->fireDev, sizeof(Dev));
+  ENSURE(ctx, ctx->red, 8 * (2 * (size_t)a.nparts + Nn * D * D + 256 * D * D + D * D) + 4 * (size_t)a.nparts);
+  for (int k = 0; k < 2; ++k) {
+    ENSURE(ctx, ctx->wP[k], 16 * Nn);
+    ENSURE(ctx, ctx->wV[k], 16 * Nn);
+    ENSURE(ctx, ctx->wQ[k], 16 * Nn);
+    a.S[k] = (float4*)ctx->wP[k].p;
+    a.V[k] = (float4*)ctx->wV[k].p;
+    a.C[k] = (int4*)ctx->wQ[k].p;
+  }
+  ENSURE(ctx, ctx->wF, 16 * Nn);
+  ENSURE(ctx, ctx->wKeys, 4 * Nn);
+  ENSURE(ctx, ctx->cstart, 4 * ((size_t)n_cells + 1));
+  Dev* dev = (Dev*)ctx->fireDev.p;
+  a.F = (float4*)ctx->wF.p;
+  a.keys = (uint32_t*)ctx->wKeys.p;
+  a.starts = (int32_t*)ctx->cstart.p;
+  a.cur = &dev->cur;
+  a.moved = &dev->moved;
+  a.vovf = &dev->vovf;
+  a.rmax_bits = &dev->rmax_bits;
+  a.stop = &dev->ps.stop;
+  a.st = &dev->fire;
+  a.part_e = (double*)ctx->red.p;
+  a.part_p = a.part_e + a.nparts;
+  double* wper = a.part_p + a.nparts;
+  double* part = wper + Nn * D * D;
+  double* out = part + 256 * D * D;
+  a.part_g = (unsigned*)(out + D * D);
+  FireP fp;
+  fp.dt0 = (float)fire->dt;
+  fp.alpha_init = (float)fire->alpha_init;
+  fp.f_inc = (float)fire->f_inc;
+  fp.f_dec = (float)fire->f_dec;
+  fp.f_alpha = (float)fire->f_alpha;
+  fp.dt_max = (float)(fire->dt * fire->dt_max_scale);
+  fp.dt_min = (float)(fire->dt * fire->dt_min_scale);
+  fp.n_min = fire->n_min;
+  fp.n_bad_max = fire->n_bad_max;
+  PrecStopP pp;
+  pp.pe_tol = pe_tol;
+  pp.pe_diff_tol = pe_diff_tol;
+  pp.force_tol = force_tol;
+  pp.dN = (double)N;
+  pp.max_steps = max_steps;
+  pp.stall_steps = p->stall_steps;
+  // optimiser state: dt = dt0, alpha = alpha_init, velocities zero (by the
+  // load); the first evaluation sorts: the flag starts set
+  Dev h;
+  std::memset(&h, 0, sizeof(h));
+  h.fire.dt = fp.dt0;
+  h.fire.alpha = fp.alpha_init;
+  h.ps.prev = INFINITY;
+  h.ps.first = 1;
+  h.moved = 1;
+  HIPCHK(ctx, hipMemcpyAsync(dev, &h, sizeof(h), hipMemcpyHostToDevice, st));
+  HIPCHK(ctx, launch_prec_load(a, st));
+
+  // the re-sort (its kernels return at once while *moved is clear), the force
+  auto eval = [&](double* w_out) -> int {
+    CellSort srt;
+    HIPCHK(ctx, cell_sort_begin(ctx, N, n_cells, &srt, st));
+    a.cnt = srt.cnt;
+    a.arr = srt.arr;
+    a.pairs = srt.pairs;
+    a.skeys = srt.sk;
+    HIPCHK(ctx, launch_prec_keys(a, st));
+    HIPCHK(ctx, cell_sort_starts(ctx, srt, n_cells, (int32_t*)ctx->cstart.p, st, a.moved));
+    HIPCHK(ctx, launch_prec_permute(a, st));
+    a.w_out = w_out;
     const int sp = span_begin(ctx, 0, 0);  // the force kernel, for its roofline
-    HIPCHK(ctx, a.vl ? launch_prec_vforce(a, st) : launch_prec_force(a, st));
+    HIPCHK(ctx, launch_prec_force(a, st));
     span_end(ctx, sp);
-    if (N == 0) HIPCHK(ctx, hipMemsetAsync(&f.st->max_grad_bits, 0, sizeof(unsigned), st));  // else the gather clears it
-    HIPCHK(ctx, launch_fire_grad_max(f, st));
-    double h = 0.0;
-    if (N > 0) {
-      HIPCHK(ctx, launch_sum_f64(per, N, 1, 1, part, out, 256, st));
-      HIPCHK(ctx, hipMemcpyAsync(&h, out, 8, hipMemcpyDeviceToHost, st));
-    }
-    unsigned bits = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&bits, &f.st->max_grad_bits, sizeof(bits), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    float g;
-    std::memcpy(&g, &bits, sizeof(g));
-    pe = h;
-    gmax = (double)g;
-    return list_overflow();
+    return JDEM_OK;
   };
-  // the first evaluation sorts: the flag starts set
-  HIPCHK(ctx, launch_fill_i32(moved, 1, 1, st));
-  int rc = eval(false);
-  if (rc) return rc;
-  double prev = INFINITY;
-  int64_t steps = 0;
-  const double tiny = 2.2250738585072014e-308;
-  const double dN = (double)std::max<int64_t>(N, 1);
-  // progress: a new low of max|F|, or of the energy by more than 1e-13 of it
-  double best_g = gmax, best_e = pe;
-  int64_t best_at = 0;
-  if (gated && N > 0) {
-    // The stopping tests run on the device (k_prec_check before every
-    // update; every kernel after a stop returns at once), so the host reads
-    // the loop's state once per chunk of iterations, not once per iteration.
-    PrecStop* ps = (PrecStop*)((char*)ctx->fireDev.p + sizeof(FireDev) + 8 * (size_t)nparts + 64);
-    PrecStop h_ps;
-    std::memset(&h_ps, 0, sizeof(h_ps));
-    h_ps.prev = INFINITY;
-    h_ps.first = 1;
-    HIPCHK(ctx, hipMemcpyAsync(ps, &h_ps, sizeof(h_ps), hipMemcpyHostToDevice, st));
-    PrecStopP pp;
-    pp.pe_tol = pe_tol;
-    pp.pe_diff_tol = pe_diff_tol;
-    pp.force_tol = force_tol;
-    pp.dN = dN;
-    pp.max_steps = max_steps;
-    pp.stall_steps = p->stall_steps;
-    a.stop = &ps->stop;
-    f.stop = &ps->stop;
-    constexpr int kChunk = 64;
-    while (true) {
-      for (int k = 0; k < kChunk; ++k) {
-        HIPCHK(ctx, launch_prec_check(ps, out, &f.st->max_grad_bits, pp, st));
-        HIPCHK(ctx, launch_fire_power(f, st));
-        HIPCHK(ctx, launch_fire_decide(f, st));
-        HIPCHK(ctx, launch_prec_move(f, a, st));
-        HIPCHK(ctx, launch_fire_commit(f, st));
-        // the evaluation (cell list re-sorted while a sphere changed cell)
-        HIPCHK(ctx, launch_prec_keys(a, st));
-        uint32_t* sk = nullptr;
-        int32_t* perm = nullptr;
-        HIPCHK(ctx, cell_sort_pairs(ctx, a.keys, N, n_cells, &sk, &perm, (int32_t*)ctx->cstart.p, st, moved));
-        a.perm = perm;
-        HIPCHK(ctx, launch_prec_gather(a, st));
-        if (a.vl) HIPCHK(ctx, launch_prec_vbuild(a, st));
-        const int sp = span_begin(ctx, 0, k);
-        HIPCHK(ctx, a.vl ? launch_prec_vforce(a, st) : launch_prec_force(a, st));
-        span_end(ctx, sp);
-        HIPCHK(ctx, launch_fire_grad_max(f, st));
-        HIPCHK(ctx, launch_sum_f64(per, N, 1, 1, part, out, 256, st));
-      }
-      HIPCHK(ctx, hipMemcpyAsync(&h_ps, ps, sizeof(h_ps), hipMemcpyDeviceToHost, st));
-      HIPCHK(ctx, hipStreamSynchronize(st));
-      rc = list_overflow();
-      if (rc) return rc;
-      if (h_ps.stop) break;
-    }
-    steps = h_ps.steps;
-    pe = h_ps.pe;
-    gmax = h_ps.gmax;
-    a.stop = nullptr;
-    f.stop = nullptr;
-  }
-  while (!(gated && N > 0) && steps < max_steps) {
-    const bool conv_pe = std::fabs(pe / dN) <= pe_tol;
-    const double denom = std::max(std::max(std::fabs(pe), std::fabs(prev)), tiny);
-    const bool conv_rel = std::fabs(pe - prev) / denom < pe_diff_tol;
-    if (gmax < best_g) best_g = gmax, best_at = steps;
-    if (pe < best_e - 1e-13 * std::fabs(best_e)) best_e = pe, best_at = steps;
-    const bool stalled = p->stall_steps > 0 && steps - best_at >= p->stall_steps;
-    if (conv_pe || conv_rel || gmax <= force_tol || stalled) break;
-    HIPCHK(ctx, launch_fire_power(f, st));
-    HIPCHK(ctx, launch_fire_decide(f, st));
-    if (!gated) HIPCHK(ctx, launch_fill_i32(moved, 1, 0, st));
-    HIPCHK(ctx, launch_prec_move(f, a, st));
-    HIPCHK(ctx, launch_fire_commit(f, st));
-    prev = pe;
-    if (!gated) {
-      // a sphere that left its cell needs a new cell list before the evaluation
-      int32_t mv = 0;
-      HIPCHK(ctx, hipMemcpyAsync(&mv, moved, sizeof(mv), hipMemcpyDeviceToHost, st));
-      HIPCHK(ctx, hipStreamSynchronize(st));
-      if (mv) sorted = false;
-    }
-    rc = eval(false);
-    if (rc) return rc;
-    ++steps;
-  }
-  if (a.vl) {
-    // list mode: fold the offsets back into [0, h) (a rebuild) for the caller
-    HIPCHK(ctx, launch_fill_i32(moved, 1, 1, st));
-    rc = eval(virial != nullptr);
-    if (rc) return rc;
-  }
-  if (virial) {
-    if (!a.vl) rc = eval(true);  // same configuration: the virial of the final state
-    if (rc) return rc;
-    double w9[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (N > 0) {
-      HIPCHK(ctx, launch_sum_f64(wper, N, D * D, D * D, part, out, 256, st));
-      HIPCHK(ctx, hipMemcpyAsync(w9, out, 8 * (size_t)(D * D), hipMemcpyDeviceToHost, st));
-      HIPCHK(ctx, hipStreamSynchronize(st));
-    }
-    for (int q = 0; q < D * D; ++q) virial[q] = w9[q];
-  }
-  if (stats) {
-    FireDev h;
-    HIPCHK(ctx, hipMemcpyAsync(&h, f.st, sizeof(h), hipMemcpyDeviceToHost, st));
+  auto read_dev = [&]() -> int {
+    HIPCHK(ctx, hipMemcpyAsync(&h, dev, sizeof(h), hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
+    return h.vovf ? fail(ctx, JDEM_EINVAL, "a neighbour row exceeds max_neighbors") : JDEM_OK;
+  };
+  int rc = eval(nullptr);
+  if (rc) return rc;
+  // The stopping tests run on the device before every update (every kernel
+  // after a stop returns at once), so the host reads the loop's state once
+  // per chunk of iterations.  The iteration after the last update only tests.
+  constexpr int64_t kChunk = 64;
+  int64_t steps = 0;
+  do {
+    const int64_t todo = std::min(kChunk, max_steps - steps + 1);
+    for (int64_t k = 0; k < todo; ++k) {
+      HIPCHK(ctx, launch_prec_update(a, &dev->ps, pp, fp, st));
+      if (k + 1 < todo || steps + todo <= max_steps) {
+        rc = eval(nullptr);
+        if (rc) return rc;
+      }
+    }
+    rc = read_dev();
+    if (rc) return rc;
+    steps = h.ps.steps;
+  } while (!h.ps.stop);
+  const double power = h.fire.power;
+  if (virial || a.vl) {
+    // list mode: the offsets folded back into [0, h) (a rebuild) for the
+    // caller; the virial, energy and max|F| of that configuration
+    a.stop = nullptr;
+    if (a.vl) HIPCHK(ctx, launch_fill_i32(a.moved, 1, 1, st));
+    rc = eval(virial ? wper : nullptr);
+    if (rc) return rc;
+    HIPCHK(ctx, launch_prec_total(a, &dev->ps, st));
+    if (virial) {
+      HIPCHK(ctx, launch_sum_f64(wper, N, D * D, D * D, part, out, 256, st));
+      HIPCHK(ctx, hipMemcpyAsync(virial, out, 8 * (size_t)(D * D), hipMemcpyDeviceToHost, st));
+    }
+    rc = read_dev();
+    if (rc) return rc;
+  }
+  HIPCHK(ctx, launch_prec_store(a, st));
+  if (stats) {
     stats->steps = steps;
-    stats->pe = pe / dN;
-    stats->max_grad = gmax;
-    stats->power = h.power;
+    stats->pe = h.ps.pe / (double)N;
+    stats->max_grad = h.ps.gmax;
+    stats->power = power;
     stats->overflow = 0;
   }
+  return JDEM_OK;
+}
+
+int jdem_precise_import(jdem_ctx* ctx, const double* pos, int64_t n, int32_t dim, const double* box_edge,
+                        const double* cell_edge, const float* cell_hi, const int32_t* dims, int32_t* cidx,
+                        float* off) {
+  if (!ctx) return JDEM_EINVAL;
+  if ((dim != 2 && dim != 3) || n < 0 || !box_edge || !cell_edge || !cell_hi || !dims ||
+      (n > 0 && (!pos || !cidx || !off)))
+    return fail(ctx, JDEM_EINVAL, "bad argument");
+  for (int q = 0; q < dim; ++q)
+    if (dims[q] < 1) return fail(ctx, JDEM_EINVAL, "dims < 1");
+  (void)hipSetDevice(ctx->device);
+  HIPCHK(ctx, launch_prec_import(pos, n, dim, box_edge, cell_edge, cell_hi, dims, cidx, off, ctx->stream));
+  return JDEM_OK;
+}
+
+int jdem_precise_export(jdem_ctx* ctx, const int32_t* cidx, const float* off, int64_t n, int32_t dim,
+                        const double* box_edge, const double* cell_edge, const float* cell_hi, const int32_t* dims,
+                        double* pos) {
+  if (!ctx) return JDEM_EINVAL;
+  if ((dim != 2 && dim != 3) || n < 0 || !box_edge || !cell_edge || !cell_hi || !dims ||
+      (n > 0 && (!pos || !cidx || !off)))
+    return fail(ctx, JDEM_EINVAL, "bad argument");
+  (void)hipSetDevice(ctx->device);
+  HIPCHK(ctx, launch_prec_export(cidx, off, n, dim, box_edge, cell_edge, cell_hi, dims, pos, ctx->stream));
   return JDEM_OK;
 }
 

@@ -508,11 +508,8 @@ size_t cell_sort_sum_words(int64_t n_cells) {
 // the totals comes first (a block reads them all).
 constexpr int kScanDirect = 1024;
 
-// The passes after the count: scan, placement, rank (+ gather).
-template <class Real>
-hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells, int32_t* starts,
-                     const Real* pos, const Real* rad, int dim, Real4<Real>* spos, hipStream_t s,
-                     const int32_t* gate) {
+// The passes after the count: scan; placement and rank (+ gather).
+hipError_t cs_starts(const CellSort& cs, int64_t n_cells, int32_t* starts, hipStream_t s, const int32_t* gate) {
   const int nchunks = (int)((n_cells + 1 + SC_CHUNK - 1) / SC_CHUNK);
   if (nchunks > 1)
     hipLaunchKernelGGL(k_scan_totals, dim3(nchunks), dim3(kBlock), 0, s, (const uint32_t*)cs.cnt, n_cells, cs.sums,
@@ -521,6 +518,14 @@ hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_
   if (scanned) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, cs.sums, nchunks, gate);
   hipLaunchKernelGGL(k_cs_scan, dim3(nchunks), dim3(kBlock), 0, s, cs.cnt, n_cells, cs.sums, scanned ? 1 : 0, starts,
                      gate);
+  return hipGetLastError();
+}
+template <class Real>
+hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells, int32_t* starts,
+                     const Real* pos, const Real* rad, int dim, Real4<Real>* spos, hipStream_t s,
+                     const int32_t* gate) {
+  const hipError_t e = cs_starts(cs, n_cells, starts, s, gate);
+  if (e != hipSuccess) return e;
   if (n > 0) {
     hipLaunchKernelGGL(k_cs_place, dim3(nblocks(n)), dim3(kBlock), 0, s, keys, n, starts, cs.arr, cs.pairs, gate);
     hipLaunchKernelGGL((k_cs_rank<Real>), dim3(nblocks(n)), dim3(kBlock), 0, s, cs.pairs, n, starts, cs.sk, cs.perm,
@@ -773,6 +778,12 @@ hipError_t cell_sort_end_run(jdem_ctx* ctx, const CellSort& cs, const uint32_t* 
                              int32_t* starts, const Real* pos, const Real* rad, int dim, Real4<Real>* spos,
                              hipStream_t s, const int32_t* gate) {
   const hipError_t e = cs_finish<Real>(cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, gate);
+  ctx->cscnt_clear = e == hipSuccess;
+  return e;
+}
+hipError_t cell_sort_starts(jdem_ctx* ctx, const CellSort& cs, int64_t n_cells, int32_t* starts, hipStream_t s,
+                            const int32_t* gate) {
+  const hipError_t e = cs_starts(cs, n_cells, starts, s, gate);
   ctx->cscnt_clear = e == hipSuccess;
   return e;
 }

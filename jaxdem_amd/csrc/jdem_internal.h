@@ -98,8 +98,8 @@ struct jdem_ctx {
   jdem::Buf ccnt;
   // clumps: members per clump (CSR), lab positions, levers, member totals
   jdem::Buf cl_start, cl_members, plab, ppr, ftot, ttot, crefl;
-  // the precision form's Verlet list and its per-sphere build state
-  jdem::Buf pvl, pvaux;
+  // the precision form's Verlet list
+  jdem::Buf pvl;
   // every scratch buffer of the context, for accounting and release
   std::vector<jdem::Buf*> bufs();
   size_t scratch_bytes();
@@ -299,6 +299,10 @@ hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, i
 // atomic returned; cell_sort_end runs the remaining passes on those keys (and,
 // with spos, gathers the sorted (x, r)).
 hipError_t cell_sort_begin(jdem_ctx* ctx, int64_t n, int64_t n_cells, CellSort* cs, hipStream_t s);
+// cell_sort_starts only scans the counts into starts: the caller places its
+// elements itself.
+hipError_t cell_sort_starts(jdem_ctx* ctx, const CellSort& cs, int64_t n_cells, int32_t* starts, hipStream_t s,
+                            const int32_t* gate);
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                          int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
@@ -692,7 +696,7 @@ struct FireDev {
   float new_dt, new_alpha, dt_rev, vs;
   double power;
   unsigned max_grad_bits;  // max |grad| component as float bits
-  int pad;
+  float dt_used;           // precision form: dt of the update just decided (dt is the next one's)
 };
 struct FireArgs {
   int64_t n;
@@ -744,42 +748,62 @@ struct PrecArgs {
   int dims[3];   // cells per axis (periodic)
   float h[3];    // cell edges: h + hlo as an unevaluated float pair
   float hlo[3];
+  // caller's arrays, by sphere
   int32_t* cidx; // (N, D) cell of each sphere
   float* off;    // (N, D) position inside the cell, [0, h)
   const float* rad;
+  float* force;  // (N, D)
   float k;
-  uint32_t* keys;        // cell key of each sphere
-  const int32_t* perm;   // cell-sorted position -> sphere
-  const int32_t* starts; // first sorted position of each cell (n_cells + 1)
-  float4* sp;            // cell-sorted (offset, radius), gathered per evaluation
-  float* force;          // (N, D)
-  double* e_out;         // (N) half the pair energies of each sphere
-  double* w_out;         // (N, D*D) half the pair virials, or null
-  int32_t* moved;        // set when a sphere changed cell
-  unsigned* gmax_bits;   // max|F| word of the FIRE state, cleared by the gather
-  int gated;             // 1: the key kernel runs only while *moved, and the gather clears *moved
+  // state by cell-sorted slot; S, V, C swap at a re-sort (word *cur)
+  float4* S[2];  // offset, radius
+  float4* V[2];  // FIRE velocity
+  int4* C[2];    // cell, sphere id
+  float4* F;
+  float4* B;     // list mode: offsets at the build
+  int32_t* cur;
+  int32_t* moved;        // a re-sort is due (or, until the next decision, done)
   const int32_t* stop;   // when set, every kernel returns at once once *stop is set
-  // Verlet list (vl set): *moved means "rebuild the list", raised when a
-  // sphere has moved skin / 2 since the build; the fold of the offsets, the
-  // sort and the list build run only then, and the list force clears *moved
-  int32_t* vl;           // (N, vm) by sorted slot: partner slot | cell difference << 24, -1 ends a row
+  unsigned* rmax_bits;   // largest radius
+  // sort
+  uint32_t* keys;        // cell key of each slot
+  int32_t* cnt;
+  int32_t* arr;
+  uint2* pairs;
+  uint32_t* skeys;       // keys in the new order
+  const int32_t* starts; // first sorted position of each cell (n_cells + 1)
+  // partials of a force evaluation
+  FireDev* st;
+  int nparts;
+  double* part_e;
+  double* part_p;
+  unsigned* part_g;
+  double* w_out;         // (N, D*D) half the pair virials by slot, or null
+  // Verlet list (vl set): *moved is raised when a sphere has moved skin / 2
+  // since the build; the fold of the offsets, the sort and the list build run
+  // only then
+  int32_t* vl;           // (vm, N) slot-major: partner slot | cell difference << 24, -1 ends a row
   int vm;
   int vsr;               // stencil half-width of the list build (1 or 2)
   float vcut;            // list reach beyond r_i + r_j (the skin)
   float vtrig;           // (skin / 2)^2
-  float* boff;           // (N, D) offsets at the build
   int32_t* vovf;         // set when a row would exceed vm
 };
-// the stopping tests of one FIRE iteration from the last evaluation's float64
-// energy sum and max|F| word; stops, or counts the update that follows
-hipError_t launch_prec_check(PrecStop* ps, const double* pe_sum, const unsigned* gmax_bits, const PrecStopP& p,
-                             hipStream_t s);
+// blocks (partials) of a force evaluation
+unsigned prec_parts(int64_t n, bool list);
+hipError_t launch_prec_load(const PrecArgs& a, hipStream_t s);
+hipError_t launch_prec_store(const PrecArgs& a, hipStream_t s);
 hipError_t launch_prec_keys(const PrecArgs& a, hipStream_t s);
-hipError_t launch_prec_gather(const PrecArgs& a, hipStream_t s);
+// placement and permute into the new order and, in list mode, the list build
+hipError_t launch_prec_permute(const PrecArgs& a, hipStream_t s);
 hipError_t launch_prec_force(const PrecArgs& a, hipStream_t s);
-hipError_t launch_prec_vbuild(const PrecArgs& a, hipStream_t s);
-hipError_t launch_prec_vforce(const PrecArgs& a, hipStream_t s);
-hipError_t launch_prec_move(const FireArgs& f, const PrecArgs& a, hipStream_t s);
+// stopping tests and FIRE scalars from the last evaluation, then the update
+hipError_t launch_prec_update(const PrecArgs& a, PrecStop* ps, const PrecStopP& p, const FireP& fp, hipStream_t s);
+// ps->pe, ps->gmax of the last evaluation
+hipError_t launch_prec_total(const PrecArgs& a, PrecStop* ps, hipStream_t s);
+hipError_t launch_prec_import(const double* pos, int64_t n, int D, const double* L, const double* h, const float* hi,
+                              const int32_t* dims, int32_t* cidx, float* off, hipStream_t s);
+hipError_t launch_prec_export(const int32_t* cidx, const float* off, int64_t n, int D, const double* L,
+                              const double* h, const float* hi, const int32_t* dims, double* pos, hipStream_t s);
 
 inline unsigned nblocks(int64_t n, int b = kBlock) { return (unsigned)((n + b - 1) / b); }
 
