@@ -800,6 +800,210 @@ __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
   }
 }
 
+// The list build of one system with a group of G lanes per particle:
+// k_nlist_work's chain of column bounds and candidates is serial per lane, and
+// below ~10^5 particles there are not enough wavefronts to hide it (154 us for
+// 37 k spheres of 31 neighbours, most of a rebuild; here 44 us).  A workgroup builds the rows
+// of one wavefront's 64 slots: each lane loads one stencil column's bounds, a
+// scan numbers the candidates, G of them are tested at a time and those within
+// the cutoff appended in candidate order; the old springs are looked up one
+// per lane; the new springs' places are a scan over the 64 slots.
+// G = 16 in 3D (9 columns of 6 to 20 candidates), 8 in 2D (3 columns of 7).
+template <int D>
+constexpr int nlist_group() {
+  return D == 3 ? 16 : 8;
+}
+constexpr int kRowGrp = 64;  // row slots collected in LDS
+
+// position of the r-th set bit of the words (r below their count)
+JD int select_bit(const uint64_t* w, int n_words, int r) {
+  for (int q = 0; q < n_words; ++q) {
+    const int c = __popcll(w[q]);
+    if (r < c) {
+      uint64_t b = w[q];
+      for (; r > 0; --r) b &= b - 1ull;
+      return q * 64 + __ffsll((unsigned long long)b) - 1;
+    }
+    r -= c;
+  }
+  return -1;
+}
+
+// MW: live words of a row (1, or 4 for rows of more than 64 slots).  Eight
+// waves per SIMD (64 VGPRs) let two 3D workgroups share a CU.
+template <int D, bool PER, int MW>
+__global__ void __launch_bounds__(64 * nlist_group<D>()) __attribute__((amdgpu_waves_per_eu(8, 8)))
+k_nlist_group(NLW a) {
+  if (a.gate && *a.gate == 0) return;  // uniform over the grid
+  constexpr int G = nlist_group<D>();
+  __shared__ int32_t rows[kRowGrp][64];
+  __shared__ int row_cnt[64], new_cnt[64], new_off[64];
+  const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1), lane = tid & 63;
+  const uint64_t below = (1ull << l) - 1ull;
+  const int64_t n = a.n;
+  const int64_t nreg = (n + 63) / 64;
+  for (int64_t reg = xcd_tile(blockIdx.x, gridDim.x); reg < nreg; reg += gridDim.x) {
+    const int64_t b = reg * 64 + p;
+    const bool active = b < n;
+    int count = 0;
+    if (active) {
+      const GridP& grid = a.grid;
+      const uint32_t key = a.skeys[b];
+      const Vec<D> xi = xyz<D>(a.P4[b]);
+      const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
+      int c0, c1, cf;
+      if (D == 3) {
+        cf = (int)(key % (uint32_t)d2);
+        const uint32_t r = key / (uint32_t)d2;
+        c1 = (int)(r % (uint32_t)d1);
+        c0 = (int)(r / (uint32_t)d1);
+      } else {
+        cf = (int)(key % (uint32_t)d1);
+        c0 = (int)(key / (uint32_t)d1);
+        c1 = 0;
+      }
+      const int sr = grid.sr, dF = (D == 3) ? d2 : d1;
+      int r0a, r0b, r1a, r1b;
+      stencil_runs(PER, cf, sr, dF, r0a, r0b, r1a, r1b);
+      const int n1 = (D == 3) ? (PER ? min(sr, d1 - sr - 1) : sr) + sr + 1 : 1;
+      const int ncol = ((PER ? min(sr, d0 - sr - 1) : sr) + sr + 1) * n1;
+      const bool chk_bond = (!a.isb) && a.bond_w > 0;
+      const int64_t ib = chk_bond ? (int64_t)a.orig[b] : 0;
+      const int32_t* __restrict__ starts = a.starts;
+      for (int cb = 0; cb < ncol; cb += G) {
+        const int col = cb + l;
+        int s0 = 0, len0 = 0, s1 = 0, len1 = 0;
+        if (col < ncol) {
+          const int cx = stencil_cell(PER, c0, (D == 3 ? col / n1 : col) - sr, d0);
+          const int cy = (D == 3) ? stencil_cell(PER, c1, col % n1 - sr, d1) : 0;
+          if (cx >= 0 && cy >= 0) {
+            const int64_t base = (D == 3) ? ((int64_t)cx * d1 + cy) * d2 : (int64_t)cx * d1;
+            s0 = starts[base + r0a];
+            len0 = starts[base + r0b + 1] - s0;
+            if (r1b >= r1a) {
+              s1 = starts[base + r1a];
+              len1 = starts[base + r1b + 1] - s1;
+            }
+          }
+        }
+        int incl = len0 + len1;
+#pragma unroll
+        for (int d = 1; d < G; d <<= 1) {
+          const int t = __shfl_up(incl, d, G);
+          if (l >= d) incl += t;
+        }
+        const int pre = incl - (len0 + len1);
+        const int total = __shfl(incl, G - 1, G);
+        for (int c8 = 0; c8 < total; c8 += G) {
+          const int cand = c8 + l;
+          int q = 0;
+#pragma unroll
+          for (int st = G / 2; st > 0; st >>= 1) q += __shfl(pre, q + st, G) <= cand ? st : 0;
+          const int o = cand - __shfl(pre, q, G), f0 = __shfl(s0, q, G), n_0 = __shfl(len0, q, G),
+                    f1 = __shfl(s1, q, G);
+          const int k = (o < n_0 ? f0 + o : f1 + (o - n_0));
+          bool hit = false;
+          if (cand < total && k != (int)b) {
+            const Vec<D> xk = xyz<D>(a.P4[k]);
+            const float dsq = dist_sq<PER>(xi, xk, a.dom);
+            hit = dsq <= a.cutoff_sq;
+            if (hit && chk_bond) hit = !bonded_o(a.bond_id, a.bond_w, ib, a.orig[k]);
+          }
+          const uint64_t m = (__ballot(hit) >> (lane & ~(G - 1))) & ((1ull << G) - 1ull);
+          if (hit) {
+            const int t = count + __popcll(m & below);
+            if (t < kRowGrp)
+              rows[t][p] = k;
+            else if (t < a.M)
+              a.nl[(int64_t)t * n + b] = k;
+          }
+          count += __popcll(m);
+        }
+      }
+    }
+    const int c = min(count, a.M);
+    if (l == 0) row_cnt[p] = active ? c : -1;
+    __syncthreads();
+    {  // the collected slots, 64 consecutive particles at a time
+      const int64_t bw = reg * 64 + lane;
+      const int cw = row_cnt[lane];
+      for (int s = tid >> 6; s < kRowGrp; s += G) {
+        if (s < cw) a.nl[(int64_t)s * n + bw] = rows[s][lane];
+        if (!__any(s + G < cw)) break;
+      }
+    }
+    if (active && l == 0) {
+      if (count < a.M) a.nl[(int64_t)count * n + b] = -1;
+      if (count > a.M) atomicOr(a.overflow, 1);
+    }
+    if (a.live) {
+      // history (remap_row): each live old spring goes to the slot of the new
+      // row that lists the same two particles, if any
+      const bool go = active && a.remap != 0;
+      const int64_t ob = go ? (a.cidx ? (int64_t)a.cidx[b] : (int64_t)a.src[b]) : 0;
+      const int64_t os = a.cidx ? a.ostride : n;
+      // start of the old springs, read before any lane writes new offsets
+      const int64_t obase = (go && a.old_W) ? (ob & ~(int64_t)63) * a.M + __float_as_int(a.old_W[ob].w) : 0;
+      uint64_t old[MW], out[MW];
+      int n_old = 0;
+#pragma unroll
+      for (int w = 0; w < MW; ++w) {
+        old[w] = go && w < a.W64 ? a.old_live[(int64_t)w * os + ob] : 0ull;
+        out[w] = 0ull;
+        n_old += __popcll(old[w]);
+      }
+      auto new_slot = [&](int r) {  // of the r-th live old spring, or -1
+        const int32_t o = a.old_nl[(int64_t)select_bit(old, MW, r) * os + ob];
+        if (o < 0) return -1;
+        const int32_t tgt = a.inv[o];
+        for (int s = 0; s < c; ++s)
+          if ((s < kRowGrp ? rows[s][p] : a.nl[(int64_t)s * n + b]) == tgt) return s;
+        return -1;
+      };
+      const int first = l < n_old ? new_slot(l) : -1;  // kept: rows rarely carry more than G springs
+      for (int r = l; r < n_old; r += G) {
+        const int s = r == l ? first : new_slot(r);
+        if (s >= 0)
+#pragma unroll
+          for (int w = 0; w < MW; ++w) out[w] |= (s >> 6) == w ? 1ull << (s & 63) : 0ull;
+      }
+#pragma unroll
+      for (int w = 0; w < MW; ++w) {
+        if (w >= a.W64) break;  // uniform
+#pragma unroll 1
+        for (int d = 1; d < G; d <<= 1) out[w] |= (uint64_t)__shfl_xor((unsigned long long)out[w], d, G);
+      }
+      if (l == 0) {
+        int k = 0;
+#pragma unroll
+        for (int w = 0; w < MW; ++w) k += __popcll(out[w]);
+        new_cnt[p] = k;
+      }
+      __syncthreads();  // old_W is read, the counts are there
+      if (tid < 64) {
+        const int off = wave_exclusive_scan(new_cnt[tid], tid);
+        new_off[tid] = off;
+        const int64_t bw = reg * 64 + tid;
+        if (a.new_W && bw < n) a.new_W[bw].w = __int_as_float(off);
+      }
+      __syncthreads();
+      const int64_t wbase = (b & ~(int64_t)63) * a.M + new_off[p];
+      for (int r = l; r < n_old; r += G) {
+        const int s = r == l ? first : new_slot(r);
+        if (s < 0) continue;
+        const int rank = MW == 1 ? __popcll(out[0] & ((1ull << s) - 1ull))
+                                 : rank_below(out[0], out[MW > 1 ? 1 : 0], out[MW > 2 ? 2 : 0], out[MW > 3 ? 3 : 0], s);
+        const int64_t oi = a.old_W ? obase + r : (int64_t)r * os + ob;
+        a.xi[a.new_W ? wbase + rank : (int64_t)rank * n + b] = a.old_xi[oi];
+      }
+      if (active && l == 0)
+#pragma unroll
+        for (int w = 0; w < MW; ++w)
+          if (w < a.W64) a.live[(int64_t)w * n + b] = out[w];
+    }
+    __syncthreads();  // the next region reuses the LDS
+  }
+}
 
 
 __global__ void __launch_bounds__(kBlock) k_copy_f4(float4* __restrict__ d, const float4* __restrict__ s, int64_t n) {
@@ -1511,6 +1715,29 @@ hipError_t ws_launch_cell_starts(const uint32_t* skeys, int64_t n, int64_t n_cel
   hipLaunchKernelGGL(k_cell_starts, dim3(nblocks(n_cells + 1)), dim3(kBlock), 0, s, skeys, n, n_cells, starts);
   return hipGetLastError();
 }
+// From this many particles on a list is built by one lane per particle, which
+// takes fewer instructions but a longer chain.  A rebuild, group / lane, us:
+// 3D bidisperse 43 / 86 at 10 k, 58 / 87 at 37 k, 84 / 91 at 100 k, 207 / 154
+// at 400 k; log-normal radii 84 / 194, 138 / 211, 374 / 346; disks 43 / 56,
+// 58 / 59, 106 / 90.
+constexpr int64_t kNlistLane = 100000;
+
+template <int MW>
+void launch_nlist_group(const NLW& a, int dim, bool per, hipStream_t s) {
+  const dim3 g(nblocks(a.n, 64)), b(64 * (dim == 3 ? nlist_group<3>() : nlist_group<2>()));
+  if (dim == 3) {
+    if (per)
+      hipLaunchKernelGGL((k_nlist_group<3, true, MW>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((k_nlist_group<3, false, MW>), g, b, 0, s, a);
+  } else {
+    if (per)
+      hipLaunchKernelGGL((k_nlist_group<2, true, MW>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((k_nlist_group<2, false, MW>), g, b, 0, s, a);
+  }
+}
+
 hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s) {
   dim3 g(nblocks(a.n)), b(kBlock);
   const bool per = naive ? a.dom.kind == JDEM_DOMAIN_PERIODIC : a.grid.periodic != 0;
@@ -1532,6 +1759,11 @@ hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s) {
       hipLaunchKernelGGL((k_nlist_work<3, 2>), gs, b, 0, s, a);
     else
       hipLaunchKernelGGL((k_nlist_work<2, 2>), gs, b, 0, s, a);
+  } else if (a.n < kNlistLane) {
+    if (a.W64 <= 1)
+      launch_nlist_group<1>(a, dim, per, s);
+    else
+      launch_nlist_group<4>(a, dim, per, s);
   } else {
     if (dim == 3) {
       if (per)

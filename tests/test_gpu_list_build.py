@@ -1,0 +1,60 @@
+"""The list build with a group of lanes per particle where it can go wrong:
+fewer particles than a workgroup's 64 slots, a last workgroup nearly empty,
+more stencil columns than lanes, rows beyond the 64 slots kept in LDS, more
+live springs than lanes, rows of one and of four words of live bits, bonded
+pairs, a row limit that overflows, and the first size of the kernel with a
+lane per particle.  Several rebuilds with live springs: states, rows, springs
+and live bits equal the oracle bit for bit."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import jaxdem_amd as jd
+from oracle import jdem_oracle as O
+from tests import oracle_bridge as B
+from tests.test_gpu_parity import _compare_states, assert_bitwise, packed
+
+pytestmark = pytest.mark.gpu
+
+# dim, domain, N, volume fraction, skin, cell edge / largest diameter, radii, row limit, bonds
+CASES = [
+    (3, "periodic", 1, 0.5, 0.1, 1.0, (0.4, 0.6), None, False),
+    (3, "reflect", 63, 0.6, 0.2, 1.0, (0.4, 0.6), None, False),
+    (2, "periodic", 65, 0.8, 0.2, 1.0, (0.4, 0.6), None, True),
+    (3, "periodic", 257, 2.5, 0.3, 0.6, (0.4, 0.6), 100, False),  # rows of 75 slots, 25 columns
+    (2, "reflect", 700, 5.0, 0.4, 1.0, (0.1, 0.6), 250, True),  # rows of 102 slots, 39 springs
+    (3, "periodic", 2000, 0.7, 0.3, 0.4, (0.2, 0.6), 60, False),  # 49 columns
+    (2, "periodic", 1500, 0.9, 0.4, 0.3, (0.4, 0.6), 64, False),  # 7 columns of 7 cells
+    (3, "reflect", 1000, 0.8, 0.2, 1.0, (0.4, 0.6), 8, False),  # rows cut at 8 slots
+    (2, "reflect", 100001, 0.7, 0.2, 1.0, (0.4, 0.6), None, False),  # one lane per disk
+]
+
+
+@pytest.mark.parametrize("dim,domain,N,phi,skin,edge,rr,limit,bonds", CASES)
+def test_rebuilds_against_the_oracle(device, dim, domain, N, phi, skin, edge, rr, limit, bonds):
+    print(f"[list] dim={dim} {domain} N={N} phi={phi} edge={edge} limit={limit}", flush=True)
+    ids = None
+    if bonds:
+        ids = np.full((N, 2), -1, np.int64)
+        ids[:-1, 0], ids[1:, 1] = np.arange(1, N), np.arange(N - 1)
+    st, box = packed(N, dim, seed=N + dim, domain=domain, phi=phi, rr=rr, bonds=ids)
+    mats = [jd.Material.create("elasticfrict", density=1.0, young=1e2, poisson=0.3, mu=0.4, e=0.7, mu_r=0.05)]
+    diam = 2.0 * float(st.rad.max())
+    ckw = dict(state=st, cutoff=diam, skin=skin, max_neighbors=limit, secondary_collider_type="CellList",
+               secondary_collider_kw=dict(state=st, cell_size=edge * diam))
+    sy = jd.System.create(st.shape, dt=4e-3, domain_type=domain, domain_kw=dict(box_size=box, anchor=np.zeros(dim)),
+                          collider_type="NeighborList", collider_kw=ckw, force_model_type="springfriction",
+                          mat_table=jd.MaterialTable.from_materials(mats))
+    steps = 3 if N > 50000 else 30
+    nls = B.nl_state_of(st, sy)
+    ost = O.step(B.state_of(st), B.params_of(st, sy), steps, nls)
+    st2, sy2 = jd.System.step(st, sy, n=steps)
+    _compare_states(st2, ost, "list")
+    got = B.nl_state_of(st2, sy2)
+    assert got.n_build == nls.n_build and got.overflow == nls.overflow == (limit == 8)
+    assert nls.n_build >= (1 if N in (1, 100001) else 2)
+    assert np.array_equal(got.nl, nls.nl)
+    assert np.array_equal(got.live, nls.live)
+    assert_bitwise("springs", got.xi, np.where(nls.live[..., None], nls.xi, np.float32(0.0)))
