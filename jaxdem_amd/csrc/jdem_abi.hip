@@ -22,7 +22,7 @@ std::vector<Buf*> jdem_ctx::bufs() {
                            &cstart,  &cend,   &spos,     &nl_new,  &xi_new,  &live_new, &flags,  &red,
                            &nl_copy, &xi_copy, &live_copy, &wF,     &wT,      &wOld,     &wWpos, &wSrc,
                            &wInv,    &wKeys,  &fireV,    &fireDev, &segp,  &segid, &segflag, &wXiRank,
-                           &route,   &ccnt,   &cscnt,  &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl};
+                           &route,   &cscnt,  &cl_start, &cl_members, &plab, &ppr, &ftot, &ttot, &crefl, &pvl};
   for (int k = 0; k < 2; ++k)
     for (Buf* b : {&wP[k], &wV[k], &wW[k], &wQ[k], &wI[k], &wOrig[k], &wNl[k], &wXi[k], &wLive[k]}) all.push_back(b);
   return all;
@@ -829,7 +829,7 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
   // the step kernel keeps springs per wavefront
   if (hist && M > 0)
     HIPCHK(ctx, ws_launch_pack_springs(N, M, W64, R ? (const float4*)R->xi.p : F4(ctx->wXiRank),
-                                       U64(ctx->wLive[0]), F4(ctx->wXi[0]), F4(ctx->wW[0]), nullptr, nullptr, st));
+                                       U64(ctx->wLive[0]), F4(ctx->wXi[0]), F4(ctx->wW[0]), st));
 
   // --- rebuild at the current positions (neighbor_list.py:545-589) ---
   // Batches: only the systems that asked for a rebuild are re-sorted and
@@ -845,44 +845,59 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
   // positions of the other systems stay where they are.  No host round trip.
   int32_t* gate = (int32_t*)ctx->flags.p + 4;
   int32_t* events = (int32_t*)ctx->flags.p + 5;
-  auto rebuild_batch = [&]() -> int {
-    const int sp = span_begin(ctx, 2, 0);
-    HIPCHK(ctx, ws_launch_gated_zero(gate, (int32_t*)ctx->flags.p + 2, st));  // overflow of this build
-    HIPCHK(ctx, ws_launch_seg_modes(sg->n_seg, sg->seg_flag, sg->n_build, sg->seg_mode, st, gate, events));
-    HIPCHK(ctx, ws_launch_seg_prefix(sg->n_seg, sg->seg_mode, sg->offsets, sg->segp, sg->cpref, sg->ccref, sg->wpref,
-                                     st));
-    // springs of the wavefronts that hold a rebuilt system: per wave -> by rank
-    if (hist && M > 0)
-      HIPCHK(ctx, ws_launch_unpack_springs(N, M, W64, F4(ctx->wXi[xc]), U64(ctx->wLive[nlc]), F4(ctx->wW[cur]),
-                                           F4(ctx->wXiRank), sg->seg, sg->seg_mode, st, gate, sg->wpref, sg->offsets,
-                                           sg->n_seg));
-    RB r;
+  RB r;
+  RBPlan plan;
+  CellSort csort;
+  if (sg) {
+    // the counts are clear between the chains; cleared here, outside any capture
+    HIPCHK(ctx, cell_sort_begin(ctx, N, std::max<int64_t>(sg->total_cells, 1), &csort, st));
     std::memset(&r, 0, sizeof(r));
     r.n = N;
-    r.fn = -1;  // the flagged-particle count is cpref[n_seg] on the device
     r.n_seg = sg->n_seg;
     r.dim = D;
-    r.gate = gate;
+    r.go = (int32_t*)ctx->flags.p + 7;
     r.M = M;
     r.W64 = W64;
     r.seg = sg->seg;
     r.segp = sg->segp;
-    r.seg_mode = sg->seg_mode;
     r.offsets = sg->offsets;
+    r.seg_mode = sg->seg_mode;
     r.cpref = sg->cpref;
     r.ccref = sg->ccref;
+    r.wpref = sg->wpref;
+    r.old4 = F4(ctx->wOld);
+    r.keep_xi = F4(ctx->wXiRank);
+    r.keys_c = (uint32_t*)ctx->wKeys.p;
+    r.slot_c = I32(ctx->cend);
+    r.cnt = csort.cnt;
+    r.arr = csort.arr;
+    r.pairs = csort.pairs;
+    r.starts = I32(ctx->cstart);
+    r.sk = csort.sk;
+    r.tlive = I32(ctx->wWpos);
+    r.inv = I32(ctx->wInv);
+    r.isb = sys->interact_same_bond_id;
+    r.bond_w = s.bond_width;
+    r.bond_id = s.bond_id;
+    r.overflow = (int32_t*)ctx->flags.p + 2;
+    plan.gate = gate;
+    plan.go = (int32_t*)ctx->flags.p + 7;
+    plan.overflow = r.overflow;
+    plan.events = events;
+    plan.seg_flag = sg->seg_flag;
+    plan.n_build = sg->n_build;
+  }
+  auto rebuild_batch = [&]() -> int {
+    const int sp = span_begin(ctx, 2, 0);
     r.P = F4(ctx->wP[cur]);
     r.V = F4(ctx->wV[cur]);
     r.W = F4(ctx->wW[cur]);
     r.Q = F4(ctx->wQ[set]);
     r.I = F4(ctx->wI[set]);
-    r.old4 = F4(ctx->wOld);
     r.orig = I32(ctx->wOrig[set]);
     r.nl = I32(ctx->wNl[nlc]);
-    r.live = hist ? U64(ctx->wLive[nlc]) : nullptr;
-    r.xi = F4(ctx->wXiRank);
-    r.keys_c = (uint32_t*)ctx->wKeys.p;
-    r.slot_c = I32(ctx->cend);
+    r.live = hist && M > 0 ? U64(ctx->wLive[nlc]) : nullptr;
+    r.xi = F4(ctx->wXi[xc]);
     // staging: buffers that hold nothing live during a batch rebuild
     r.tP = F4(ctx->wP[1 - cur]);
     r.tV = F4(ctx->wV[1 - cur]);
@@ -890,64 +905,14 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
     r.tQ = F4(ctx->wQ[1 - set]);
     r.tI = F4(ctx->wI[1 - set]);
     r.torig = I32(ctx->wOrig[1 - set]);
-    r.cs = I32(ctx->wWpos);
     r.tnl = I32(ctx->wNl[1 - nlc]);
-    r.tlive = U64(ctx->wLive[1 - nlc]);
     r.txi = F4(ctx->wXi[1 - xc]);
-    r.inv = I32(ctx->wInv);
-    r.cidx = I32(ctx->wSrc);
-    HIPCHK(ctx, ws_launch_hash_flagged(r, D, st));
-    uint32_t* sk = nullptr;
-    int32_t* perm = nullptr;
-    // counting sort by compact cell, sized for every particle and every cell
-    // of the batch; the kernels read the flagged particle and cell counts on
-    // the device
-    HIPCHK(ctx, cell_sort_dev(ctx, r.keys_c, N, std::max<int64_t>(sg->total_cells, 1), sg->cpref + sg->n_seg,
-                              sg->ccref + sg->n_seg, &sk, &perm, st, gate));
-    r.perm = perm;
-    HIPCHK(ctx, ws_launch_place(r, sk, I32(ctx->cstart), st));
-    if (M > 0) {
-      NLW b;
-      std::memset(&b, 0, sizeof(b));
-      b.n = N;
-      b.M = M;
-      b.isb = sys->interact_same_bond_id;
-      b.bond_w = s.bond_width;
-      b.bond_id = s.bond_id;
-      b.orig = I32(ctx->wOrig[set]);
-      b.P4 = F4(ctx->wP[cur]);
-      b.skeys = sk;  // compact sorted keys: slot b's key is sk[cidx[b]]
-      b.ccref = sg->ccref;
-      b.cidx = I32(ctx->wSrc);
-      b.starts = I32(ctx->cstart);
-      b.grid = g;
-      b.dom = dom;
-      b.seg = sg->seg;
-      b.segp = sg->segp;
-      b.seg_mode = sg->seg_mode;
-      b.nl = I32(ctx->wNl[nlc]);
-      b.overflow = (int32_t*)ctx->flags.p + 2;
-      b.gate = gate;
-      b.wpref = sg->wpref;
-      b.offsets = sg->offsets;
-      b.n_seg = sg->n_seg;
-      if (hist) {
-        b.W64 = W64;
-        b.inv = I32(ctx->wInv);
-        b.ostride = N;
-        b.old_nl = r.tnl;
-        b.old_xi = r.txi;
-        b.old_live = r.tlive;
-        b.xi = F4(ctx->wXiRank);
-        b.live = U64(ctx->wLive[nlc]);
-      }
-      HIPCHK(ctx, ws_launch_nlist(b, D, false, st));
-    }
-    if (hist && M > 0)
-      HIPCHK(ctx, ws_launch_pack_springs(N, M, W64, F4(ctx->wXiRank), U64(ctx->wLive[nlc]), F4(ctx->wXi[xc]),
-                                         F4(ctx->wW[cur]), sg->seg, sg->seg_mode, st, gate, sg->wpref, sg->offsets,
-                                         sg->n_seg));
-    HIPCHK(ctx, ws_launch_gate_end(gate, st));
+    HIPCHK(ctx, ws_launch_rebuild_plan(r, plan, st));
+    HIPCHK(ctx, ws_launch_rebuild_keys(r, st));
+    HIPCHK(ctx, cell_sort_dev(csort, r.keys_c, N, std::max<int64_t>(sg->total_cells, 1), r.cpref + r.n_seg,
+                              r.ccref + r.n_seg, r.starts, st, r.go));
+    HIPCHK(ctx, ws_launch_rebuild_gather(r, st));
+    HIPCHK(ctx, ws_launch_rebuild_rows(r, st));
     span_end(ctx, sp);
     return JDEM_OK;
   };
@@ -1360,6 +1325,7 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
       if (rc) return rc;
     }
   }
+  if (sg) ctx->cscnt_clear = true;  // every chain that counted has scanned
   if (rebuilt_here) L.overflow = ctx->host_flags[2] != 0;
   S->overflow = L.overflow;
   // --- exit: back to the caller's order and layouts ---
@@ -1377,7 +1343,7 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
     HIPCHK(ctx, ws_launch_out(io, false, st));
     if (hist && M > 0)
       HIPCHK(ctx, ws_launch_unpack_springs(N, M, W64, F4(ctx->wXi[xc]), U64(ctx->wLive[nlc]), F4(ctx->wW[cur]),
-                                           F4(ctx->wXiRank), nullptr, nullptr, st));
+                                           F4(ctx->wXiRank), st));
     jdem_resident* res = new (std::nothrow) jdem_resident();
     if (!res) return fail(ctx, JDEM_ENOMEM, "resident working set");
     res->ctx = ctx;
@@ -1427,7 +1393,7 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
   io.xi = F4(ctx->wXiRank);
   if (hist && M > 0)
     HIPCHK(ctx, ws_launch_unpack_springs(N, M, W64, F4(ctx->wXi[xc]), U64(ctx->wLive[nlc]), F4(ctx->wW[cur]),
-                                         F4(ctx->wXiRank), nullptr, nullptr, st));
+                                         F4(ctx->wXiRank), st));
   HIPCHK(ctx, ws_launch_out(io, M > 0, st));
   if (free_done) {
     for (int a = 0; a < D; ++a) {

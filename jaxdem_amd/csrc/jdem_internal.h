@@ -62,7 +62,6 @@ struct jdem_ctx {
   // scratch, grown on demand and reused across calls
   jdem::Buf pos2, vel2, ang2;          // ping-pong kinematics
   jdem::Buf keys[2], vals[2], hist;    // radix sort
-  jdem::Buf ccur;                      // batch counting sort: per-cell cursors
   jdem::Buf cscnt;                     // counting sort: per-cell counts, left clear by every finished sort
   bool cscnt_clear = false;
   jdem::Buf cstart, cend, spos;        // cell tables, sorted (x, r)
@@ -95,7 +94,6 @@ struct jdem_ctx {
   jdem::Buf route;
   std::vector<char> route_host;
   // per-cell counts / starts of the batch rebuild's counting sort
-  jdem::Buf ccnt;
   // clumps: members per clump (CSR), lab positions, levers, member totals
   jdem::Buf cl_start, cl_members, plab, ppr, ftot, ttot, crefl;
   // the precision form's Verlet list
@@ -312,15 +310,14 @@ hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys
                          hipStream_t s);
 hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
                            int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
-// The counting sort with both counts on the device: the first *n_dev of
-// the keys (n bounds it), every key below *c_dev (n_cells bounds it).  The
-// launches are sized by the bounds and capped (kCappedGrid workgroups that
-// walk the work in turn), so a rebuild of a few systems of a large batch
-// costs what its particles and cells need.  Results as cell_sort_pairs; the
-// cell starts (compact, *c_dev + 1 entries) go to the context's scratch.
-hipError_t cell_sort_dev(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, const int64_t* n_dev,
-                         const int64_t* c_dev, uint32_t** keys_out, int32_t** vals_out, hipStream_t s,
-                         const int32_t* gate);
+// The counting sort of a batch rebuild, between cell_sort_begin and the
+// caller's rank pass: the first *n_dev of the keys (n bounds it), every key
+// below *c_dev (n_cells bounds it), starts of *c_dev + 1 entries, (key, id) at
+// their cells in cs.pairs.  The launches are sized by the bounds and capped
+// (kCappedGrid workgroups that walk the work in turn), so a rebuild of a few
+// systems of a large batch costs what its particles and cells need.
+hipError_t cell_sort_dev(const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells, const int64_t* n_dev,
+                         const int64_t* c_dev, int32_t* starts, hipStream_t s, const int32_t* gate);
 // cend[c] = starts[c + 1] for c < n_cells
 hipError_t launch_starts_to_ends(const int32_t* starts, int64_t n_cells, int32_t* cend, hipStream_t s);
 // key bits of a grid of n_cells cells (at least 1)
@@ -467,73 +464,67 @@ struct NLW {
   const int32_t* inv;       // old work slot -> new work slot
   const int32_t* old_nl;
   const float4* old_xi;
-  // old springs per wavefront (the step kernel's layout), their offsets in
-  // old_W[.].w; null: old_xi is by rank
+  // old and new springs are kept per wavefront (the step kernel's layout), the
+  // start of a slot's in old_W[.].w and new_W[.].w
   const float4* old_W;
-  // new springs per wavefront with their offsets written to new_W[.].w
-  // (one wave-wide scan of the new counts); null: xi is by rank
   float4* new_W;
   const uint64_t* old_live;
   float4* xi;
   uint64_t* live;
-  // segmented batch: system of each work slot, the systems' parameters and
-  // what this rebuild does to each system's rows (SEG_KEEP / SEG_FRESH /
-  // SEG_REMAP)
-  const int32_t* seg;
-  const SegP* segp;
-  const int32_t* seg_mode;
-  // batches rebuild in place: the old rows, springs and live words of the
-  // particle now at b are at compact index cidx[b] (stride ostride)
-  const int32_t* cidx;
-  int64_t ostride;
-  const int64_t* ccref;  // compact key of system s's first cell
-  const int32_t* gate;   // when set, the kernel returns at once while *gate == 0
-  // with wpref (flagged systems' wavefront prefix), the launch walks only the
-  // wavefronts that hold a flagged system's slots
-  const int64_t* wpref;
-  const int64_t* offsets;
-  int n_seg;
 };
 enum { SEG_KEEP = 0, SEG_FRESH = 1, SEG_REMAP = 2 };
 
 // In-place rebuild of the flagged systems of a batch (jdem_resident.hip).
+// Flagged particles have a compact index (system s: [cpref[s], cpref[s + 1]),
+// in original order before the sort and in the new slots' order after it),
+// their cells a compact key from ccref[s]; wpref counts the wavefronts of
+// slots that hold a flagged system.
 struct RB {
-  int64_t n, fn;  // particles; flagged particles (-1: read on the device, cpref[n_seg])
+  int64_t n;
   int n_seg;
   int dim;
-  const int32_t* gate;  // when set, every kernel returns at once while *gate == 0
+  const int32_t* go;  // every kernel but the first returns at once while *go == 0
   int M, W64;
-  const int32_t* seg;
+  const int32_t* seg;  // system of each work slot
   const SegP* segp;
-  const int32_t* seg_mode;
   const int64_t* offsets;
-  const int64_t* cpref;
-  const int64_t* ccref;
+  // the plan of this rebuild
+  int32_t *seg_mode;  // SEG_KEEP / SEG_FRESH / SEG_REMAP of each system
+  int64_t *cpref, *ccref, *wpref;
   // work set (updated in place)
   float4 *P, *V, *W, *Q, *I, *old4;
   int32_t* orig;
-  const int32_t* nl;
-  const uint64_t* live;
-  const float4* xi;
-  // compact sort input / output
+  int32_t* nl;
+  uint64_t* live;  // null: no history
+  float4* xi;      // per wavefront
+  float4* keep_xi; // by rank, of the kept systems' slots in a rebuilt wavefront
+  // counting sort
   uint32_t* keys_c;
-  int32_t* slot_c;
-  const int32_t* perm;
-  // staging, compact index
+  int32_t* slot_c;  // slot of compact index i before the sort
+  int32_t *cnt, *arr;
+  const uint2* pairs;
+  int32_t* starts;
+  // staging, compact index of the new slot
+  uint32_t* sk;
   float4 *tP, *tV, *tW, *tQ, *tI;
   int32_t* torig;
-  int32_t* cs;
+  int32_t* tlive;  // live springs, each with its partner's old slot, by rank (stride n)
   int32_t* tnl;
-  uint64_t* tlive;
   float4* txi;
-  // maps
-  int32_t* inv;
-  int32_t* cidx;
+  int32_t* inv;  // old slot -> new slot
+  int isb;
+  int bond_w;
+  const int32_t* bond_id;
+  int32_t* overflow;
 };
-hipError_t ws_launch_seg_prefix(int n_seg, const int32_t* seg_mode, const int64_t* offsets, const SegP* segp,
-                               int64_t* cpref, int64_t* ccref, int64_t* wpref, hipStream_t s);
-hipError_t ws_launch_hash_flagged(const RB& r, int dim, hipStream_t s);
-hipError_t ws_launch_place(const RB& r, const uint32_t* sk, int32_t* starts, hipStream_t s);
+// what the first kernel of the chain works on
+struct RBPlan {
+  int32_t *gate, *go, *overflow, *events, *seg_flag, *n_build;
+};
+hipError_t ws_launch_rebuild_plan(const RB& r, const RBPlan& p, hipStream_t s);
+hipError_t ws_launch_rebuild_keys(const RB& r, hipStream_t s);
+hipError_t ws_launch_rebuild_gather(const RB& r, hipStream_t s);
+hipError_t ws_launch_rebuild_rows(const RB& r, hipStream_t s);
 
 // Workgroups are dispatched round-robin over the 8 XCDs of the chip, each
 // with its own L2: workgroup w runs on XCD w % 8.  xcd_tile maps them so
@@ -649,13 +640,9 @@ hipError_t ws_launch_copy_rows(const int32_t* src, int32_t* dst, int64_t n, int 
 // wpref (the flagged systems' wavefront prefix of k_seg_prefix) the launch
 // walks those wavefronts only.
 hipError_t ws_launch_pack_springs(int64_t n, int M, int W64, const float4* rank, const uint64_t* live, float4* wave,
-                                  float4* W, const int32_t* seg, const int32_t* seg_mode, hipStream_t s,
-                                  const int32_t* gate = nullptr, const int64_t* wpref = nullptr,
-                                  const int64_t* offsets = nullptr, int n_seg = 0);
+                                  float4* W, hipStream_t s);
 hipError_t ws_launch_unpack_springs(int64_t n, int M, int W64, const float4* wave, const uint64_t* live,
-                                    const float4* W, float4* rank, const int32_t* seg, const int32_t* seg_mode,
-                                    hipStream_t s, const int32_t* gate = nullptr, const int64_t* wpref = nullptr,
-                                    const int64_t* offsets = nullptr, int n_seg = 0);
+                                    const float4* W, float4* rank, hipStream_t s);
 hipError_t ws_launch_inverse(const int32_t* orig, int64_t n, int32_t* wpos, hipStream_t s);
 hipError_t ws_launch_iota(int32_t* p, int64_t n, hipStream_t s);
 hipError_t ws_launch_copy4(float4* d, const float4* src, int64_t n, hipStream_t s);
@@ -670,13 +657,9 @@ hipError_t ws_launch_permute(int64_t n, const int32_t* new_orig, const int32_t* 
 // batch rebuilds: per-system mode from the flags (and bump the build counts),
 // and the flags of never-built systems
 // With gate set, *events counts the calls that find *gate != 0 (rebuilds).
-hipError_t ws_launch_seg_modes(int n_seg, int32_t* seg_flag, int32_t* n_build, int32_t* seg_mode, hipStream_t s,
-                               const int32_t* gate = nullptr, int32_t* events = nullptr);
 hipError_t ws_launch_seg_init_flags(int n_seg, const int32_t* n_build, int32_t* seg_flag, hipStream_t s,
                                    int32_t* gate = nullptr);
 // *gate = 0 (the end of a gated rebuild); *word = 0 when *gate is set
-hipError_t ws_launch_gate_end(int32_t* gate, hipStream_t s);
-hipError_t ws_launch_gated_zero(const int32_t* gate, int32_t* word, hipStream_t s);
 
 hipError_t ws_launch_cell_starts(const uint32_t* skeys, int64_t n, int64_t n_cells, int32_t* starts, hipStream_t s);
 hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s);

@@ -324,20 +324,6 @@ __global__ void __launch_bounds__(kBlock) k_permute(int64_t n, const int32_t* __
   inv_out[s] = (int32_t)b;
 }
 
-// Batch rebuilds.  mode of system s: KEEP when it did not ask for a
-// rebuild, FRESH for its first build, REMAP otherwise; its build count grows
-// and its flag is cleared.
-__global__ void k_seg_modes(int n_seg, int32_t* __restrict__ seg_flag, int32_t* __restrict__ n_build,
-                            int32_t* __restrict__ seg_mode, const int32_t* __restrict__ gate,
-                            int32_t* __restrict__ events) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s == 0 && events && gate && *gate) *events += 1;
-  if (s >= n_seg) return;
-  const int f = seg_flag[s] != 0;
-  seg_mode[s] = f ? (n_build[s] > 0 ? SEG_REMAP : SEG_FRESH) : SEG_KEEP;
-  n_build[s] += f;
-  seg_flag[s] = 0;
-}
 // Call start, before the first step kernel: a system without a list asks
 // for a build (and raises *gate when set), every other flag starts clear.
 __global__ void k_seg_init_flags(int n_seg, const int32_t* __restrict__ n_build, int32_t* __restrict__ seg_flag,
@@ -355,32 +341,51 @@ __global__ void k_seg_init_flags(int n_seg, const int32_t* __restrict__ n_build,
 // particles are numbered compactly: system s's particles take the compact
 // range [cpref[s], cpref[s + 1]) in original order, its cells the compact
 // key range starting at ccref[s].
+//
+// The chain runs after every step and mostly finds nothing to do, so what it
+// costs is its launches: plan, keys, scan totals, scan, placement, gather and
+// rows, seven where every pass had a kernel of its own (eighteen: 55 us of a
+// step of 256 systems of disks, 31 us now).
 
-// Exclusive prefix sums over the systems of the flagged particle and cell
-// counts (one block).
 // Wavefronts (64 work slots) that hold particles of system s.
 JD int64_t seg_waves(const int64_t* __restrict__ offsets, int s) {
   const int64_t a = offsets[s], e = offsets[s + 1];
   return e > a ? ((e - 1) >> 6) - (a >> 6) + 1 : 0;
 }
 
-// Exclusive prefix sums over the systems of the flagged particle, cell and
-// wavefront counts (one block).
-__global__ void __launch_bounds__(1024) k_seg_prefix(int n_seg, const int32_t* __restrict__ seg_mode,
-                                                      const int64_t* __restrict__ offsets,
-                                                      const SegP* __restrict__ segp, int64_t* __restrict__ cpref,
-                                                      int64_t* __restrict__ ccref, int64_t* __restrict__ wpref) {
-  __shared__ int64_t sp[1024], sc[1024], sw[1024];
+// The plan (one block): the gate word moves to go, which the other kernels of
+// the chain read, so the next step kernel finds it clear.  If it is set: the
+// mode of each system (KEEP when it did not ask for a rebuild, FRESH for its
+// first build, REMAP otherwise; its build count grows and its flag is cleared)
+// and the exclusive prefix sums over the systems of the flagged particle, cell
+// and wavefront counts.
+__global__ void __launch_bounds__(1024) k_rebuild_plan(RB r, RBPlan q) {
+  const bool go = *q.gate != 0;
+  __syncthreads();  // every thread has read the gate
   const int t = threadIdx.x;
-  const int per = (n_seg + 1023) / 1024;
-  const int s0 = t * per, s1 = min(n_seg, s0 + per);
-  int64_t np = 0, nc = 0, nw = 0;
-  for (int s = s0; s < s1; ++s)
-    if (seg_mode[s] != SEG_KEEP) {
-      np += offsets[s + 1] - offsets[s];
-      nc += segp[s].grid.n_cells;
-      nw += seg_waves(offsets, s);
+  if (t == 0) {
+    *q.go = go ? 1 : 0;
+    if (go) {
+      *q.gate = 0;
+      *q.overflow = 0;
+      *q.events += 1;
     }
+  }
+  if (!go) return;
+  __shared__ int64_t sp[1024], sc[1024], sw[1024];
+  const int per = (r.n_seg + 1023) / 1024;
+  const int s0 = t * per, s1 = min(r.n_seg, s0 + per);
+  int64_t np = 0, nc = 0, nw = 0;
+  for (int s = s0; s < s1; ++s) {
+    const int f = q.seg_flag[s] != 0;
+    r.seg_mode[s] = f ? (q.n_build[s] > 0 ? SEG_REMAP : SEG_FRESH) : SEG_KEEP;
+    if (!f) continue;
+    q.n_build[s] += 1;
+    q.seg_flag[s] = 0;
+    np += r.offsets[s + 1] - r.offsets[s];
+    nc += r.segp[s].grid.n_cells;
+    nw += seg_waves(r.offsets, s);
+  }
   sp[t] = np;
   sc[t] = nc;
   sw[t] = nw;
@@ -395,19 +400,19 @@ __global__ void __launch_bounds__(1024) k_seg_prefix(int n_seg, const int32_t* _
   }
   int64_t p = sp[t] - np, c = sc[t] - nc, w = sw[t] - nw;
   for (int s = s0; s < s1; ++s) {
-    cpref[s] = p;
-    ccref[s] = c;
-    wpref[s] = w;
-    if (seg_mode[s] != SEG_KEEP) {
-      p += offsets[s + 1] - offsets[s];
-      c += segp[s].grid.n_cells;
-      w += seg_waves(offsets, s);
+    r.cpref[s] = p;
+    r.ccref[s] = c;
+    r.wpref[s] = w;
+    if (r.seg_mode[s] != SEG_KEEP) {
+      p += r.offsets[s + 1] - r.offsets[s];
+      c += r.segp[s].grid.n_cells;
+      w += seg_waves(r.offsets, s);
     }
   }
   if (t == 1023) {
-    cpref[n_seg] = sp[t];
-    ccref[n_seg] = sc[t];
-    wpref[n_seg] = sw[t];
+    r.cpref[r.n_seg] = sp[t];
+    r.ccref[r.n_seg] = sc[t];
+    r.wpref[r.n_seg] = sw[t];
   }
 }
 
@@ -427,109 +432,81 @@ JD int seg_of_compact(const int64_t* __restrict__ pref, int n_seg, int64_t k) {
   return lo;
 }
 
-// compact key of every particle of a flagged system, at its compact index
+// The compact key of every particle of a flagged system, at its compact
+// index, counted; and the springs of the kept systems' slots in the first and
+// last wavefront of a flagged system, whose springs are placed anew.
 template <int D>
-__global__ void __launch_bounds__(kBlock) k_hash_flagged(RB r) {
-  if (r.gate && *r.gate == 0) return;
+__global__ void __launch_bounds__(kBlock) k_rebuild_keys(RB r) {
+  if (*r.go == 0) return;
+  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t fn = r.cpref[r.n_seg];
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < fn; k += (int64_t)gridDim.x * blockDim.x) {
-  const int s = seg_of_compact(r.cpref, r.n_seg, k);
-  const int64_t b = r.offsets[s] + (k - r.cpref[s]);
-  const SegP& sp = r.segp[s];
-  const float4 p = r.P[b];
-  const float x[3] = {p.x, p.y, p.z};
-  int c[3] = {0, 0, 0};
-  const bool per = sp.dom.kind == JDEM_DOMAIN_PERIODIC;
+  for (int64_t k = t0; k < fn; k += stride) {
+    const int s = seg_of_compact(r.cpref, r.n_seg, k);
+    const int64_t b = r.offsets[s] + (k - r.cpref[s]);
+    const SegP& sp = r.segp[s];
+    const float4 p = r.P[b];
+    const float x[3] = {p.x, p.y, p.z};
+    int c[3] = {0, 0, 0};
+    const bool per = sp.dom.kind == JDEM_DOMAIN_PERIODIC;
 #pragma unroll
-  for (int a = 0; a < D; ++a) c[a] = per ? ccoord<true>(x[a], a, sp.dom, sp.grid) : ccoord<false>(x[a], a, sp.dom, sp.grid);
-  const int64_t i = r.cpref[s] + (r.orig[b] - r.offsets[s]);
-  r.keys_c[i] = (uint32_t)(r.ccref[s] + wkey<D>(c, sp.grid));
-  r.slot_c[i] = (int32_t)b;
+    for (int a = 0; a < D; ++a)
+      c[a] = per ? ccoord<true>(x[a], a, sp.dom, sp.grid) : ccoord<false>(x[a], a, sp.dom, sp.grid);
+    const int64_t i = r.cpref[s] + (r.orig[b] - r.offsets[s]);
+    const uint32_t key = (uint32_t)(r.ccref[s] + wkey<D>(c, sp.grid));
+    r.keys_c[i] = key;
+    r.slot_c[i] = (int32_t)b;
+    r.arr[i] = atomicAdd(&r.cnt[key], 1);
+  }
+  if (!r.live) return;
+  for (int64_t t = t0; t < (int64_t)r.n_seg * 128; t += stride) {
+    const int s = (int)(t >> 7);
+    const int64_t a = r.offsets[s], e = r.offsets[s + 1];
+    if (r.seg_mode[s] == SEG_KEEP || e <= a) continue;
+    const int64_t b = (((t & 64) ? e - 1 : a) & ~(int64_t)63) + (t & 63);
+    if (b >= r.n || r.seg_mode[r.seg[b]] != SEG_KEEP) continue;
+    int cnt = 0;
+    for (int w = 0; w < r.W64; ++w) cnt += __popcll(r.live[(int64_t)w * r.n + b]);
+    const float4* src = r.xi + (b & ~(int64_t)63) * r.M + __float_as_int(r.W[b].w);
+    for (int k = 0; k < cnt; ++k) r.keep_xi[(int64_t)k * r.n + b] = src[k];
   }
 }
 
-// sorted position k -> staging (k) of the particle's fields and old list
-// Flagged particles of the rebuild: r.fn, or (r.fn < 0) the device count.
-JD int64_t rb_fn(const RB& r) { return r.fn >= 0 ? r.fn : r.cpref[r.n_seg]; }
-
-// The staging arrays hold the compact index k at stride n (rows, live words
-// and springs of k at c * n + k).
-__global__ void __launch_bounds__(kBlock) k_place_gather(RB r) {
-  if (r.gate && *r.gate == 0) return;
-  const int64_t fn = rb_fn(r);
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < fn; k += (int64_t)gridDim.x * blockDim.x) {
-  const int32_t ob = r.slot_c[r.perm[k]];
-  const int s = r.seg[ob];
-  const int64_t nb = r.offsets[s] + (k - r.cpref[s]);
-  r.tP[k] = r.P[ob];
-  r.tV[k] = r.V[ob];
-  r.tW[k] = r.W[ob];
-  r.tQ[k] = r.Q[ob];
-  r.tI[k] = r.I[ob];
-  r.torig[k] = r.orig[ob];
-  r.cs[k] = s;
-  r.inv[ob] = (int32_t)nb;
-  if (r.M > 0) {
-    int c = 0;
-    for (; c < r.M; ++c) {
-      const int32_t j = r.nl[(int64_t)c * r.n + ob];
-      r.tnl[(int64_t)c * r.n + k] = j;
-      if (j < 0) break;
-    }
-    if (r.live) {
-      int nlive = 0;
-      for (int w = 0; w < r.W64; ++w) {
-        const uint64_t bits = r.live[(int64_t)w * r.n + ob];
-        r.tlive[(int64_t)w * r.n + k] = bits;
-        nlive += __popcll(bits);
+// The rank pass of the sort, then the fields of the particle that goes to
+// compact index k, and its live springs with their partners' old slots.
+__global__ void __launch_bounds__(kBlock) k_rebuild_gather(RB r) {
+  if (*r.go == 0) return;
+  const int64_t fn = r.cpref[r.n_seg];
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < fn; j += (int64_t)gridDim.x * blockDim.x) {
+    const uint2 me = r.pairs[j];
+    const int32_t cs = r.starts[me.x], ce = r.starts[me.x + 1];
+    int32_t k = cs;
+    for (int32_t m = cs; m < ce; ++m) k += r.pairs[m].y < me.y ? 1 : 0;
+    const int32_t ob = r.slot_c[me.y];
+    const int s = r.seg[ob];
+    r.sk[k] = me.x;
+    r.tP[k] = r.P[ob];
+    r.tV[k] = r.V[ob];
+    r.tW[k] = r.W[ob];
+    r.tQ[k] = r.Q[ob];
+    r.tI[k] = r.I[ob];
+    r.torig[k] = r.orig[ob];
+    r.inv[ob] = (int32_t)(r.offsets[s] + (k - r.cpref[s]));
+    if (!r.live) continue;
+    int q = 0;
+    if (r.seg_mode[s] == SEG_REMAP) {
+      const float4* src = r.xi + ((int64_t)ob & ~(int64_t)63) * r.M + __float_as_int(r.W[ob].w);
+      for (int c = 0; c < r.W64; ++c) {
+        uint64_t bits = r.live[(int64_t)c * r.n + ob];
+        while (bits) {
+          const int sl = c * 64 + __ffsll((unsigned long long)bits) - 1;
+          bits &= bits - 1ull;
+          r.tnl[(int64_t)q * r.n + k] = r.nl[(int64_t)sl * r.n + ob];
+          r.txi[(int64_t)q * r.n + k] = src[q];
+          ++q;
+        }
       }
-      for (int q = 0; q < nlive; ++q) r.txi[(int64_t)q * r.n + k] = r.xi[(int64_t)q * r.n + ob];
     }
-  }
-  }
-}
-
-// staging (k) -> the particle's new work slot in its system's range
-__global__ void __launch_bounds__(kBlock) k_place_scatter(RB r) {
-  if (r.gate && *r.gate == 0) return;
-  const int64_t fn = rb_fn(r);
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < fn; k += (int64_t)gridDim.x * blockDim.x) {
-  const int s = r.cs[k];
-  const int64_t nb = r.offsets[s] + (k - r.cpref[s]);
-  float4 p = r.tP[k];
-  float4 v = r.tV[k];
-  r.old4[nb] = p;  // build position
-  if (r.dim == 2) {  // and in the 2D records' free lanes
-    p.z = p.x;
-    v.z = p.y;
-  }
-  r.P[nb] = p;
-  r.V[nb] = v;
-  r.W[nb] = r.tW[k];
-  r.Q[nb] = r.tQ[k];
-  r.I[nb] = r.tI[k];
-  r.orig[nb] = r.torig[k];
-  r.cidx[nb] = (int32_t)k;
-  }
-}
-
-// cell starts of the flagged systems: thread k fills the cells of its system
-// from the one after its predecessor's key to its own key (the last particle
-// of a system also fills to the end of the system's grid)
-__global__ void __launch_bounds__(kBlock) k_cell_starts_flagged(RB r, const uint32_t* __restrict__ sk,
-                                                                 int32_t* __restrict__ starts) {
-  if (r.gate && *r.gate == 0) return;
-  const int64_t fn = rb_fn(r);
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < fn; k += (int64_t)gridDim.x * blockDim.x) {
-  const int s = r.cs[k];
-  const SegP& sp = r.segp[s];
-  const int64_t first = r.cpref[s], last = r.cpref[s + 1] - 1;
-  const int64_t key = (int64_t)sk[k] - r.ccref[s];
-  const int64_t lo = (k == first) ? 0 : (int64_t)sk[k - 1] - r.ccref[s] + 1;
-  const int32_t slot = (int32_t)(r.offsets[s] + (k - first));
-  for (int64_t h = lo; h <= key; ++h) starts[sp.cell_base + h] = slot;
-  if (k == last)
-    for (int64_t h = key + 1; h <= sp.grid.n_cells; ++h) starts[sp.cell_base + h] = (int32_t)r.offsets[s + 1];
+    r.tlive[k] = q;
   }
 }
 
@@ -584,7 +561,7 @@ JD int wave_exclusive_scan(int v, int lane) {
   return incl - v;
 }
 
-// With new_W set, every lane of the wave must call it (inactive lanes with
+// Every lane of the wave must call it (inactive lanes with
 // active = false): the new springs are placed per wavefront after a
 // wave-wide scan of the new counts.
 template <class Row>
@@ -593,23 +570,22 @@ JD void remap_row(const NLW& a, int64_t b, bool active, int nrow, Row row, bool 
   const int64_t n = a.n;
   uint64_t out0 = 0ull, out1 = 0ull, out2 = 0ull, out3 = 0ull;
   // the old row of the particle now at b: at slot src[b] of the previous
-  // buffers, or (batches) at compact index cidx[b] of the staged rows
+  // buffers
   const bool go = active && remap;
-  const int64_t ob = go ? (a.cidx ? (int64_t)a.cidx[b] : (int64_t)a.src[b]) : 0;
-  const int64_t os = a.cidx ? a.ostride : n;
+  const int64_t ob = go ? (int64_t)a.src[b] : 0;
   // start of the old springs, read before any lane writes new offsets (old_W
   // and new_W are one buffer when the rebuild does not re-sort)
-  const int64_t obase = (go && a.old_W) ? (ob & ~(int64_t)63) * a.M + __float_as_int(a.old_W[ob].w) : 0;
+  const int64_t obase = go ? (ob & ~(int64_t)63) * a.M + __float_as_int(a.old_W[ob].w) : 0;
   // visit(t, o_slot_new): each live old slot t whose partner is listed
   // again, with the rank of t among the live old slots
   auto sweep = [&](auto&& f) {
     int rank_old = 0;
     for (int w = 0; w < a.W64; ++w) {
-      uint64_t bits = a.old_live[(int64_t)w * os + ob];
+      uint64_t bits = a.old_live[(int64_t)w * n + ob];
       while (bits) {
         const int t = w * 64 + (__ffsll((unsigned long long)bits) - 1);
         bits &= bits - 1ull;
-        const int32_t o = a.old_nl[(int64_t)t * os + ob];
+        const int32_t o = a.old_nl[(int64_t)t * n + ob];
         const int s = o < 0 ? -1 : find_in_row(a.inv[o], nrow, row);
         if (s >= 0) f(s, rank_old);
         ++rank_old;
@@ -625,18 +601,14 @@ JD void remap_row(const NLW& a, int64_t b, bool active, int nrow, Row row, bool 
       out2 |= ws == 2 ? bit : 0ull;
       out3 |= ws == 3 ? bit : 0ull;
     });
-  int64_t wbase = 0;
-  if (a.new_W) {
-    const int cnt = __popcll(out0) + __popcll(out1) + __popcll(out2) + __popcll(out3);
-    const int off = wave_exclusive_scan(cnt, (int)(threadIdx.x & 63));
-    if (active) a.new_W[b].w = __int_as_float(off);
-    wbase = (b & ~(int64_t)63) * a.M + off;
-  }
+  const int cnt = __popcll(out0) + __popcll(out1) + __popcll(out2) + __popcll(out3);
+  const int off = wave_exclusive_scan(cnt, (int)(threadIdx.x & 63));
+  if (active) a.new_W[b].w = __int_as_float(off);
+  const int64_t wbase = (b & ~(int64_t)63) * a.M + off;
   if (go)
     sweep([&](int s, int rank_old) {
       const int rank_new = rank_below(out0, out1, out2, out3, s);
-      const int64_t oi = a.old_W ? obase + rank_old : (int64_t)rank_old * os + ob;
-      a.xi[a.new_W ? wbase + rank_new : (int64_t)rank_new * n + b] = a.old_xi[oi];
+      a.xi[wbase + rank_new] = a.old_xi[obase + rank_old];
     });
   if (!active) return;
   a.live[b] = out0;
@@ -660,63 +632,19 @@ JD void end_row(const NLW& a, int64_t b, bool active, int count) {
 // slot are contiguous; later slots go straight to memory.
 constexpr int kRowLds = 16;
 
-// PM: 0 = one non-periodic system, 1 = one periodic system, 2 = a segmented
-// batch, where each work slot takes the grid, domain and cutoff of its system.
-template <int D, int PM>
+template <int D, bool PER>
 __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
-  if (a.gate && *a.gate == 0) return;  // uniform over the grid
   __shared__ int32_t rows[kRowLds][kBlock];
   __shared__ int row_max;
   const int tid = threadIdx.x;
-  // one tile of kBlock slots per workgroup, or (a grid smaller than the
-  // tiles, as batches launch it) several in turn.  A batch with wpref walks
-  // the wavefronts of the flagged systems only: a tile is four of them.
-  const bool by_wave = PM == 2 && a.wpref;
-  const int64_t nwaves = by_wave ? a.wpref[a.n_seg] : 0;
-  const int64_t ntiles = by_wave ? (nwaves + kBlock / 64 - 1) / (kBlock / 64) : (a.n + kBlock - 1) / kBlock;
-  for (int64_t tile = xcd_tile(blockIdx.x, gridDim.x); tile < ntiles; tile += gridDim.x) {
-  int64_t b = tile * blockDim.x + tid;
-  if (by_wave) {
-    const int64_t cw = tile * (kBlock / 64) + (tid >> 6);
-    if (cw < nwaves) {
-      const int s = seg_of_compact(a.wpref, a.n_seg, cw);
-      b = ((a.offsets[s] >> 6) + (cw - a.wpref[s])) * 64 + (tid & 63);
-    } else {
-      b = a.n;
-    }
-  }
-  // a batch workgroup whose systems all keep their rows has nothing to do
-  if (PM == 2 && !__syncthreads_or(b < a.n && a.seg_mode[a.seg[b]] != SEG_KEEP)) continue;
+  const int64_t b = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * kBlock + tid;
   if (tid == 0) row_max = 0;
   __syncthreads();
-  bool remap = a.remap != 0;
-  if (PM == 2 && b < a.n) {
-    const int mode = a.seg_mode[a.seg[b]];
-    if (mode == SEG_KEEP) b = a.n;  // the system keeps its rows (the barrier below is still reached)
-    remap = mode == SEG_REMAP;
-  }
   const bool active = b < a.n;
   int count = 0;
   if (active) {
-    GridP grid;
-    DomP dom;
-    float cutoff_sq;
-    uint32_t cbase = 0, key;
-    if (PM == 2) {
-      const int sg = a.seg[b];
-      const SegP& sp = a.segp[sg];
-      grid = sp.grid;
-      dom = sp.dom;
-      cutoff_sq = sp.cutoff_sq;
-      cbase = sp.cell_base;
-      key = a.skeys[a.cidx[b]] - (uint32_t)a.ccref[sg];  // batches sort the flagged systems compactly
-    } else {
-      grid = a.grid;
-      dom = a.dom;
-      cutoff_sq = a.cutoff_sq;
-      key = a.skeys[b];
-    }
-    const bool PER = PM == 2 ? dom.kind == JDEM_DOMAIN_PERIODIC : PM == 1;
+    const GridP& grid = a.grid;
+    const uint32_t key = a.skeys[b];
     const Vec<D> xi = xyz<D>(a.P4[b]);
     const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
     int c0, c1, cf;
@@ -744,13 +672,13 @@ __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
       const int cx = stencil_cell(PER, c0, ox, d0);
       if (cx < 0) continue;
       for (int oy = lo1; oy <= hi1; ++oy) {
-        int64_t base = cbase;
+        int64_t base;
         if (D == 3) {
           const int cy = stencil_cell(PER, c1, oy, d1);
           if (cy < 0) continue;
-          base += (int64_t)(cx * d1 + cy) * d2;
+          base = (int64_t)(cx * d1 + cy) * d2;
         } else {
-          base += (int64_t)cx * d1;
+          base = (int64_t)cx * d1;
         }
         // both runs' bounds are loaded before either is walked
         const int k0 = starts[base + r0a], k0e = starts[base + r0b + 1];
@@ -769,9 +697,8 @@ __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
               const int k = kg + u;
               if (k >= ke) break;
               if (k == b) continue;
-              const float dsq =
-                  PER ? dist_sq<true>(xi, xyz<D>(pk[u]), dom) : dist_sq<false>(xi, xyz<D>(pk[u]), dom);
-              if (!(dsq <= cutoff_sq)) continue;
+              const float dsq = dist_sq<PER>(xi, xyz<D>(pk[u]), a.dom);
+              if (!(dsq <= a.cutoff_sq)) continue;
               if (chk_bond && bonded_o(a.bond_id, a.bond_w, ib, a.orig[k])) continue;
               if (count < kRowLds)
                 rows[count][tid] = k;
@@ -795,16 +722,14 @@ __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
     if (count > a.M) atomicOr(a.overflow, 1);
   }
   remap_row(a, b, active, c, [&](int s) { return s < kRowLds ? rows[s][tid] : a.nl[(int64_t)s * a.n + b]; },
-            remap);
-  __syncthreads();  // the next tile reuses rows and row_max
-  }
+            a.remap != 0);
 }
 
-// The list build of one system with a group of G lanes per particle:
-// k_nlist_work's chain of column bounds and candidates is serial per lane, and
-// below ~10^5 particles there are not enough wavefronts to hide it (154 us for
-// 37 k spheres of 31 neighbours, most of a rebuild; here 44 us).  A workgroup builds the rows
-// of one wavefront's 64 slots: each lane loads one stencil column's bounds, a
+// The list build with a group of G lanes per particle: k_nlist_work's chain of
+// column bounds and candidates is serial per lane, and below ~10^5 particles
+// there are not enough wavefronts to hide it (154 us for 37 k spheres of 31
+// neighbours, most of a rebuild; here 44 us).  A workgroup builds the rows of
+// one wavefront's 64 slots: each lane loads one stencil column's bounds, a
 // scan numbers the candidates, G of them are tested at a time and those within
 // the cutoff appended in candidate order; the old springs are looked up one
 // per lane; the new springs' places are a scan over the 64 slots.
@@ -829,182 +754,327 @@ JD int select_bit(const uint64_t* w, int n_words, int r) {
   return -1;
 }
 
-// MW: live words of a row (1, or 4 for rows of more than 64 slots).  Eight
-// waves per SIMD (64 VGPRs) let two 3D workgroups share a CU.
+struct RowLds {
+  int32_t rows[kRowGrp][64];
+  int row_cnt[64], new_cnt[64], new_off[64];
+};
+
+// The row of the particle at slot b, whose lanes p * G .. p * G + G - 1 of the
+// workgroup all call this: its own index among the candidates is self, a
+// candidate's slot is its index + shift.  Returns the neighbours found, which
+// may be more than the M slots kept.
+template <int D, bool PER>
+JD int group_row(RowLds& lds, const float4* __restrict__ P4, const int32_t* __restrict__ orig, int self, int shift,
+                 uint32_t key, const GridP& grid, const DomP& dom, float cutoff_sq,
+                 const int32_t* __restrict__ starts, const int32_t* __restrict__ bond_id, int bond_w, bool chk_bond,
+                 int32_t* __restrict__ nl, int64_t n, int M, int64_t b) {
+  constexpr int G = nlist_group<D>();
+  const int p = threadIdx.x / G, l = threadIdx.x & (G - 1), lane = threadIdx.x & 63;
+  const uint64_t below = (1ull << l) - 1ull;
+  const Vec<D> xi = xyz<D>(P4[self]);
+  const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
+  int c0, c1, cf;
+  if (D == 3) {
+    cf = (int)(key % (uint32_t)d2);
+    const uint32_t r = key / (uint32_t)d2;
+    c1 = (int)(r % (uint32_t)d1);
+    c0 = (int)(r / (uint32_t)d1);
+  } else {
+    cf = (int)(key % (uint32_t)d1);
+    c0 = (int)(key / (uint32_t)d1);
+    c1 = 0;
+  }
+  const int sr = grid.sr, dF = (D == 3) ? d2 : d1;
+  int r0a, r0b, r1a, r1b;
+  stencil_runs(PER, cf, sr, dF, r0a, r0b, r1a, r1b);
+  const int n1 = (D == 3) ? (PER ? min(sr, d1 - sr - 1) : sr) + sr + 1 : 1;
+  const int ncol = ((PER ? min(sr, d0 - sr - 1) : sr) + sr + 1) * n1;
+  const int64_t ib = chk_bond ? (int64_t)orig[self] : 0;
+  int count = 0;
+  for (int cb = 0; cb < ncol; cb += G) {
+    const int col = cb + l;
+    int s0 = 0, len0 = 0, s1 = 0, len1 = 0;
+    if (col < ncol) {
+      const int cx = stencil_cell(PER, c0, (D == 3 ? col / n1 : col) - sr, d0);
+      const int cy = (D == 3) ? stencil_cell(PER, c1, col % n1 - sr, d1) : 0;
+      if (cx >= 0 && cy >= 0) {
+        const int64_t base = (D == 3) ? ((int64_t)cx * d1 + cy) * d2 : (int64_t)cx * d1;
+        s0 = starts[base + r0a];
+        len0 = starts[base + r0b + 1] - s0;
+        if (r1b >= r1a) {
+          s1 = starts[base + r1a];
+          len1 = starts[base + r1b + 1] - s1;
+        }
+      }
+    }
+    int incl = len0 + len1;
+#pragma unroll
+    for (int d = 1; d < G; d <<= 1) {
+      const int t = __shfl_up(incl, d, G);
+      if (l >= d) incl += t;
+    }
+    const int pre = incl - (len0 + len1);
+    const int total = __shfl(incl, G - 1, G);
+    for (int c8 = 0; c8 < total; c8 += G) {
+      const int cand = c8 + l;
+      int q = 0;
+#pragma unroll
+      for (int st = G / 2; st > 0; st >>= 1) q += __shfl(pre, q + st, G) <= cand ? st : 0;
+      const int o = cand - __shfl(pre, q, G), f0 = __shfl(s0, q, G), n_0 = __shfl(len0, q, G),
+                f1 = __shfl(s1, q, G);
+      const int k = o < n_0 ? f0 + o : f1 + (o - n_0);
+      bool hit = false;
+      if (cand < total && k != self) {
+        const Vec<D> xk = xyz<D>(P4[k]);
+        const float dsq = dist_sq<PER>(xi, xk, dom);
+        hit = dsq <= cutoff_sq;
+        if (hit && chk_bond) hit = !bonded_o(bond_id, bond_w, ib, orig[k]);
+      }
+      const uint64_t m = (__ballot(hit) >> (lane & ~(G - 1))) & ((1ull << G) - 1ull);
+      if (hit) {
+        const int t = count + __popcll(m & below);
+        if (t < kRowGrp)
+          lds.rows[t][p] = k + shift;
+        else if (t < M)
+          nl[(int64_t)t * n + b] = k + shift;
+      }
+      count += __popcll(m);
+    }
+  }
+  return count;
+}
+
+// The collected slots of the region's rows, 64 consecutive particles at a time
+// (after a barrier; row_cnt is -1 where no row was built).
+template <int G>
+JD void write_rows(const RowLds& lds, int32_t* __restrict__ nl, int64_t n, int64_t region) {
+  const int lane = threadIdx.x & 63;
+  const int cw = lds.row_cnt[lane];
+  for (int s = threadIdx.x >> 6; s < kRowGrp; s += G) {
+    if (s < cw) nl[(int64_t)s * n + region + lane] = lds.rows[s][lane];
+    if (!__any(s + G < cw)) break;
+  }
+}
+
+// The history of the new row of c slots at b (as remap_row): the r-th of n_old
+// live old springs goes to the slot of the new row that lists its partner
+// (slot partner(r) now), if any.  place(lane, off) is called once for each
+// slot of the region with the start of its springs; spring(r) gives the r-th
+// old one; a slot whose row was not built (built = false) keeps kept springs.
+// Every thread of the workgroup calls this.
+template <int G, int MW, class Partner, class Spring, class Place, class Kept>
+JD void group_springs(RowLds& lds, bool built, int c, int n_old, int n_kept, const int32_t* __restrict__ nl,
+                      int64_t n, int M, int W64, int64_t region, float4* __restrict__ xi, uint64_t* __restrict__ live,
+                      Partner partner, Spring spring, Place place, Kept kept) {
+  const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1);
+  const int64_t b = region + p;
+  uint64_t out[MW];
+#pragma unroll
+  for (int w = 0; w < MW; ++w) out[w] = 0ull;
+  auto new_slot = [&](int r) {
+    const int32_t tgt = partner(r);
+    if (tgt < 0) return -1;
+    for (int s = 0; s < c; ++s)
+      if ((s < kRowGrp ? lds.rows[s][p] : nl[(int64_t)s * n + b]) == tgt) return s;
+    return -1;
+  };
+  const int first = l < n_old ? new_slot(l) : -1;  // kept: rows rarely carry more than G springs
+  for (int r = l; r < n_old; r += G) {
+    const int s = r == l ? first : new_slot(r);
+    if (s >= 0)
+#pragma unroll
+      for (int w = 0; w < MW; ++w) out[w] |= (s >> 6) == w ? 1ull << (s & 63) : 0ull;
+  }
+#pragma unroll
+  for (int w = 0; w < MW; ++w) {
+    if (w >= W64) break;  // uniform
+#pragma unroll 1
+    for (int d = 1; d < G; d <<= 1) out[w] |= (uint64_t)__shfl_xor((unsigned long long)out[w], d, G);
+  }
+  if (l == 0) {
+    int k = n_kept;
+#pragma unroll
+    for (int w = 0; w < MW; ++w) k += __popcll(out[w]);
+    lds.new_cnt[p] = k;
+  }
+  __syncthreads();  // the old offsets are read, the counts are there
+  if (tid < 64) {
+    const int off = wave_exclusive_scan(lds.new_cnt[tid], tid);
+    lds.new_off[tid] = off;
+    place(tid, off);
+  }
+  __syncthreads();
+  const int64_t wbase = region * M + lds.new_off[p];
+  for (int r = l; r < n_old; r += G) {
+    const int s = r == l ? first : new_slot(r);
+    if (s < 0) continue;
+    const int rank = MW == 1 ? __popcll(out[0] & ((1ull << s) - 1ull))
+                             : rank_below(out[0], out[MW > 1 ? 1 : 0], out[MW > 2 ? 2 : 0], out[MW > 3 ? 3 : 0], s);
+    xi[wbase + rank] = spring(r);
+  }
+  for (int r = l; r < n_kept; r += G) xi[wbase + r] = kept(r);
+  if (built && l == 0)
+#pragma unroll
+    for (int w = 0; w < MW; ++w)
+      if (w < W64) live[(int64_t)w * n + b] = out[w];
+}
+
+// One system.  MW: live words of a row (1, or 4 for rows of more than 64
+// slots).  Eight waves per SIMD (64 VGPRs) let two 3D workgroups share a CU.
 template <int D, bool PER, int MW>
 __global__ void __launch_bounds__(64 * nlist_group<D>()) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_nlist_group(NLW a) {
-  if (a.gate && *a.gate == 0) return;  // uniform over the grid
   constexpr int G = nlist_group<D>();
-  __shared__ int32_t rows[kRowGrp][64];
-  __shared__ int row_cnt[64], new_cnt[64], new_off[64];
-  const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1), lane = tid & 63;
-  const uint64_t below = (1ull << l) - 1ull;
+  __shared__ RowLds lds;
+  const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1);
   const int64_t n = a.n;
-  const int64_t nreg = (n + 63) / 64;
+  const int64_t region = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * 64, b = region + p;
+  const bool active = b < n;
+  int count = 0;
+  if (active)
+    count = group_row<D, PER>(lds, a.P4, a.orig, (int)b, 0, a.skeys[b], a.grid, a.dom, a.cutoff_sq, a.starts,
+                                      a.bond_id, a.bond_w, (!a.isb) && a.bond_w > 0, a.nl, n, a.M, b);
+  const int c = min(count, a.M);
+  if (l == 0) lds.row_cnt[p] = active ? c : -1;
+  __syncthreads();
+  write_rows<G>(lds, a.nl, n, region);
+  if (active && l == 0) {
+    if (count < a.M) a.nl[(int64_t)count * n + b] = -1;
+    if (count > a.M) atomicOr(a.overflow, 1);
+  }
+  if (!a.live) return;
+  const bool go = active && a.remap != 0;
+  const int64_t ob = go ? (int64_t)a.src[b] : 0;
+  const int64_t obase = go ? (ob & ~(int64_t)63) * a.M + __float_as_int(a.old_W[ob].w) : 0;
+  uint64_t old[MW];
+  int n_old = 0;
+#pragma unroll
+  for (int w = 0; w < MW; ++w) {
+    old[w] = go && w < a.W64 ? a.old_live[(int64_t)w * n + ob] : 0ull;
+    n_old += __popcll(old[w]);
+  }
+  group_springs<G, MW>(
+      lds, active, c, n_old, 0, a.nl, n, a.M, a.W64, region, a.xi, a.live,
+      [&](int r) {
+        const int32_t o = a.old_nl[(int64_t)select_bit(old, MW, r) * n + ob];
+        return o < 0 ? -1 : a.inv[o];
+      },
+      [&](int r) { return a.old_xi[obase + r]; },
+      [&](int lane, int off) {
+        if (region + lane < n) a.new_W[region + lane].w = __int_as_float(off);
+      },
+      [&](int) { return make_float4(0.f, 0.f, 0.f, 0.f); });
+}
+
+// The flagged systems of a batch, from the staged particles: rows, springs
+// and the particles' fields in their new slots, over the wavefronts that hold
+// a flagged system (one shared by two of them is written twice, alike).
+// With k_nlist_work's lane per particle in its place (119 us a rebuild of eight
+// systems of 1 k to 150 k polydisperse spheres, 58 us now) a rebuild of one
+// system left most of the chip idle; all 10^6 disks of 256 systems at once, the
+// first build, take longer with groups, 87 -> 236 us, which the passes saved in
+// every later step outweigh.
+template <int D, int MW>
+__global__ void __launch_bounds__(64 * nlist_group<D>()) __attribute__((amdgpu_waves_per_eu(8, 8)))
+k_rebuild_rows(RB r) {
+  if (*r.go == 0) return;
+  constexpr int G = nlist_group<D>();
+  __shared__ RowLds lds;
+  const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1), lane = tid & 63;
+  const int64_t n = r.n, nreg = r.wpref[r.n_seg];
   for (int64_t reg = xcd_tile(blockIdx.x, gridDim.x); reg < nreg; reg += gridDim.x) {
-    const int64_t b = reg * 64 + p;
-    const bool active = b < n;
+    const int fs = seg_of_compact(r.wpref, r.n_seg, reg);
+    const int64_t region = ((r.offsets[fs] >> 6) + (reg - r.wpref[fs])) * 64, b = region + p;
+    const int sg = b < n ? r.seg[b] : -1;
+    const int mode = b < n ? r.seg_mode[sg] : SEG_FRESH;
+    const bool active = b < n && mode != SEG_KEEP;
+    const int64_t k = active ? r.cpref[sg] + (b - r.offsets[sg]) : 0;  // compact index
     int count = 0;
-    if (active) {
-      const GridP& grid = a.grid;
-      const uint32_t key = a.skeys[b];
-      const Vec<D> xi = xyz<D>(a.P4[b]);
-      const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
-      int c0, c1, cf;
-      if (D == 3) {
-        cf = (int)(key % (uint32_t)d2);
-        const uint32_t r = key / (uint32_t)d2;
-        c1 = (int)(r % (uint32_t)d1);
-        c0 = (int)(r / (uint32_t)d1);
-      } else {
-        cf = (int)(key % (uint32_t)d1);
-        c0 = (int)(key / (uint32_t)d1);
-        c1 = 0;
-      }
-      const int sr = grid.sr, dF = (D == 3) ? d2 : d1;
-      int r0a, r0b, r1a, r1b;
-      stencil_runs(PER, cf, sr, dF, r0a, r0b, r1a, r1b);
-      const int n1 = (D == 3) ? (PER ? min(sr, d1 - sr - 1) : sr) + sr + 1 : 1;
-      const int ncol = ((PER ? min(sr, d0 - sr - 1) : sr) + sr + 1) * n1;
-      const bool chk_bond = (!a.isb) && a.bond_w > 0;
-      const int64_t ib = chk_bond ? (int64_t)a.orig[b] : 0;
-      const int32_t* __restrict__ starts = a.starts;
-      for (int cb = 0; cb < ncol; cb += G) {
-        const int col = cb + l;
-        int s0 = 0, len0 = 0, s1 = 0, len1 = 0;
-        if (col < ncol) {
-          const int cx = stencil_cell(PER, c0, (D == 3 ? col / n1 : col) - sr, d0);
-          const int cy = (D == 3) ? stencil_cell(PER, c1, col % n1 - sr, d1) : 0;
-          if (cx >= 0 && cy >= 0) {
-            const int64_t base = (D == 3) ? ((int64_t)cx * d1 + cy) * d2 : (int64_t)cx * d1;
-            s0 = starts[base + r0a];
-            len0 = starts[base + r0b + 1] - s0;
-            if (r1b >= r1a) {
-              s1 = starts[base + r1a];
-              len1 = starts[base + r1b + 1] - s1;
-            }
-          }
-        }
-        int incl = len0 + len1;
-#pragma unroll
-        for (int d = 1; d < G; d <<= 1) {
-          const int t = __shfl_up(incl, d, G);
-          if (l >= d) incl += t;
-        }
-        const int pre = incl - (len0 + len1);
-        const int total = __shfl(incl, G - 1, G);
-        for (int c8 = 0; c8 < total; c8 += G) {
-          const int cand = c8 + l;
-          int q = 0;
-#pragma unroll
-          for (int st = G / 2; st > 0; st >>= 1) q += __shfl(pre, q + st, G) <= cand ? st : 0;
-          const int o = cand - __shfl(pre, q, G), f0 = __shfl(s0, q, G), n_0 = __shfl(len0, q, G),
-                    f1 = __shfl(s1, q, G);
-          const int k = (o < n_0 ? f0 + o : f1 + (o - n_0));
-          bool hit = false;
-          if (cand < total && k != (int)b) {
-            const Vec<D> xk = xyz<D>(a.P4[k]);
-            const float dsq = dist_sq<PER>(xi, xk, a.dom);
-            hit = dsq <= a.cutoff_sq;
-            if (hit && chk_bond) hit = !bonded_o(a.bond_id, a.bond_w, ib, a.orig[k]);
-          }
-          const uint64_t m = (__ballot(hit) >> (lane & ~(G - 1))) & ((1ull << G) - 1ull);
-          if (hit) {
-            const int t = count + __popcll(m & below);
-            if (t < kRowGrp)
-              rows[t][p] = k;
-            else if (t < a.M)
-              a.nl[(int64_t)t * n + b] = k;
-          }
-          count += __popcll(m);
-        }
+    if (r.M > 0) {
+      // system by system (mostly one), so that the grid and domain are uniform
+      const int s_last = __builtin_amdgcn_readfirstlane(r.seg[min(region + 63, n - 1)]);
+      for (int s = __builtin_amdgcn_readfirstlane(r.seg[region]); s <= s_last; ++s) {
+        const SegP& sp = r.segp[s];
+        const int64_t c0 = r.ccref[s];
+        auto row = [&](auto per) {
+          return group_row<D, decltype(per)::value>(lds, r.tP, r.torig, (int)k, (int)(b - k), r.sk[k] - (uint32_t)c0,
+                                                    sp.grid, sp.dom, sp.cutoff_sq, r.starts + c0, r.bond_id, r.bond_w,
+                                                    (!r.isb) && r.bond_w > 0, r.nl, n, r.M, b);
+        };
+        if (active && sg == s)
+          count = sp.dom.kind == JDEM_DOMAIN_PERIODIC ? row(std::true_type{}) : row(std::false_type{});
       }
     }
-    const int c = min(count, a.M);
-    if (l == 0) row_cnt[p] = active ? c : -1;
+    const int c = min(count, r.M);
+    if (l == 0) lds.row_cnt[p] = active ? c : -1;
     __syncthreads();
-    {  // the collected slots, 64 consecutive particles at a time
-      const int64_t bw = reg * 64 + lane;
-      const int cw = row_cnt[lane];
-      for (int s = tid >> 6; s < kRowGrp; s += G) {
-        if (s < cw) a.nl[(int64_t)s * n + bw] = rows[s][lane];
-        if (!__any(s + G < cw)) break;
-      }
-    }
+    write_rows<G>(lds, r.nl, n, region);
     if (active && l == 0) {
-      if (count < a.M) a.nl[(int64_t)count * n + b] = -1;
-      if (count > a.M) atomicOr(a.overflow, 1);
+      if (count < r.M) r.nl[(int64_t)count * n + b] = -1;
+      if (count > r.M) atomicOr(r.overflow, 1);
     }
-    if (a.live) {
-      // history (remap_row): each live old spring goes to the slot of the new
-      // row that lists the same two particles, if any
-      const bool go = active && a.remap != 0;
-      const int64_t ob = go ? (a.cidx ? (int64_t)a.cidx[b] : (int64_t)a.src[b]) : 0;
-      const int64_t os = a.cidx ? a.ostride : n;
-      // start of the old springs, read before any lane writes new offsets
-      const int64_t obase = (go && a.old_W) ? (ob & ~(int64_t)63) * a.M + __float_as_int(a.old_W[ob].w) : 0;
-      uint64_t old[MW], out[MW];
-      int n_old = 0;
-#pragma unroll
-      for (int w = 0; w < MW; ++w) {
-        old[w] = go && w < a.W64 ? a.old_live[(int64_t)w * os + ob] : 0ull;
-        out[w] = 0ull;
-        n_old += __popcll(old[w]);
+    {  // the fields, one kind per wavefront
+      const int64_t bw = region + lane;
+      if (lds.row_cnt[lane] >= 0) {
+        const int sw = r.seg[bw];
+        const int64_t kw = r.cpref[sw] + (bw - r.offsets[sw]);
+        switch (tid >> 6) {
+          case 0: {
+            const float4 x = r.tP[kw];
+            r.old4[bw] = x;  // build position
+            r.P[bw] = D == 2 ? make_float4(x.x, x.y, x.x, x.w) : x;  // and in the 2D records' free lanes
+            break;
+          }
+          case 1: {
+            const float4 v = r.tV[kw];
+            r.V[bw] = D == 2 ? make_float4(v.x, v.y, r.tP[kw].y, v.w) : v;
+            break;
+          }
+          case 2:
+            r.Q[bw] = r.tQ[kw];
+            break;
+          case 3:
+            r.I[bw] = r.tI[kw];
+            break;
+          case 4:
+            r.orig[bw] = r.torig[kw];
+            break;
+          case 5:
+            if (!r.live) r.W[bw] = r.tW[kw];
+            break;
+          default:
+            break;
+        }
       }
-      auto new_slot = [&](int r) {  // of the r-th live old spring, or -1
-        const int32_t o = a.old_nl[(int64_t)select_bit(old, MW, r) * os + ob];
-        if (o < 0) return -1;
-        const int32_t tgt = a.inv[o];
-        for (int s = 0; s < c; ++s)
-          if ((s < kRowGrp ? rows[s][p] : a.nl[(int64_t)s * n + b]) == tgt) return s;
-        return -1;
-      };
-      const int first = l < n_old ? new_slot(l) : -1;  // kept: rows rarely carry more than G springs
-      for (int r = l; r < n_old; r += G) {
-        const int s = r == l ? first : new_slot(r);
-        if (s >= 0)
-#pragma unroll
-          for (int w = 0; w < MW; ++w) out[w] |= (s >> 6) == w ? 1ull << (s & 63) : 0ull;
-      }
-#pragma unroll
-      for (int w = 0; w < MW; ++w) {
-        if (w >= a.W64) break;  // uniform
-#pragma unroll 1
-        for (int d = 1; d < G; d <<= 1) out[w] |= (uint64_t)__shfl_xor((unsigned long long)out[w], d, G);
-      }
-      if (l == 0) {
-        int k = 0;
-#pragma unroll
-        for (int w = 0; w < MW; ++w) k += __popcll(out[w]);
-        new_cnt[p] = k;
-      }
-      __syncthreads();  // old_W is read, the counts are there
-      if (tid < 64) {
-        const int off = wave_exclusive_scan(new_cnt[tid], tid);
-        new_off[tid] = off;
-        const int64_t bw = reg * 64 + tid;
-        if (a.new_W && bw < n) a.new_W[bw].w = __int_as_float(off);
-      }
-      __syncthreads();
-      const int64_t wbase = (b & ~(int64_t)63) * a.M + new_off[p];
-      for (int r = l; r < n_old; r += G) {
-        const int s = r == l ? first : new_slot(r);
-        if (s < 0) continue;
-        const int rank = MW == 1 ? __popcll(out[0] & ((1ull << s) - 1ull))
-                                 : rank_below(out[0], out[MW > 1 ? 1 : 0], out[MW > 2 ? 2 : 0], out[MW > 3 ? 3 : 0], s);
-        const int64_t oi = a.old_W ? obase + r : (int64_t)r * os + ob;
-        a.xi[a.new_W ? wbase + rank : (int64_t)rank * n + b] = a.old_xi[oi];
-      }
-      if (active && l == 0)
-#pragma unroll
-        for (int w = 0; w < MW; ++w)
-          if (w < a.W64) a.live[(int64_t)w * n + b] = out[w];
+    }
+    if (r.live) {
+      const int n_old = active ? r.tlive[k] : 0;
+      int n_kept = 0;
+      if (b < n && !active)
+        for (int w = 0; w < r.W64; ++w) n_kept += __popcll(r.live[(int64_t)w * n + b]);
+      group_springs<G, MW>(
+          lds, active, c, n_old, n_kept, r.nl, n, r.M, r.W64, region, r.xi, r.live,
+          [&](int q) {
+            const int32_t o = r.tnl[(int64_t)q * n + k];
+            return o < 0 ? -1 : r.inv[o];
+          },
+          [&](int q) { return r.txi[(int64_t)q * n + k]; },
+          [&](int ln, int off) {
+            const int64_t bw = region + ln;
+            if (bw >= n) return;
+            if (lds.row_cnt[ln] >= 0) {
+              const int sw = r.seg[bw];
+              const float4 w = r.tW[r.cpref[sw] + (bw - r.offsets[sw])];
+              r.W[bw] = make_float4(w.x, w.y, w.z, __int_as_float(off));
+            } else {
+              r.W[bw].w = __int_as_float(off);
+            }
+          },
+          [&](int q) { return r.keep_xi[(int64_t)q * n + b]; });
     }
     __syncthreads();  // the next region reuses the LDS
   }
 }
-
 
 __global__ void __launch_bounds__(kBlock) k_copy_f4(float4* __restrict__ d, const float4* __restrict__ s, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1021,101 +1091,29 @@ __global__ void __launch_bounds__(kBlock) k_iota(int32_t* __restrict__ p, int64_
 // spring layouts: by rank <-> per wavefront
 // ---------------------------------------------------------------------------
 
-JD bool wave_touched(int64_t b, int64_t n, const int32_t* seg, const int32_t* seg_mode) {
-  if (!seg_mode) return true;
-  const bool mine = b < n && seg_mode[seg[b]] != SEG_KEEP;
-  return __ballot(mine) != 0ull;
-}
-
 __global__ void __launch_bounds__(kBlock) k_pack_springs(int64_t n, int M, int W64, const float4* __restrict__ rank,
                                                           const uint64_t* __restrict__ live, float4* __restrict__ wave,
-                                                          float4* __restrict__ W, const int32_t* __restrict__ seg,
-                                                          const int32_t* __restrict__ seg_mode,
-                                                          const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  const int lane = threadIdx.x & 63;
-  const int64_t npad = (n + 63) & ~(int64_t)63;  // whole waves: every lane of a wave loops alike
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < npad; b += stride) {
-    if (!wave_touched(b, n, seg, seg_mode)) continue;  // wave-uniform
-    int cnt = 0;
-    if (b < n)
-      for (int w = 0; w < W64; ++w) cnt += __popcll(live[(int64_t)w * n + b]);
-    const int off = wave_exclusive_scan(cnt, lane);
-    if (b >= n) continue;
-    float4* dst = wave + (b & ~(int64_t)63) * M + off;
-    for (int k = 0; k < cnt; ++k) dst[k] = rank[(int64_t)k * n + b];
-    W[b].w = __int_as_float(off);
-  }
-}
-
-// The same conversions in a batch rebuild, over the wavefronts that hold a
-// flagged system's particles only (a wavefront shared by two flagged
-// systems is converted twice, to the same values).
-__global__ void __launch_bounds__(kBlock) k_pack_springs_seg(int64_t n, int M, int W64, const float4* __restrict__ rank,
-                                                              const uint64_t* __restrict__ live,
-                                                              float4* __restrict__ wave, float4* __restrict__ W,
-                                                              const int64_t* __restrict__ wpref,
-                                                              const int64_t* __restrict__ offsets, int n_seg,
-                                                              const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  const int lane = threadIdx.x & 63;
-  const int64_t nt = wpref[n_seg] * 64;  // whole waves: every lane of a wave loops alike
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += stride) {
-    const int64_t cw = t >> 6;
-    const int s = seg_of_compact(wpref, n_seg, cw);
-    const int64_t b = ((offsets[s] >> 6) + (cw - wpref[s])) * 64 + lane;
-    int cnt = 0;
-    if (b < n)
-      for (int w = 0; w < W64; ++w) cnt += __popcll(live[(int64_t)w * n + b]);
-    const int off = wave_exclusive_scan(cnt, lane);
-    if (b >= n) continue;
-    float4* dst = wave + (b & ~(int64_t)63) * M + off;
-    for (int k = 0; k < cnt; ++k) dst[k] = rank[(int64_t)k * n + b];
-    W[b].w = __int_as_float(off);
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) k_unpack_springs_seg(int64_t n, int M, int W64,
-                                                                const float4* __restrict__ wave,
-                                                                const uint64_t* __restrict__ live,
-                                                                const float4* __restrict__ W, float4* __restrict__ rank,
-                                                                const int64_t* __restrict__ wpref,
-                                                                const int64_t* __restrict__ offsets, int n_seg,
-                                                                const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  const int lane = threadIdx.x & 63;
-  const int64_t nt = wpref[n_seg] * 64;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += stride) {
-    const int64_t cw = t >> 6;
-    const int s = seg_of_compact(wpref, n_seg, cw);
-    const int64_t b = ((offsets[s] >> 6) + (cw - wpref[s])) * 64 + lane;
-    if (b >= n) continue;
-    int cnt = 0;
+                                                          float4* __restrict__ W) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int cnt = 0;
+  if (b < n)
     for (int w = 0; w < W64; ++w) cnt += __popcll(live[(int64_t)w * n + b]);
-    const float4* src = wave + (b & ~(int64_t)63) * M + __float_as_int(W[b].w);
-    for (int k = 0; k < cnt; ++k) rank[(int64_t)k * n + b] = src[k];
-  }
+  const int off = wave_exclusive_scan(cnt, threadIdx.x & 63);
+  if (b >= n) return;
+  float4* dst = wave + (b & ~(int64_t)63) * M + off;
+  for (int k = 0; k < cnt; ++k) dst[k] = rank[(int64_t)k * n + b];
+  W[b].w = __int_as_float(off);
 }
 
 __global__ void __launch_bounds__(kBlock) k_unpack_springs(int64_t n, int M, int W64, const float4* __restrict__ wave,
                                                             const uint64_t* __restrict__ live,
-                                                            const float4* __restrict__ W, float4* __restrict__ rank,
-                                                            const int32_t* __restrict__ seg,
-                                                            const int32_t* __restrict__ seg_mode,
-                                                            const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  const int64_t npad = (n + 63) & ~(int64_t)63;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < npad; b += stride) {
-    if (!wave_touched(b, n, seg, seg_mode) || b >= n) continue;
-    int cnt = 0;
-    for (int w = 0; w < W64; ++w) cnt += __popcll(live[(int64_t)w * n + b]);
-    const float4* src = wave + (b & ~(int64_t)63) * M + __float_as_int(W[b].w);
-    for (int k = 0; k < cnt; ++k) rank[(int64_t)k * n + b] = src[k];
-  }
+                                                            const float4* __restrict__ W, float4* __restrict__ rank) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= n) return;
+  int cnt = 0;
+  for (int w = 0; w < W64; ++w) cnt += __popcll(live[(int64_t)w * n + b]);
+  const float4* src = wave + (b & ~(int64_t)63) * M + __float_as_int(W[b].w);
+  for (int k = 0; k < cnt; ++k) rank[(int64_t)k * n + b] = src[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -1530,30 +1528,15 @@ hipError_t launch_ws_dim(const WS& a, int law, bool per, hipStream_t s) {
 }
 
 hipError_t ws_launch_pack_springs(int64_t n, int M, int W64, const float4* rank, const uint64_t* live, float4* wave,
-                                  float4* W, const int32_t* seg, const int32_t* seg_mode, hipStream_t s,
-                                  const int32_t* gate, const int64_t* wpref, const int64_t* offsets, int n_seg) {
+                                  float4* W, hipStream_t s) {
   if (n == 0 || M == 0) return hipSuccess;
-  if (wpref)
-    hipLaunchKernelGGL(k_pack_springs_seg, dim3(std::min<unsigned>(nblocks(n + 64 * (int64_t)n_seg), (unsigned)kCappedGrid)),
-                       dim3(kBlock), 0, s, n, M, W64, rank, live, wave, W, wpref, offsets, n_seg, gate);
-  else
-    hipLaunchKernelGGL(k_pack_springs, dim3(gate ? std::min<unsigned>(nblocks(n), (unsigned)kCappedGrid) : nblocks(n)),
-                       dim3(kBlock), 0, s, n, M, W64, rank, live, wave, W, seg, seg_mode, gate);
+  hipLaunchKernelGGL(k_pack_springs, dim3(nblocks(n)), dim3(kBlock), 0, s, n, M, W64, rank, live, wave, W);
   return hipGetLastError();
 }
 hipError_t ws_launch_unpack_springs(int64_t n, int M, int W64, const float4* wave, const uint64_t* live,
-                                    const float4* W, float4* rank, const int32_t* seg, const int32_t* seg_mode,
-                                    hipStream_t s, const int32_t* gate, const int64_t* wpref,
-                                    const int64_t* offsets, int n_seg) {
+                                    const float4* W, float4* rank, hipStream_t s) {
   if (n == 0 || M == 0) return hipSuccess;
-  if (wpref)
-    hipLaunchKernelGGL(k_unpack_springs_seg,
-                       dim3(std::min<unsigned>(nblocks(n + 64 * (int64_t)n_seg), (unsigned)kCappedGrid)), dim3(kBlock),
-                       0, s, n, M, W64, wave, live, W, rank, wpref, offsets, n_seg, gate);
-  else
-    hipLaunchKernelGGL(k_unpack_springs,
-                       dim3(gate ? std::min<unsigned>(nblocks(n), (unsigned)kCappedGrid) : nblocks(n)), dim3(kBlock),
-                       0, s, n, M, W64, wave, live, W, rank, seg, seg_mode, gate);
+  hipLaunchKernelGGL(k_unpack_springs, dim3(nblocks(n)), dim3(kBlock), 0, s, n, M, W64, wave, live, W, rank);
   return hipGetLastError();
 }
 
@@ -1608,18 +1591,6 @@ hipError_t ws_launch_out(const InOut& io, bool with_nl, hipStream_t s) {
   dim3 g(nblocks(io.n)), b(kBlock);
   hipLaunchKernelGGL(k_out_state, g, b, 0, s, io);
   if (with_nl) hipLaunchKernelGGL(k_out_nlist, g, b, 0, s, io);
-  return hipGetLastError();
-}
-__global__ void k_gate_end(int32_t* __restrict__ gate) { *gate = 0; }
-__global__ void k_gated_zero(const int32_t* __restrict__ gate, int32_t* __restrict__ word) {
-  if (*gate) *word = 0;
-}
-hipError_t ws_launch_gate_end(int32_t* gate, hipStream_t s) {
-  hipLaunchKernelGGL(k_gate_end, dim3(1), dim3(1), 0, s, gate);
-  return hipGetLastError();
-}
-hipError_t ws_launch_gated_zero(const int32_t* gate, int32_t* word, hipStream_t s) {
-  hipLaunchKernelGGL(k_gated_zero, dim3(1), dim3(1), 0, s, gate, word);
   return hipGetLastError();
 }
 hipError_t ws_launch_export(const InOut& io, hipStream_t s) {
@@ -1677,33 +1648,38 @@ hipError_t ws_launch_permute(int64_t n, const int32_t* new_orig, const int32_t* 
                      Q2, I2, orig2, src, inv, old2, dim);
   return hipGetLastError();
 }
-hipError_t ws_launch_seg_prefix(int n_seg, const int32_t* seg_mode, const int64_t* offsets, const SegP* segp,
-                               int64_t* cpref, int64_t* ccref, int64_t* wpref, hipStream_t s) {
-  hipLaunchKernelGGL(k_seg_prefix, dim3(1), dim3(1024), 0, s, n_seg, seg_mode, offsets, segp, cpref, ccref, wpref);
+hipError_t ws_launch_rebuild_plan(const RB& r, const RBPlan& p, hipStream_t s) {
+  hipLaunchKernelGGL(k_rebuild_plan, dim3(1), dim3(1024), 0, s, r, p);
   return hipGetLastError();
 }
-hipError_t ws_launch_hash_flagged(const RB& r, int dim, hipStream_t s) {
-  if (r.n == 0) return hipSuccess;
-  const dim3 g(r.gate ? std::min<unsigned>(nblocks(r.n), (unsigned)kCappedGrid) : nblocks(r.n));
-  if (dim == 3)
-    hipLaunchKernelGGL(k_hash_flagged<3>, g, dim3(kBlock), 0, s, r);
+hipError_t ws_launch_rebuild_keys(const RB& r, hipStream_t s) {
+  const dim3 g(std::min<unsigned>(nblocks(r.n), (unsigned)kCappedGrid));
+  if (r.dim == 3)
+    hipLaunchKernelGGL(k_rebuild_keys<3>, g, dim3(kBlock), 0, s, r);
   else
-    hipLaunchKernelGGL(k_hash_flagged<2>, g, dim3(kBlock), 0, s, r);
+    hipLaunchKernelGGL(k_rebuild_keys<2>, g, dim3(kBlock), 0, s, r);
   return hipGetLastError();
 }
-hipError_t ws_launch_place(const RB& r, const uint32_t* sk, int32_t* starts, hipStream_t s) {
-  if (r.fn == 0) return hipSuccess;
-  // a device count: a capped grid that walks the flagged particles in turn
-  const dim3 g(r.fn >= 0 ? nblocks(r.fn) : std::min<unsigned>(nblocks(r.n), (unsigned)kCappedGrid)), b(kBlock);
-  hipLaunchKernelGGL(k_place_gather, g, b, 0, s, r);
-  hipLaunchKernelGGL(k_place_scatter, g, b, 0, s, r);
-  hipLaunchKernelGGL(k_cell_starts_flagged, g, b, 0, s, r, sk, starts);
+hipError_t ws_launch_rebuild_gather(const RB& r, hipStream_t s) {
+  hipLaunchKernelGGL(k_rebuild_gather, dim3(std::min<unsigned>(nblocks(r.n), (unsigned)kCappedGrid)), dim3(kBlock), 0,
+                     s, r);
   return hipGetLastError();
 }
-hipError_t ws_launch_seg_modes(int n_seg, int32_t* seg_flag, int32_t* n_build, int32_t* seg_mode, hipStream_t s,
-                               const int32_t* gate, int32_t* events) {
-  hipLaunchKernelGGL(k_seg_modes, dim3(nblocks(n_seg)), dim3(kBlock), 0, s, n_seg, seg_flag, n_build, seg_mode, gate,
-                     events);
+template <int D>
+void launch_rebuild_rows(const RB& r, hipStream_t s) {
+  // as many workgroups as are resident at once
+  const unsigned resident = 256u * 2048u / (64u * nlist_group<D>());
+  const dim3 g(std::min<unsigned>(nblocks(r.n, 64), resident)), b(64 * nlist_group<D>());
+  if (r.W64 <= 1)
+    hipLaunchKernelGGL((k_rebuild_rows<D, 1>), g, b, 0, s, r);
+  else
+    hipLaunchKernelGGL((k_rebuild_rows<D, 4>), g, b, 0, s, r);
+}
+hipError_t ws_launch_rebuild_rows(const RB& r, hipStream_t s) {
+  if (r.dim == 3)
+    launch_rebuild_rows<3>(r, s);
+  else
+    launch_rebuild_rows<2>(r, s);
   return hipGetLastError();
 }
 hipError_t ws_launch_seg_init_flags(int n_seg, const int32_t* n_build, int32_t* seg_flag, hipStream_t s,
@@ -1753,12 +1729,6 @@ hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s) {
       else
         hipLaunchKernelGGL((k_nlist_work_naive<2, false>), g, b, 0, s, a);
     }
-  } else if (a.segp) {
-    const dim3 gs(a.gate ? std::min<unsigned>(g.x, (unsigned)kCappedGrid) : g.x);
-    if (dim == 3)
-      hipLaunchKernelGGL((k_nlist_work<3, 2>), gs, b, 0, s, a);
-    else
-      hipLaunchKernelGGL((k_nlist_work<2, 2>), gs, b, 0, s, a);
   } else if (a.n < kNlistLane) {
     if (a.W64 <= 1)
       launch_nlist_group<1>(a, dim, per, s);
@@ -1767,14 +1737,14 @@ hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s) {
   } else {
     if (dim == 3) {
       if (per)
-        hipLaunchKernelGGL((k_nlist_work<3, 1>), g, b, 0, s, a);
+        hipLaunchKernelGGL((k_nlist_work<3, true>), g, b, 0, s, a);
       else
-        hipLaunchKernelGGL((k_nlist_work<3, 0>), g, b, 0, s, a);
+        hipLaunchKernelGGL((k_nlist_work<3, false>), g, b, 0, s, a);
     } else {
       if (per)
-        hipLaunchKernelGGL((k_nlist_work<2, 1>), g, b, 0, s, a);
+        hipLaunchKernelGGL((k_nlist_work<2, true>), g, b, 0, s, a);
       else
-        hipLaunchKernelGGL((k_nlist_work<2, 0>), g, b, 0, s, a);
+        hipLaunchKernelGGL((k_nlist_work<2, false>), g, b, 0, s, a);
     }
   }
   return hipGetLastError();

@@ -58,3 +58,31 @@ def test_rebuilds_against_the_oracle(device, dim, domain, N, phi, skin, edge, rr
     assert np.array_equal(got.nl, nls.nl)
     assert np.array_equal(got.live, nls.live)
     assert_bitwise("springs", got.xi, np.where(nls.live[..., None], nls.xi, np.float32(0.0)))
+
+
+@pytest.mark.parametrize("dim,sizes,phi,rr,limit", [
+    (3, (63, 5, 129, 700, 64), 0.7, (0.4, 0.6), 64),  # wavefronts shared by rebuilt and kept systems
+    (3, (257, 40, 300), 2.5, (0.4, 0.6), 100),  # rows of up to 80 slots
+    (2, (30, 500, 1, 65), 4.0, (0.1, 0.6), 250),  # rows of 90 slots, tens of springs
+])
+def test_batch_rebuilds_equal_alone(device, dim, sizes, phi, rr, limit):
+    """Systems of a batch that rebuild at different steps, each as stepped
+    alone (in two calls, the second starting from lists with live springs)."""
+    print(f"[list] batch dim={dim} sizes={sizes}", flush=True)
+    mats = [jd.Material.create("elasticfrict", density=1.0, young=1e2, poisson=0.3, mu=0.4, e=0.7, mu_r=0.05)]
+    pairs = []
+    for k, N in enumerate(sizes):
+        domain = "periodic" if k % 2 else "reflect"
+        st, box = packed(N, dim, seed=N + dim, domain=domain, phi=phi, rr=rr)
+        ckw = dict(state=st, cutoff=1.2, skin=0.1 + 0.1 * k, max_neighbors=min(limit, N), secondary_collider_type="CellList",
+                   secondary_collider_kw=dict(state=st))
+        pairs.append((st, jd.System.create(
+            st.shape, dt=4e-3, domain_type=domain, domain_kw=dict(box_size=box, anchor=np.zeros(dim)),
+            collider_type="NeighborList", collider_kw=ckw, force_model_type="springfriction",
+            mat_table=jd.MaterialTable.from_materials(mats))))
+    out = jd.Batch.pack(pairs).step(17).step(16).unpack()
+    for k, ((st, sy), (sb, yb)) in enumerate(zip(pairs, out)):
+        sa, ya = jd.System.step(st, sy, n=17)
+        sa, ya = jd.System.step(sa, ya, n=16)
+        _compare_states(sb, B.state_of(sa), f"system {k}")
+        assert ya.collider.n_build_times == yb.collider.n_build_times >= (1 if sizes[k] == 1 else 2)
