@@ -1143,9 +1143,10 @@ JD Vec<D> disp_pm(Vec<D> a, Vec<D> b, const DomP& d) {
   return disp_<PM == 1>(a, b, d);
 }
 
-// LDS of the lane-balanced force pass: per wave, kPairCap pair descriptors
-// (a wave with more marked slots takes them in several chunks) and one round
-// of 64 pair results (force + contact flag, torque, spring).
+// LDS of the lane-balanced force pass: per 64 particles and wave that works
+// on them, kPairCap pair descriptors (more marked slots are taken in several
+// chunks) and one round of 64 pair results (force + contact flag, torque,
+// spring).
 constexpr int kPairCap = 128;
 // pass 1 keeps the partner index of a lane's first kStash marked slots in LDS,
 // so the pair evaluation need not reload it from the list
@@ -1155,19 +1156,35 @@ constexpr int kStash = 4;
 // the per-lane slot masks then take 2 * MW registers
 // BS = workgroup size (the tile width: 256, or 128 for batches when the
 // autotuner prefers it)
-template <int D, int LAW, int PM, int MW, int BS = kBlock>
+// NW = waves per 64 particles: 1, or 4 for small systems (below kWsSplit particles), where a
+// lane's walk of its row, two dependent loads per four slots, is what a step
+// takes and too few waves hide it.  Then the workgroup's waves share the
+// rows of 64 particles, four slots in turn each, and the marked pairs; the
+// first wave adds up and integrates.
+template <int D, int LAW, int PM, int MW, int BS = kBlock, int NW = 1>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_waves<D, LAW, PM, MW>(), 8))) k_ws_step(WS a) {
-  __shared__ int pdesc[BS / 64][kPairCap];
-  __shared__ int pjx[BS / 64][kPairCap];
+  static_assert(NW == 1 || NW == BS / 64, "the waves of a workgroup share 64 particles, or none");
+  constexpr int kSets = NW == 1 ? BS / 64 : 1, kCap = kPairCap * NW, kRound = 64 * NW;
+  __shared__ int pdesc[kSets][kCap];
+  __shared__ int pjx[kSets][kCap];
   __shared__ int pstash[BS / 64][kStash][64];
-  __shared__ float4 pres[BS / 64][3][64];
+  __shared__ float4 pres[kSets][3][kRound];
+  __shared__ int row_end[64];
+  __shared__ uint64_t marks[NW][MW][64];
+  auto sync = [] {
+    if (NW == 1)
+      wave_sync();
+    else
+      __syncthreads();
+  };
   if (a.flag_rd && *a.flag_rd) {
     if (a.flag_wr) *a.flag_wr = *a.flag_rd;
     return;
   }
   // every lane of a wave stays to the end of the force pass, which works
   // wave-wide; a lane past the end reads the last particle and writes nothing
-  const int64_t b0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, set = NW == 1 ? wv : 0;
+  const int64_t b0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * (BS / NW) + (NW == 1 ? (int)threadIdx.x : lane);
   const bool active = b0 < a.n;
   const int64_t b = active ? b0 : a.n - 1;
   DomP dom;
@@ -1205,9 +1222,13 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
 #pragma unroll
     for (int q = 0; q < MW; ++q) cm[q] = 0ull;
     int n_marked = 0;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (NW > 1) {  // the first -1 that any wave has come to
+      if (wv == 0) row_end[lane] = a.M;
+      __syncthreads();
+    }
     bool done = false;
-    for (int s0 = 0; s0 < a.M && !done; s0 += PF) {
+    for (int s0 = NW == 1 ? 0 : wv * PF; s0 < a.M && !done; s0 += NW * PF) {
+      if (NW > 1 && s0 >= *(volatile int*)&row_end[lane]) break;
       int32_t js[PF];
       float4 pjs[PF];
 #pragma unroll
@@ -1215,12 +1236,17 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
       // the row ends at its first -1: what follows is stale
 #pragma unroll
       for (int k = 1; k < PF; ++k) js[k] = js[k - 1] < 0 ? -1 : js[k];
+      // (a wave of several may have come past the end of the row: what it
+      // finds there is dropped below, but must not be read through)
 #pragma unroll
-      for (int k = 0; k < PF; ++k) pjs[k] = (js[k] >= 0) ? a.P[js[k]] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int k = 0; k < PF; ++k)
+        pjs[k] = (NW == 1 ? js[k] >= 0 : (uint64_t)(int64_t)js[k] < (uint64_t)a.n) ? a.P[js[k]]
+                                                                                 : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int k = 0; k < PF; ++k) {
         if (js[k] < 0) {
           done = true;
+          if (NW > 1 && s0 + k < a.M) atomicMin(&row_end[lane], s0 + k);
           break;
         }
         const float4 pj = pjs[k];
@@ -1244,6 +1270,26 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
       if (!active) cm[q] = 0ull;
       nc += __popcll(cm[q]);
     }
+    // all waves' marks up to the row's end; cm keeps this wave's
+    uint64_t all[MW];
+    if constexpr (NW > 1) {
+#pragma unroll
+      for (int q = 0; q < MW; ++q) marks[wv][q][lane] = cm[q];
+      __syncthreads();
+      const int end = row_end[lane];
+      nc = 0;
+#pragma unroll
+      for (int q = 0; q < MW; ++q) {
+        const int e = end - q * 64;
+        const uint64_t keep = e >= 64 ? ~0ull : (e <= 0 ? 0ull : (1ull << e) - 1ull);
+        all[q] = 0ull;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) all[q] |= marks[w][q][lane];
+        all[q] &= keep;
+        cm[q] &= keep;
+        nc += __popcll(all[q]);
+      }
+    }
     // Pass 2, lane-balanced: the wave's marked slots are numbered lane by
     // lane (slot order within a lane) and dealt out 64 at a time, one pair
     // per lane, so the law runs ceil(total / 64) times per wave instead of
@@ -1263,16 +1309,17 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
 #pragma unroll
     for (int q = 0; q < MW; ++q) ln[q] = 0ull;
     int rank_new = 0;  // springs are stored by rank
-    for (int cb = 0; cb < total; cb += kPairCap) {  // wave-uniform
-      // descriptors of pairs cb .. cb + kPairCap - 1: owner lane | slot << 6
+    for (int cb = 0; cb < total; cb += kCap) {  // uniform over the waves of a set
+      // descriptors of pairs cb .. cb + kCap - 1: owner lane | slot << 6
       // | (old spring's place in the wave's region + 1) << 14, and the
       // partner index
-      if (off < cb + kPairCap && off + nc > cb) {
+      if (off < cb + kCap && off + nc > cb) {
         // old springs: this slot's start in the wave's spring region
         int idx = off, rank_base = LawTraits<LAW>::hist ? __float_as_int(a.W[b].w) : 0, c = 0;
 #pragma unroll
         for (int w = 0; w < MW; ++w) {
           uint64_t cmw = w < n_words ? cm[w] : 0ull;
+          const int first = idx;  // of this word's marked slots
           uint64_t live_old = 0ull;
           if constexpr (LawTraits<LAW>::hist)
             if (w < n_words) live_old = a.live[(int64_t)w * a.n + b];
@@ -1280,29 +1327,32 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
           while (cmw) {
             const int sl = __ffsll((unsigned long long)cmw) - 1;
             cmw &= cmw - 1ull;
+            if constexpr (NW > 1) idx = first + __popcll(all[w] & ((1ull << sl) - 1ull));
             int k = -1;
             if constexpr (LawTraits<LAW>::hist)
               if ((live_old >> sl) & 1ull) k = rank_base + __popcll(live_old & ((1ull << sl) - 1ull));
-            if (idx >= cb && idx < cb + kPairCap) {
-              pdesc[wv][idx - cb] = lane | ((w * 64 + sl) << 6) | ((k + 1) << 14);
+            if (idx >= cb && idx < cb + kCap) {
+              pdesc[set][idx - cb] = lane | ((w * 64 + sl) << 6) | ((k + 1) << 14);
               // the LDS read is unconditional, so the two sources stay two
               // loads (not one flat load through a selected pointer)
               int jj = pstash[wv][min(c, kStash - 1)][lane];
               if (c >= kStash) jj = a.nl[(int64_t)(w * 64 + sl) * a.n + b];
-              pjx[wv][idx - cb] = jj;
+              pjx[set][idx - cb] = jj;
             }
             ++idx;
             ++c;
           }
+          if constexpr (NW > 1) idx = first + __popcll(all[w]);
           if constexpr (LawTraits<LAW>::hist) rank_base += __popcll(live_old);
         }
       }
-      const int tc = min(total - cb, kPairCap);
-      for (int r0 = 0; r0 < tc; r0 += 64) {
-        wave_sync();
-        if (r0 + lane < tc) {
-          const int dsc = pdesc[wv][r0 + lane];
-          const int32_t j = pjx[wv][r0 + lane];
+      const int tc = min(total - cb, kCap);
+      const int pl = NW == 1 ? lane : (int)threadIdx.x;  // place in the round
+      for (int r0 = 0; r0 < tc; r0 += kRound) {
+        sync();
+        if (r0 + pl < tc) {
+          const int dsc = pdesc[set][r0 + pl];
+          const int32_t j = pjx[set][r0 + pl];
           const int64_t bo = b0 - lane + (dsc & 63);
           const int k = (dsc >> 14) - 1;
           // every load of the pair is issued before any is used
@@ -1356,23 +1406,23 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
           const Vec<D> rij = disp_pm<PM>(mo.x, o.x, dom_o);
           const float d_sq = dot(rij, rij);
           const PairOut<D> r = law_eval<D, LAW>(a.law, mo, o, rij, d_sq, xold, dt_o);
-          pres[wv][0][lane] = f4(r.F, r.contact ? 1.0f : 0.0f);
-          if constexpr (LawTraits<LAW>::torque) pres[wv][1][lane] = f4a(r.T);
-          if constexpr (LawTraits<LAW>::hist) pres[wv][2][lane] = f4(r.xi, 0.0f);
+          pres[set][0][pl] = f4(r.F, r.contact ? 1.0f : 0.0f);
+          if constexpr (LawTraits<LAW>::torque) pres[set][1][pl] = f4a(r.T);
+          if constexpr (LawTraits<LAW>::hist) pres[set][2][pl] = f4(r.xi, 0.0f);
         }
-        wave_sync();
-        const int q0 = cb + r0, q1 = min(off + nc, q0 + 64);
+        sync();
+        const int q0 = cb + r0, q1 = NW > 1 && wv > 0 ? 0 : min(off + nc, q0 + kRound);
 #pragma unroll 1
         for (int q = max(off, q0); q < q1; ++q) {
-          const float4 fr = pres[wv][0][q - q0];
+          const float4 fr = pres[set][0][q - q0];
           F = F + xyz<D>(fr);
-          if constexpr (LawTraits<LAW>::torque) T = T + ang4<D>(pres[wv][1][q - q0]);
+          if constexpr (LawTraits<LAW>::torque) T = T + ang4<D>(pres[set][1][q - q0]);
           if constexpr (LawTraits<LAW>::hist) {
             if (fr.w != 0.0f) {
-              const int sl = (pdesc[wv][q - cb] >> 6) & 255;
+              const int sl = (pdesc[set][q - cb] >> 6) & 255;
               // new springs from the slot's marked-pair prefix: the wave's
               // springs fill one contiguous run of its region
-              a.xi_wr[(b0 - lane) * a.M + off + rank_new] = pres[wv][2][q - q0];
+              a.xi_wr[(b0 - lane) * a.M + off + rank_new] = pres[set][2][q - q0];
               ++rank_new;
               const uint64_t bit = 1ull << (sl & 63);
               const int ws = sl >> 6;
@@ -1382,8 +1432,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
           }
         }
       }
-      wave_sync();  // the next chunk's descriptors overwrite these
+      sync();  // the next chunk's descriptors overwrite these
     }
+    if (NW > 1 && wv > 0) return;
     if constexpr (LawTraits<LAW>::hist)
       if (active)
 #pragma unroll
@@ -1393,6 +1444,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
             if (a.live[li] != ln[w]) a.live[li] = ln[w];
           }
   } else {
+    if (NW > 1 && wv > 0) return;
     F = xyz<D>(a.F[b]);
     T = ang4<D>(a.T[b]);
   }
@@ -1483,9 +1535,28 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
   }
 }
 
+// Below this many spheres four waves share the rows of 64.  A step with one /
+// four, us: spring-friction, bidisperse 17 / 9.6 at 10 k, 17.6 / 10.8 at 37 k,
+// 18.5 / 13.3 at 70 k, 19.3 / 16.8 at 100 k, 24 / 26 at 200 k; log-normal radii
+// 19 / 12, 21 / 14, 21 / 18, 24 / 27.  Rows of disks are short: 8 / 7 below
+// 20 k, 8 / 8 at 37 k, 9.3 / 12.5 at 100 k, so one wave takes them all.
+constexpr int64_t kWsSplit = 80000;
+
 template <int D, int LAW, int MW>
 void launch_ws_mw(const WS& a, bool per, hipStream_t s) {
   dim3 g(nblocks(a.n)), b(kBlock);
+  if constexpr (D == 3) {
+    if (a.n < kWsSplit) {
+      const dim3 g4(nblocks(a.n, 64));
+      if (a.segp)
+        hipLaunchKernelGGL((k_ws_step<D, LAW, 2, MW, kBlock, 4>), g4, b, 0, s, a);
+      else if (per)
+        hipLaunchKernelGGL((k_ws_step<D, LAW, 1, MW, kBlock, 4>), g4, b, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_ws_step<D, LAW, 0, MW, kBlock, 4>), g4, b, 0, s, a);
+      return;
+    }
+  }
   if (a.segp && a.block == 128)
     hipLaunchKernelGGL((k_ws_step<D, LAW, 2, MW, 128>), dim3(nblocks(a.n, 128)), dim3(128), 0, s, a);
   else if (a.segp)
