@@ -90,3 +90,26 @@ def test_batch_rebuilds_equal_alone(device, dim, sizes, phi, rr, limit):
         sa, ya = jd.System.step(sa, ya, n=16)
         _compare_states(sb, B.state_of(sa), f"system {k}")
         assert ya.collider.n_build_times == yb.collider.n_build_times >= (1 if sizes[k] == 1 else 2)
+
+
+@pytest.mark.parametrize("strides", [(7, 7, 1, 7, 13), (0, 2, 0, 31), (0, 0)])
+def test_rollout_segments_equal_steps(device, strides):
+    """Rebuilds every few steps, predicted across the segments of a rollout
+    (also ones of no step, and a rollout of none, whose list stays unbuilt):
+    each frame as stepped there, the same builds."""
+    print(f"[list] rollout strides={strides}", flush=True)
+    st, box = packed(300, 3, seed=9, domain="periodic", phi=0.6)
+    mats = [jd.Material.create("elasticfrict", density=1.0, young=1e2, poisson=0.3, mu=0.4, e=0.7, mu_r=0.05)]
+    ckw = dict(state=st, cutoff=1.2, skin=0.15, secondary_collider_type="CellList", secondary_collider_kw=dict(state=st))
+    sy = jd.System.create(st.shape, dt=4e-3, domain_type="periodic", domain_kw=dict(box_size=box, anchor=np.zeros(3)),
+                          collider_type="NeighborList", collider_kw=ckw, force_model_type="springfriction",
+                          mat_table=jd.MaterialTable.from_materials(mats))
+    fs, fy, traj = jd.System.trajectory_rollout(st, sy, strides=np.array(strides), save_fn=jd.save_state)
+    sa, ya = st, sy
+    for f, k in enumerate(strides):
+        if k:
+            sa, ya = jd.System.step(sa, ya, n=k)
+        assert_bitwise(f"frame {f}", traj.pos_c[f].cpu().numpy(), sa.pos_c.cpu().numpy())
+    _compare_states(fs, B.state_of(sa), "end")
+    assert fy.collider.n_build_times == ya.collider.n_build_times
+    assert np.array_equal(fy.collider.neighbor_list.cpu().numpy(), ya.collider.neighbor_list.cpu().numpy())
