@@ -1935,8 +1935,13 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
   hipStream_t st = ctx->stream;
   const int nparts = std::max(1u, nblocks(N));
   ENSURE(ctx, ctx->fireV, 4 * (size_t)std::max<int64_t>(N, 1) * (D + A));
-  ENSURE(ctx, ctx->fireDev, sizeof(FireDev) + 8 * (size_t)nparts);
-  ENSURE(ctx, ctx->red, 8 * ((size_t)std::max<int64_t>(N, 1) + 256 + 1));
+  struct Dev {
+    FireDev fire;
+    FireStop ls;
+  };
+  ENSURE(ctx, ctx->fireDev, sizeof(Dev));
+  ENSURE(ctx, ctx->red, 8 * ((size_t)std::max<int64_t>(N, 1) + 2 * (size_t)nparts) + 4 * (size_t)nparts);
+  Dev* dev = (Dev*)ctx->fireDev.p;
   FireArgs f;
   std::memset(&f, 0, sizeof(f));
   f.n = N;
@@ -1951,8 +1956,8 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
   f.p.dt_min = (float)(fire->dt * fire->dt_min_scale);
   f.p.n_min = fire->n_min;
   f.p.n_bad_max = fire->n_bad_max;
-  f.st = (FireDev*)ctx->fireDev.p;
-  f.part = (double*)((char*)ctx->fireDev.p + sizeof(FireDev));
+  f.st = &dev->fire;
+  f.ls = &dev->ls;
   f.nparts = nparts;
   f.force = s.force;
   f.torque = s.torque;
@@ -1964,20 +1969,23 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
   for (int c = 0; c < 3; ++c) f.g[c] = sys->gravity[c];
   f.mass = s.mass;
   double* per = (double*)ctx->red.p;
-  double* part = per + std::max<int64_t>(N, 1);
-  double* out = part + 256;
-  f.e_out = per;
-  const bool grav = sys->gravity[0] != 0.0f || sys->gravity[1] != 0.0f || sys->gravity[2] != 0.0f;
+  f.part = per + std::max<int64_t>(N, 1);
+  f.gpart = (unsigned*)(f.part + 2 * (size_t)nparts);
+  f.stop.pe_tol = pe_tol;
+  f.stop.pe_diff_tol = pe_diff_tol;
+  f.stop.force_tol = force_tol;
+  f.stop.dN = (double)std::max<int64_t>(N, 1);
+  f.stop.max_steps = max_steps;
   // optimiser state: zero velocities, dt = dt0, alpha = alpha_init (optimizers.py:231-239)
   HIPCHK(ctx, hipMemsetAsync(ctx->fireV.p, 0, 4 * (size_t)std::max<int64_t>(N, 1) * (D + A), st));
-  FireDev h0;
-  std::memset(&h0, 0, sizeof(h0));
-  h0.dt = (float)fire->dt;
-  h0.alpha = (float)fire->alpha_init;
-  HIPCHK(ctx, hipMemcpyAsync(f.st, &h0, sizeof(h0), hipMemcpyHostToDevice, st));
+  Dev h;
+  std::memset(&h, 0, sizeof(h));
+  h.fire.dt = (float)fire->dt;
+  h.fire.alpha = (float)fire->alpha_init;
+  h.ls.prev = INFINITY;
+  HIPCHK(ctx, hipMemcpyAsync(dev, &h, sizeof(h), hipMemcpyHostToDevice, st));
 
-  // eval_step (routines.py:228-245): force, ForceManager, energy, max |grad|
-  double pe = 0.0, gmax = 0.0;
+  // eval_step (routines.py:228-245) and the next update's decision
   auto eval = [&]() -> int {
     if (sys->collider_kind == JDEM_COLLIDER_NEIGHBOR_LIST) {
       bool rebuilt = false;
@@ -1994,60 +2002,38 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
       a.do_force = 1;
       HIPCHK(ctx, launch_step(a, D, a.law.kind, src_of(sys->collider_kind), st));
     }
-    if (N > 0) HIPCHK(ctx, launch_stage(a, D, JDEM_STAGE_FORCE_MANAGER, st));
-    HIPCHK(ctx, hipMemsetAsync(&f.st->max_grad_bits, 0, sizeof(unsigned), st));
-    HIPCHK(ctx, launch_fire_grad_max(f, st));
-    double h[2] = {0.0, 0.0};
-    if (N > 0) {
-      if (sys->collider_kind != JDEM_COLLIDER_NONE) {
-        a.e_out = per;
-        HIPCHK(ctx, launch_energy(a, D, a.law.kind, src_of(sys->collider_kind), st));
-      } else {
-        HIPCHK(ctx, hipMemsetAsync(per, 0, 8 * (size_t)N, st));
-      }
-      if (grav) HIPCHK(ctx, launch_fire_gravity_energy(f, st));
-      HIPCHK(ctx, launch_sum_f64(per, N, 1, 1, part, out, 256, st));
-      HIPCHK(ctx, hipMemcpyAsync(&h[0], out, 8, hipMemcpyDeviceToHost, st));
+    f.e_in = nullptr;
+    if (N > 0 && sys->collider_kind != JDEM_COLLIDER_NONE) {
+      a.e_out = per;
+      HIPCHK(ctx, launch_energy(a, D, a.law.kind, src_of(sys->collider_kind), st));
+      f.e_in = per;
     }
-    unsigned bits = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&bits, &f.st->max_grad_bits, sizeof(bits), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    float g;
-    std::memcpy(&g, &bits, sizeof(g));
-    pe = h[0];
-    gmax = (double)g;
+    HIPCHK(ctx, launch_fire_terms(f, st));
+    HIPCHK(ctx, launch_fire_decide(f, st));
     return JDEM_OK;
   };
 
   rc = eval();
   if (rc) return rc;
-  double prev = INFINITY;
-  int64_t steps = 0;
-  const double tiny = 2.2250738585072014e-308;  // smallest normal float64
-  const double dN = (double)std::max<int64_t>(N, 1);
-  while (steps < max_steps) {
-    const bool conv_pe = std::fabs(pe / dN) <= pe_tol;
-    const double denom = std::max(std::max(std::fabs(pe), std::fabs(prev)), tiny);
-    const bool conv_rel = std::fabs(pe - prev) / denom < pe_diff_tol;
-    const bool conv_f = gmax <= force_tol;
-    if (conv_pe || conv_rel || conv_f) break;
-    HIPCHK(ctx, launch_fire_power(f, st));
-    HIPCHK(ctx, launch_fire_decide(f, st));
-    HIPCHK(ctx, launch_fire_move(f, st));
-    HIPCHK(ctx, launch_fire_commit(f, st));  // dt, alpha <- the values just decided
-    prev = pe;
-    rc = eval();
-    if (rc) return rc;
-    ++steps;
+  // Iterations run in chunks between two reads of the loop's state, each a
+  // quarter of the steps so far (4 to 32), so that few are launched past a stop.
+  for (int64_t done = 0;;) {
+    HIPCHK(ctx, hipMemcpyAsync(&h, dev, sizeof(h), hipMemcpyDeviceToHost, st));
+    HIPCHK(ctx, hipStreamSynchronize(st));
+    if (h.ls.stop) break;
+    const int64_t todo = std::min(max_steps - done, std::min<int64_t>(32, std::max<int64_t>(4, done / 4)));
+    for (int64_t k = 0; k < todo; ++k) {
+      HIPCHK(ctx, launch_fire_move(f, st));
+      rc = eval();
+      if (rc) return rc;
+    }
+    done += todo;
   }
   if (stats) {
-    FireDev h;
-    HIPCHK(ctx, hipMemcpyAsync(&h, f.st, sizeof(h), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    stats->steps = steps;
-    stats->pe = pe / dN;
-    stats->max_grad = gmax;
-    stats->power = h.power;
+    stats->steps = h.ls.steps;
+    stats->pe = h.ls.pe / f.stop.dN;
+    stats->max_grad = h.ls.gmax;
+    stats->power = h.fire.power;
     stats->overflow = sys->collider_kind == JDEM_COLLIDER_NEIGHBOR_LIST ? sys->nlist.overflow : 0;
   }
   return JDEM_OK;

@@ -678,33 +678,41 @@ struct FireDev {
   int n_good, n_bad;
   float new_dt, new_alpha, dt_rev, vs;
   double power;
-  unsigned max_grad_bits;  // max |grad| component as float bits
-  float dt_used;           // precision form: dt of the update just decided (dt is the next one's)
+  float dt_used;  // dt of the update just decided (dt is the next one's)
+};
+// Where a FIRE loop decided on the device stands, and its tests (routines.py:
+// 284-314).
+struct FireStop {
+  double pe, prev, gmax;
+  long long steps;
+  int32_t stop;
+};
+struct FireStopP {
+  double pe_tol, pe_diff_tol, force_tol, dN;
+  long long max_steps;
 };
 struct FireArgs {
   int64_t n;
   int dim;
   FireP p;
   FireDev* st;
-  const float* force;
+  FireStop* ls;
+  FireStopP stop;
+  float* force;
   const float* torque;
   const uint8_t* fixed;
   float* vel_pos;
   float* vel_rot;
   float* pos;
   float* q;
-  double* part;
+  const double* e_in;  // pair energy of each particle (null: none)
+  double* part;        // block partials: power and energy, largest gradient component
+  unsigned* gpart;
   int nparts;
-  // potential energy of gravity (force_manager.py:450-459)
   float g[3];
   const float* mass;
-  double* e_out;
-  // when set, every kernel returns at once once *stop is set (device-side
-  // stopping tests of the precision form)
-  const int32_t* stop;
 };
-// Stopping state of a FIRE loop decided on the device (routines.py:284-314
-// tests plus a stall test): k_prec_check runs before every update.
+// The same of the precision form, which also tests for a stall.
 struct PrecStop {
   double pe, prev, best_g, best_e, gmax;
   long long best_at, steps;
@@ -715,14 +723,9 @@ struct PrecStopP {
   double pe_tol, pe_diff_tol, force_tol, dN;
   long long max_steps, stall_steps;
 };
-hipError_t launch_fire_power(const FireArgs& a, hipStream_t s);
+hipError_t launch_fire_terms(const FireArgs& a, hipStream_t s);
 hipError_t launch_fire_decide(const FireArgs& a, hipStream_t s);
 hipError_t launch_fire_move(const FireArgs& a, hipStream_t s);
-hipError_t launch_fire_commit(const FireArgs& a, hipStream_t s);
-// max |force| / |torque| component into st->max_grad_bits; gravity energy
-// added into e_out (per particle) when g != 0
-hipError_t launch_fire_grad_max(const FireArgs& a, hipStream_t s);
-hipError_t launch_fire_gravity_energy(const FireArgs& a, hipStream_t s);
 
 // ---- precision form: integer cell + float32 offset (jdem_fire.hip) ----------
 struct PrecArgs {
