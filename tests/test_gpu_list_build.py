@@ -113,3 +113,31 @@ def test_rollout_segments_equal_steps(device, strides):
     _compare_states(fs, B.state_of(sa), "end")
     assert fy.collider.n_build_times == ya.collider.n_build_times
     assert np.array_equal(fy.collider.neighbor_list.cpu().numpy(), ya.collider.neighbor_list.cpu().numpy())
+
+
+@pytest.mark.parametrize("dim,domain,N,phi,edge,cutoff,M,bonds", [
+    (3, "periodic", 1, 0.3, 1.0, 1.2, 4, False),
+    (3, "periodic", 40, 0.6, 1.0, 1.2, 30, False),  # one or two cells per axis
+    (3, "reflect", 1001, 0.5, 0.5, 1.2, 30, True),  # 343 cells, in groups of lanes
+    (2, "periodic", 1500, 4.0, 1.0, 1.5, 64, False),  # more hits than lanes
+    (2, "reflect", 777, 0.8, 1.0, 1.5, 3, False),  # rows cut short
+    (3, "reflect", 131071, 0.4, 1.0, 1.1, 24, False),  # the last size of groups, the first of a lane per sphere
+    (3, "periodic", 131072, 0.4, 1.0, 1.1, 24, False),
+])
+def test_caller_lists_equal_the_oracle(device, dim, domain, N, phi, edge, cutoff, M, bonds):
+    """Lists in the caller's order from a cell list, rows entry by entry."""
+    print(f"[list] caller dim={dim} {domain} N={N} edge={edge}", flush=True)
+    ids = None
+    if bonds:
+        ids = np.full((N, 2), -1, np.int64)
+        ids[:-1, 0], ids[1:, 1] = np.arange(1, N), np.arange(N - 1)
+    st, box = packed(N, dim, seed=N, domain=domain, phi=phi, bonds=ids)
+    mats = [jd.Material.create("elastic", density=1.0, young=1e2, poisson=0.3)]
+    sy = jd.System.create(st.shape, dt=1e-3, domain_type=domain, domain_kw=dict(box_size=box, anchor=np.zeros(dim)),
+                          collider_type="CellList", collider_kw=dict(state=st, cell_size=edge * 1.2),
+                          force_model_type="spring", mat_table=jd.MaterialTable.from_materials(mats))
+    _, _, got, ovf = sy.collider.create_neighbor_list(st, sy, cutoff, M)
+    P = B.params_of(st, sy)
+    want, over = O.neighbor_list_cells(B.state_of(st), P.domain, P.cell_size, P.search_range, np.float32(cutoff), M)
+    assert bool(ovf) == bool(over)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
