@@ -1105,7 +1105,7 @@ int resident_nl_step(jdem_ctx* ctx, jdem_system* sys, int64_t n, jdem_step_stats
     // the gated rebuild chain) repeat with the same arguments every two
     // steps: a chunk of kGraphSteps of them is captured once in a hipGraph
     // on a private stream and replayed, which removes the host's kernel
-    // launches (~27 per step) from the critical path.  Short calls and
+    // launches (8 per step) from the critical path.  Short calls and
     // timed calls (HIP events per kernel) launch one by one.
     constexpr int64_t kGraphSteps = 50;  // even: the ping-pong buffers return to their start
     if (sg->launch_mode == 0 && !ctx->timing && ns - t >= 2 * kGraphSteps) {

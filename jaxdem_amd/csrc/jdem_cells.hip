@@ -915,7 +915,7 @@ __global__ void __launch_bounds__(kBlock) k_nlist_naive(NLBuildT<Real> b) {
 // those within the cutoff appended in candidate order, side by side in the
 // particle's row.  Walked by one lane, 27 pairs of bounds and their candidates
 // are one dependent chain and the rows' stores touch a line each (83 us for
-// 100 k spheres, some 50 here).
+// 100 k spheres, 40 here).
 // G = 32 in 3D (27 cells), 16 in 2D (9).
 template <int D, bool PER, class Real>
 __global__ void __launch_bounds__(kBlock) k_nlist_cells_group(NLBuildT<Real> b) {

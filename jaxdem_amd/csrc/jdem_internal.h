@@ -632,13 +632,10 @@ hipError_t ws_launch_copy_rows(const int32_t* src, int32_t* dst, int64_t n, int 
 // Tangential springs of the step kernel, per wavefront: the 64 work slots
 // of wave w own the region [64 w M, 64 (w + 1) M) of the spring buffer, and
 // slot b's springs (in slot order of its live bits) start at offset W[b].w
-// (an int in the float bits) of that region.  The list rebuild, the entry
-// and the exit keep springs by rank instead ([k N + b], k-th live slot).
+// (an int in the float bits) of that region.  The entry and the exit keep
+// springs by rank instead ([k N + b], k-th live slot).
 // pack: by rank -> per wave (offsets = prefix of the live counts);
-// unpack: per wave -> by rank.  With seg_mode, only wavefronts holding a
-// slot of a system that is rebuilt (mode != SEG_KEEP) are converted; with
-// wpref (the flagged systems' wavefront prefix of k_seg_prefix) the launch
-// walks those wavefronts only.
+// unpack: per wave -> by rank.
 hipError_t ws_launch_pack_springs(int64_t n, int M, int W64, const float4* rank, const uint64_t* live, float4* wave,
                                   float4* W, hipStream_t s);
 hipError_t ws_launch_unpack_springs(int64_t n, int M, int W64, const float4* wave, const uint64_t* live,
