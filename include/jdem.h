@@ -272,8 +272,8 @@ typedef struct jdem_minimize_stats {
  * timing is enabled (jdem_ctx_set_timing).  Step kernels that found a
  * neighbour-list rebuild pending and did no work are counted apart. */
 typedef struct jdem_timing {
-  double step_kernel_ms;   /* fused step kernels that did work          */
-  int64_t step_kernels;
+  double step_kernel_ms;   /* fused step kernels that did work, or the  */
+  int64_t step_kernels;    /* force evaluations of a minimisation       */
   double idle_kernel_ms;   /* step kernels that returned early          */
   int64_t idle_kernels;
   double rebuild_ms;       /* neighbour-list / cell-list rebuilds       */
@@ -299,8 +299,9 @@ const char* jdem_last_error(const jdem_ctx* ctx);
 /* Bytes of scratch the context holds now. */
 int jdem_ctx_scratch_bytes(const jdem_ctx* ctx, size_t* bytes);
 /* Enable (1) or disable (0) HIP-event timing of the kernels that
- * jdem_system_step launches.  Has no counterpart in the reference (JaxDEM
- * times whole jitted calls, benchmarks/run_benchmarks.py:27-51). */
+ * jdem_system_step and the minimisers launch.  Has no counterpart in the
+ * reference (JaxDEM times whole jitted calls,
+ * benchmarks/run_benchmarks.py:27-51). */
 int jdem_ctx_set_timing(jdem_ctx* ctx, int enable);
 /* Synchronise the stream, return the accumulated timing and reset it. */
 int jdem_ctx_get_timing(jdem_ctx* ctx, jdem_timing* out);

@@ -492,7 +492,8 @@ int build_cells(jdem_ctx* ctx, const Real* pos, const Real* rad, int64_t n, int 
 
 // Device words in ctx->flags: [0], [1] rebuild-pending ping-pong, [2] list
 // overflow, [3] displacement flag of the standalone check, [4] rebuild gate
-// and [5] rebuild events of a batch, [6] default-inertia flag of a call.
+// and [5] rebuild events of a batch, [6] default-inertia flag of a call, [7]
+// go word of a batch's rebuild chain, [8] stop word of a minimisation.
 int ensure_flags(jdem_ctx* ctx) {
   ENSURE(ctx, ctx->flags, 64);
   if (!ctx->host_flags) {
@@ -607,7 +608,9 @@ float nl_trigger(const jdem_nlist& L) {
 }
 
 // _check_and_rebuild on its own (neighbor_list.py:58-131).
-int nl_check_and_rebuild(jdem_ctx* ctx, jdem_system* sys, bool* rebuilt) {
+// With stopped, the read also fetches flags[8]; if that word is set nothing is
+// rebuilt and *stopped says so.
+int nl_check_and_rebuild(jdem_ctx* ctx, jdem_system* sys, bool* rebuilt, bool* stopped = nullptr) {
   jdem_nlist& L = sys->nlist;
   const jdem_state& s = sys->state;
   *rebuilt = false;
@@ -619,8 +622,12 @@ int nl_check_and_rebuild(jdem_ctx* ctx, jdem_system* sys, bool* rebuilt) {
     hipLaunchKernelGGL(k_disp_check<float>, dim3(nblocks(s.n)), dim3(kBlock), 0, ctx->stream, s.pos, L.old_pos, s.n, s.dim,
                        nl_trigger(L), (int32_t*)ctx->flags.p + 3);
     HIPCHK(ctx, hipGetLastError());
-    rc = read_flags(ctx, 4);
+    rc = read_flags(ctx, stopped ? 9 : 4);
     if (rc) return rc;
+    if (stopped && ctx->host_flags[8]) {
+      *stopped = true;
+      return JDEM_OK;
+    }
     need = ctx->host_flags[3] != 0;
   }
   if (need) {
@@ -1985,13 +1992,23 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
   h.ls.prev = INFINITY;
   HIPCHK(ctx, hipMemcpyAsync(dev, &h, sizeof(h), hipMemcpyHostToDevice, st));
 
+  const bool listed = sys->collider_kind == JDEM_COLLIDER_NEIGHBOR_LIST && N > 0;
+  bool stopped = false;  // seen by the list's check
+  if (listed) {
+    rc = ensure_flags(ctx);
+    if (rc) return rc;
+    f.stop_word = (int32_t*)ctx->flags.p + 8;
+    HIPCHK(ctx, launch_fill_i32(f.stop_word, 1, 0, st));
+  }
+
   // eval_step (routines.py:228-245) and the next update's decision
   auto eval = [&]() -> int {
     if (sys->collider_kind == JDEM_COLLIDER_NEIGHBOR_LIST) {
       bool rebuilt = false;
-      int r = nl_check_and_rebuild(ctx, sys, &rebuilt);
-      if (r) return r;
+      int r = nl_check_and_rebuild(ctx, sys, &rebuilt, listed ? &stopped : nullptr);
+      if (r || stopped) return r;
     }
+    const int sp = span_begin(ctx, 0, 0);  // counts the evaluations
     StepArgs a = base_args(ctx, sys);
     if (sys->collider_kind == JDEM_COLLIDER_NONE) {
       HIPCHK(ctx, hipMemsetAsync(s.force, 0, 4 * (size_t)N * D, st));
@@ -2010,19 +2027,24 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
     }
     HIPCHK(ctx, launch_fire_terms(f, st));
     HIPCHK(ctx, launch_fire_decide(f, st));
+    span_end(ctx, sp);
     return JDEM_OK;
   };
 
   rc = eval();
   if (rc) return rc;
-  // Iterations run in chunks between two reads of the loop's state, each a
-  // quarter of the steps so far (4 to 32), so that few are launched past a stop.
+  // Iterations run in chunks between two reads of the loop's state: 1, 1, 2, 4
+  // and then a quarter of the steps so far, up to 32, so that few are launched
+  // past a stop (a call that stops after one step, 262 k spheres: 1061 us with
+  // a first chunk of four).  With a list every iteration sees the stop itself
+  // (1558 us for the same call when it did not).
   for (int64_t done = 0;;) {
     HIPCHK(ctx, hipMemcpyAsync(&h, dev, sizeof(h), hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
     if (h.ls.stop) break;
-    const int64_t todo = std::min(max_steps - done, std::min<int64_t>(32, std::max<int64_t>(4, done / 4)));
-    for (int64_t k = 0; k < todo; ++k) {
+    const int64_t first = std::min<int64_t>(4, std::max<int64_t>(1, done));
+    const int64_t todo = std::min(max_steps - done, std::min<int64_t>(32, std::max<int64_t>(first, done / 4)));
+    for (int64_t k = 0; (listed || k < todo) && !stopped; ++k) {
       HIPCHK(ctx, launch_fire_move(f, st));
       rc = eval();
       if (rc) return rc;

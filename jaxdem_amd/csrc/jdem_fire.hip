@@ -15,7 +15,11 @@
 // recomputes the forces of the final positions.  So the host reads the loop's
 // state once per chunk of iterations: with a read per iteration and a kernel
 // for each of these terms an iteration of 16 k spheres was 21 launches and
-// 130 us, bounded by them; now 10 and 66 us.
+// 130 us, bounded by them; now 10 and 66 us.  The chunks grow with the steps
+// done (1, 1, 2, 4, then a quarter of them up to 32), so the evaluations past a
+// stop stay below half of those needed.  A neighbour list is checked by the
+// host before every evaluation anyway; the stop word comes with that read, and
+// nothing is launched past a stop.
 // Every float32 expression follows the reference's operation order, so
 // positions match the float32 oracle bit for bit while the power decisions
 // agree.
@@ -216,6 +220,7 @@ __global__ void __launch_bounds__(kBlock) k_fire_decide(FireArgs a) {
   const bool conv_rel = fabs(pe - ls.prev) / denom < a.stop.pe_diff_tol;
   if (ls.steps >= a.stop.max_steps || conv_pe || conv_rel || gmax <= a.stop.force_tol) {
     ls.stop = 1;
+    if (a.stop_word) *a.stop_word = 1;
     return;
   }
   ls.prev = pe;

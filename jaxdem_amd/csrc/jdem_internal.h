@@ -694,6 +694,7 @@ struct FireArgs {
   FireP p;
   FireDev* st;
   FireStop* ls;
+  int32_t* stop_word;  // set with ls->stop (null: none)
   FireStopP stop;
   float* force;
   const float* torque;
