@@ -2217,10 +2217,11 @@ int jdem_precise_minimize(jdem_ctx* ctx, jdem_precise* p, const jdem_fire* fire,
   constexpr int64_t kChunk = 64;
   int64_t steps = 0;
   do {
-    const int64_t todo = std::min(kChunk, max_steps - steps + 1);
+    const int64_t left = max_steps - steps;  // max_steps may be the type's largest value
+    const int64_t todo = left < kChunk ? left + 1 : kChunk;
     for (int64_t k = 0; k < todo; ++k) {
       HIPCHK(ctx, launch_prec_update(a, &dev->ps, pp, fp, st));
-      if (k + 1 < todo || steps + todo <= max_steps) {
+      if (k + 1 < todo || todo <= left) {
         rc = eval(nullptr);
         if (rc) return rc;
       }

@@ -71,3 +71,22 @@ def test_small_systems_against_float64(device, dim, N, phi, skin):
     assert abs(r["pe"] * N - e) <= 1e-5 * max(e, 1e-3)
     assert np.abs(r["virial"] - W).max() <= 1e-5 * max(np.abs(W).max(), 1e-3)
     assert r["max_grad"] == np.abs(r["force"].cpu().numpy()).max()
+
+
+@pytest.mark.parametrize("skin", [0.0, 0.05])
+@pytest.mark.parametrize("max_steps", [0, 63, 64, 65, 2**63 - 2, 2**63 - 1])
+def test_step_limits(device, max_steps, skin):
+    """A limit at the edges of the loop's chunks, and none at all: the largest
+    integers that the argument holds (the loop stops by its energy test)."""
+    print(f"[precision] max_steps={max_steps} skin={skin}", flush=True)
+    rng = np.random.Generator(np.random.PCG64(2))
+    rad = np.where(np.arange(200) % 2 == 0, 0.5, 0.7)
+    kw = dict(pe_tol=0.0, skin=skin, device=device)
+    p, box = rng.uniform(0.0, 6.5, (200, 3)), np.full(3, 6.5)
+    if max_steps < 100:
+        r = PR.minimize_precise(p, rad, box, max_steps=max_steps, pe_diff_tol=-1.0, **kw)
+        assert r["steps"] == max_steps
+        return
+    r = PR.minimize_precise(p, rad, box, max_steps=max_steps, pe_diff_tol=1e-3, **kw)
+    want = PR.minimize_precise(p, rad, box, max_steps=5000, pe_diff_tol=1e-3, **kw)
+    assert 0 < r["steps"] == want["steps"] < 5000 and np.array_equal(r["pos"], want["pos"])
