@@ -313,14 +313,15 @@ __global__ void __launch_bounds__(kBlock) k_prec_load(PrecArgs a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   float r = 0.0f;
   if (i < a.n) {
-    r = a.rad[i];
-    a.S[0][i] = make_float4(a.off[D * i], a.off[D * i + 1], D == 3 ? a.off[D * i + 2] : 0.0f, r);
+    const float ri = a.rad[i];
+    r = ri > 0.0f ? ri : 0.0f;  // -0 and less would order above every radius below
+    a.S[0][i] = make_float4(a.off[D * i], a.off[D * i + 1], D == 3 ? a.off[D * i + 2] : 0.0f, ri);
     a.V[0][i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     a.C[0][i] = make_int4(a.cidx[D * i], a.cidx[D * i + 1], D == 3 ? a.cidx[D * i + 2] : 0, (int)i);
   }
   for (int off = 32; off > 0; off >>= 1) r = fmaxf(r, __shfl_xor(r, off));
-  // radii are not negative, so their bits order like the values; most waves
-  // find the maximum already there
+  // not negative, so the bits order like the values; most waves find the
+  // maximum already there
   if ((threadIdx.x & 63) == 0 && __float_as_uint(r) > *a.rmax_bits) atomicMax(a.rmax_bits, __float_as_uint(r));
 }
 

@@ -90,3 +90,19 @@ def test_step_limits(device, max_steps, skin):
     r = PR.minimize_precise(p, rad, box, max_steps=max_steps, pe_diff_tol=1e-3, **kw)
     want = PR.minimize_precise(p, rad, box, max_steps=5000, pe_diff_tol=1e-3, **kw)
     assert 0 < r["steps"] == want["steps"] < 5000 and np.array_equal(r["pos"], want["pos"])
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_points_among_spheres(device, dim):
+    """A wavefront of points whose radius is minus zero, inside larger
+    spheres: the list finds every partner that the stencil finds."""
+    print(f"[precision] points dim={dim}", flush=True)
+    rng = np.random.Generator(np.random.PCG64(dim))
+    rad = np.concatenate([np.full(64, -0.0), rng.uniform(0.4, 0.6, 136)])
+    box = np.full(dim, 12.0 if dim == 2 else 6.0)
+    pos = rng.uniform(0.0, 1.0, (200, dim)) * box
+    kw = dict(max_steps=0, device=device, max_neighbors=200)
+    r = PR.minimize_precise(pos, rad, box, skin=0.05, **kw)
+    F, e, _ = forces64(r["pos"], rad.astype(np.float32).astype(np.float64), box)
+    assert np.abs(r["force"].cpu().numpy() - F).max() <= 1e-6 * 100  # as for the small systems above
+    assert np.abs(F[:64]).max() > 0.01 and abs(r["pe"] * 200 - e) <= 1e-5 * e
