@@ -657,6 +657,76 @@ JD void end_row(const NLW& a, int64_t b, bool active, int count) {
 // slot are contiguous; later slots go straight to memory.
 constexpr int kRowLds = 16;
 
+// The neighbours of the particle self, one lane's walk: put(t, k) takes the
+// t-th, in candidate order.  Returns how many there are.
+template <int D, bool PER, class Put>
+JD int lane_row(const float4* __restrict__ P4, const int32_t* __restrict__ orig, int64_t self, uint32_t key,
+                const GridP& grid, const DomP& dom, float cutoff_sq, const int32_t* __restrict__ starts,
+                const int32_t* __restrict__ bond_id, int bond_w, bool chk_bond, Put&& put) {
+  const Vec<D> xi = xyz<D>(P4[self]);
+  const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
+  int c0, c1, cf;
+  if (D == 3) {
+    cf = (int)(key % (uint32_t)d2);
+    const uint32_t r = key / (uint32_t)d2;
+    c1 = (int)(r % (uint32_t)d1);
+    c0 = (int)(r / (uint32_t)d1);
+  } else {
+    cf = (int)(key % (uint32_t)d1);
+    c0 = (int)(key / (uint32_t)d1);
+    c1 = 0;
+  }
+  const int sr = grid.sr;
+  const int dF = (D == 3) ? d2 : d1;
+  int r0a, r0b, r1a, r1b;
+  stencil_runs(PER, cf, sr, dF, r0a, r0b, r1a, r1b);
+  const int hi0 = PER ? min(sr, d0 - sr - 1) : sr;
+  const int lo1 = (D == 3) ? -sr : 0;
+  const int hi1 = (D == 3) ? (PER ? min(sr, d1 - sr - 1) : sr) : 0;
+  const int64_t ib = chk_bond ? (int64_t)orig[self] : 0;
+  int count = 0;
+  for (int ox = -sr; ox <= hi0; ++ox) {
+    const int cx = stencil_cell(PER, c0, ox, d0);
+    if (cx < 0) continue;
+    for (int oy = lo1; oy <= hi1; ++oy) {
+      int64_t base;
+      if (D == 3) {
+        const int cy = stencil_cell(PER, c1, oy, d1);
+        if (cy < 0) continue;
+        base = (int64_t)(cx * d1 + cy) * d2;
+      } else {
+        base = (int64_t)cx * d1;
+      }
+      // both runs' bounds are loaded before either is walked
+      const int k0 = starts[base + r0a], k0e = starts[base + r0b + 1];
+      const int k1 = (r1b >= r1a) ? starts[base + r1a] : 0;
+      const int k1e = (r1b >= r1a) ? starts[base + r1b + 1] : 0;
+#pragma unroll
+      for (int run = 0; run < 2; ++run) {
+        const int kb = run ? k1 : k0, ke = run ? k1e : k0e;
+        // candidates in groups of four, loaded back to back
+        for (int kg = kb; kg < ke; kg += 4) {
+          float4 pk[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) pk[u] = (kg + u < ke) ? P4[kg + u] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int k = kg + u;
+            if (k >= ke) break;
+            if (k == self) continue;
+            const float dsq = dist_sq<PER>(xi, xyz<D>(pk[u]), dom);
+            if (!(dsq <= cutoff_sq)) continue;
+            if (chk_bond && bonded_o(bond_id, bond_w, ib, orig[k])) continue;
+            put(count, k);
+            ++count;
+          }
+        }
+      }
+    }
+  }
+  return count;
+}
+
 template <int D, bool PER>
 __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
   __shared__ int32_t rows[kRowLds][kBlock];
@@ -667,76 +737,15 @@ __global__ void __launch_bounds__(kBlock) k_nlist_work(NLW a) {
   __syncthreads();
   const bool active = b < a.n;
   int count = 0;
-  if (active) {
-    const GridP& grid = a.grid;
-    const uint32_t key = a.skeys[b];
-    const Vec<D> xi = xyz<D>(a.P4[b]);
-    const int d0 = grid.dims[0], d1 = grid.dims[1], d2 = (D == 3) ? grid.dims[2] : 1;
-    int c0, c1, cf;
-    if (D == 3) {
-      cf = (int)(key % (uint32_t)d2);
-      const uint32_t r = key / (uint32_t)d2;
-      c1 = (int)(r % (uint32_t)d1);
-      c0 = (int)(r / (uint32_t)d1);
-    } else {
-      cf = (int)(key % (uint32_t)d1);
-      c0 = (int)(key / (uint32_t)d1);
-      c1 = 0;
-    }
-    const int sr = grid.sr;
-    const int dF = (D == 3) ? d2 : d1;
-    int r0a, r0b, r1a, r1b;
-    stencil_runs(PER, cf, sr, dF, r0a, r0b, r1a, r1b);
-    const int hi0 = PER ? min(sr, d0 - sr - 1) : sr;
-    const int lo1 = (D == 3) ? -sr : 0;
-    const int hi1 = (D == 3) ? (PER ? min(sr, d1 - sr - 1) : sr) : 0;
-    const bool chk_bond = (!a.isb) && a.bond_w > 0;
-    const int64_t ib = chk_bond ? (int64_t)a.orig[b] : 0;
-    const int32_t* __restrict__ starts = a.starts;
-    for (int ox = -sr; ox <= hi0; ++ox) {
-      const int cx = stencil_cell(PER, c0, ox, d0);
-      if (cx < 0) continue;
-      for (int oy = lo1; oy <= hi1; ++oy) {
-        int64_t base;
-        if (D == 3) {
-          const int cy = stencil_cell(PER, c1, oy, d1);
-          if (cy < 0) continue;
-          base = (int64_t)(cx * d1 + cy) * d2;
-        } else {
-          base = (int64_t)cx * d1;
-        }
-        // both runs' bounds are loaded before either is walked
-        const int k0 = starts[base + r0a], k0e = starts[base + r0b + 1];
-        const int k1 = (r1b >= r1a) ? starts[base + r1a] : 0;
-        const int k1e = (r1b >= r1a) ? starts[base + r1b + 1] : 0;
-#pragma unroll
-        for (int run = 0; run < 2; ++run) {
-          const int kb = run ? k1 : k0, ke = run ? k1e : k0e;
-          // candidates in groups of four, loaded back to back
-          for (int kg = kb; kg < ke; kg += 4) {
-            float4 pk[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pk[u] = (kg + u < ke) ? a.P4[kg + u] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int k = kg + u;
-              if (k >= ke) break;
-              if (k == b) continue;
-              const float dsq = dist_sq<PER>(xi, xyz<D>(pk[u]), a.dom);
-              if (!(dsq <= a.cutoff_sq)) continue;
-              if (chk_bond && bonded_o(a.bond_id, a.bond_w, ib, a.orig[k])) continue;
-              if (count < kRowLds)
-                rows[count][tid] = k;
-              else if (count < a.M)
-                a.nl[(int64_t)count * a.n + b] = k;
-              ++count;
-            }
-          }
-        }
-      }
-    }
-    atomicMax(&row_max, min(count, kRowLds));
-  }
+  if (active)
+    count = lane_row<D, PER>(a.P4, a.orig, b, a.skeys[b], a.grid, a.dom, a.cutoff_sq, a.starts, a.bond_id, a.bond_w,
+                             (!a.isb) && a.bond_w > 0, [&](int t, int k) {
+                               if (t < kRowLds)
+                                 rows[t][tid] = k;
+                               else if (t < a.M)
+                                 a.nl[(int64_t)t * a.n + b] = k;
+                             });
+  if (active) atomicMax(&row_max, min(count, kRowLds));
   __syncthreads();
   const int c = min(count, a.M);
   if (active) {
@@ -991,38 +1000,146 @@ k_nlist_group(NLW a) {
       [&](int) { return make_float4(0.f, 0.f, 0.f, 0.f); });
 }
 
+// A batch rebuild of many particles, one lane each: a wavefront builds the rows
+// of one region of 64 slots and moves their fields and springs.
+template <int D, int MW>
+JD void lane_regions(const RB& r, int32_t (*rows)[64 * nlist_group<D>()]) {
+  constexpr int G = nlist_group<D>();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t n = r.n, nreg = r.wpref[r.n_seg];
+  const int64_t w0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * G + (tid >> 6);
+  for (int64_t reg = w0; reg < nreg; reg += (int64_t)gridDim.x * G) {  // uniform over the wavefront
+    const int fs = seg_of_compact(r.wpref, r.n_seg, reg);
+    const int region = (int)((r.offsets[fs] >> 6) + (reg - r.wpref[fs])) * 64, b = region + lane;
+    const int sg = b < n ? r.seg[b] : -1;
+    const bool active = b < n && r.seg_mode[sg] != SEG_KEEP;
+    const int k = active ? (int)(r.cpref[sg] + (b - r.offsets[sg])) : 0;  // compact index
+    int count = 0;
+    if (r.M > 0) {
+      const int s_last = __builtin_amdgcn_readfirstlane(r.seg[min((int64_t)region + 63, n - 1)]);
+      for (int s = __builtin_amdgcn_readfirstlane(r.seg[region]); s <= s_last; ++s) {
+        const SegP& sp = r.segp[s];
+        const int64_t c0 = r.ccref[s];
+        auto row = [&](auto per) {
+          return lane_row<D, decltype(per)::value>(r.tP, r.torig, k, r.sk[k] - (uint32_t)c0, sp.grid, sp.dom,
+                                                   sp.cutoff_sq, r.starts + c0, r.bond_id, r.bond_w,
+                                                   (!r.isb) && r.bond_w > 0, [&](int t, int j) {
+                                                     const int32_t slot = (int32_t)(j + (b - k));
+                                                     if (t < kRowLds)
+                                                       rows[t][tid] = slot;
+                                                     else if (t < r.M)
+                                                       r.nl[(int64_t)t * n + b] = slot;
+                                                   });
+        };
+        if (active && sg == s)
+          count = sp.dom.kind == JDEM_DOMAIN_PERIODIC ? row(std::true_type{}) : row(std::false_type{});
+      }
+    }
+    const int c = min(count, r.M);
+    if (active) {
+      for (int t = 0; t < min(c, kRowLds); ++t) r.nl[(int64_t)t * n + b] = rows[t][tid];
+      if (count < r.M) r.nl[(int64_t)count * n + b] = -1;
+      if (count > r.M) atomicOr(r.overflow, 1);
+      const float4 x = r.tP[k], v = r.tV[k];
+      r.old4[b] = x;  // build position
+      r.P[b] = D == 2 ? make_float4(x.x, x.y, x.x, x.w) : x;  // and in the 2D records' free lanes
+      r.V[b] = D == 2 ? make_float4(v.x, v.y, x.y, v.w) : v;
+      r.Q[b] = r.tQ[k];
+      r.I[b] = r.tI[k];
+      r.orig[b] = r.torig[k];
+      if (!r.live) r.W[b] = r.tW[k];
+    }
+    if (!r.live) continue;
+    const int n_old = active ? r.tlive[k] : 0;
+    int n_kept = 0;
+    if (b < n && !active)
+      for (int w = 0; w < r.W64; ++w) n_kept += __popcll(r.live[(int64_t)w * n + b]);
+    // each old spring's slot in the new row (as group_springs)
+    auto new_slot = [&](int q) {
+      const int32_t o = r.tnl[(int64_t)q * n + k];
+      return o < 0 ? -1 : find_in_row(r.inv[o], c, [&](int t) { return t < kRowLds ? rows[t][tid] : r.nl[(int64_t)t * n + b]; });
+    };
+    uint64_t out[MW];
+#pragma unroll
+    for (int w = 0; w < MW; ++w) out[w] = 0ull;
+    for (int q = 0; q < n_old; ++q) {
+      const int t = new_slot(q);
+#pragma unroll
+      for (int w = 0; w < MW; ++w) out[w] |= t >= 0 && (t >> 6) == w ? 1ull << (t & 63) : 0ull;
+    }
+    int cnt = n_kept;
+#pragma unroll
+    for (int w = 0; w < MW; ++w) cnt += __popcll(out[w]);
+    const int off = wave_exclusive_scan(cnt, lane);
+    if (b >= n) continue;
+    const int64_t wbase = (int64_t)region * r.M + off;
+    if (!active) {
+      r.W[b].w = __int_as_float(off);
+      for (int q = 0; q < n_kept; ++q) r.xi[wbase + q] = r.keep_xi[(int64_t)q * n + b];
+      continue;
+    }
+    const float4 w4 = r.tW[k];
+    r.W[b] = make_float4(w4.x, w4.y, w4.z, __int_as_float(off));
+    for (int q = 0; q < n_old; ++q) {
+      const int t = new_slot(q);
+      if (t < 0) continue;
+      const int rank = MW == 1 ? __popcll(out[0] & ((1ull << t) - 1ull))
+                               : rank_below(out[0], out[MW > 1 ? 1 : 0], out[MW > 2 ? 2 : 0], out[MW > 3 ? 3 : 0], t);
+      r.xi[wbase + rank] = r.txi[(int64_t)q * n + k];
+    }
+#pragma unroll
+    for (int w = 0; w < MW; ++w)
+      if (w < r.W64) r.live[(int64_t)w * n + b] = out[w];
+  }
+}
+
+// From this many particles to rebuild at once, groups of lanes would only add
+// instructions.  A rebuild of all systems of a batch, group / lane, us (the
+// whole chain): disks of like size with springs 70 / 81 at 120 k, 99 / 86 at
+// 250 k, 184 / 104 at 500 k, 388 / 215 at 10^6; spheres 126 / 155, 217 / 165,
+// 454 / 223, 938 / 455; log-normal spheres without springs 141 / 272,
+// 238 / 275, 437 / 337, 871 / 644.  Below 10^5 groups take half the time.
+constexpr int64_t kRebuildLane = 300000;
+
 // The flagged systems of a batch, from the staged particles: rows, springs
 // and the particles' fields in their new slots, over the wavefronts that hold
 // a flagged system (one shared by two of them is written twice, alike).
-// With k_nlist_work's lane per particle in its place (119 us a rebuild of eight
-// systems of 1 k to 150 k polydisperse spheres, 58 us now) a rebuild of one
-// system left most of the chip idle; all 10^6 disks of 256 systems at once, the
-// first build, take longer with groups, 87 -> 236 us, which the passes saved in
-// every later step outweigh.
+// Groups of lanes or, from kRebuildLane particles on, a lane each: with lanes a
+// rebuild of one of eight systems of 1 k to 150 k polydisperse spheres left
+// most of the chip idle (this kernel 119 us, 58 with groups).
 template <int D, int MW>
 __global__ void __launch_bounds__(64 * nlist_group<D>()) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_rebuild_rows(RB r) {
   if (*r.go == 0) return;
   constexpr int G = nlist_group<D>();
-  __shared__ RowLds lds;
+  union Lds {
+    RowLds group;
+    int32_t lanes[kRowLds][64 * G];
+  };
+  __shared__ Lds both;
+  if (r.cpref[r.n_seg] >= kRebuildLane) {
+    lane_regions<D, MW>(r, both.lanes);
+    return;
+  }
+  RowLds& lds = both.group;
   const int tid = threadIdx.x, p = tid / G, l = tid & (G - 1), lane = tid & 63;
   const int64_t n = r.n, nreg = r.wpref[r.n_seg];
   for (int64_t reg = xcd_tile(blockIdx.x, gridDim.x); reg < nreg; reg += gridDim.x) {
     const int fs = seg_of_compact(r.wpref, r.n_seg, reg);
-    const int64_t region = ((r.offsets[fs] >> 6) + (reg - r.wpref[fs])) * 64, b = region + p;
+    const int region = (int)((r.offsets[fs] >> 6) + (reg - r.wpref[fs])) * 64, b = region + p;
     const int sg = b < n ? r.seg[b] : -1;
     const int mode = b < n ? r.seg_mode[sg] : SEG_FRESH;
     const bool active = b < n && mode != SEG_KEEP;
-    const int64_t k = active ? r.cpref[sg] + (b - r.offsets[sg]) : 0;  // compact index
+    const int k = active ? (int)(r.cpref[sg] + (b - r.offsets[sg])) : 0;  // compact index
     int count = 0;
     if (r.M > 0) {
       // system by system (mostly one), so that the grid and domain are uniform
-      const int s_last = __builtin_amdgcn_readfirstlane(r.seg[min(region + 63, n - 1)]);
+      const int s_last = __builtin_amdgcn_readfirstlane(r.seg[min((int64_t)region + 63, n - 1)]);
       for (int s = __builtin_amdgcn_readfirstlane(r.seg[region]); s <= s_last; ++s) {
         const SegP& sp = r.segp[s];
         const int64_t c0 = r.ccref[s];
         auto row = [&](auto per) {
-          return group_row<D, decltype(per)::value>(lds, r.tP, r.torig, (int)k, (int)(b - k), r.sk[k] - (uint32_t)c0,
+          return group_row<D, decltype(per)::value>(lds, r.tP, r.torig, k, b - k, r.sk[k] - (uint32_t)c0,
                                                     sp.grid, sp.dom, sp.cutoff_sq, r.starts + c0, r.bond_id, r.bond_w,
                                                     (!r.isb) && r.bond_w > 0, r.nl, n, r.M, b);
         };
@@ -1039,7 +1156,7 @@ k_rebuild_rows(RB r) {
       if (count > r.M) atomicOr(r.overflow, 1);
     }
     {  // the fields, one kind per wavefront
-      const int64_t bw = region + lane;
+      const int bw = region + lane;
       if (lds.row_cnt[lane] >= 0) {
         const int sw = r.seg[bw];
         const int64_t kw = r.cpref[sw] + (bw - r.offsets[sw]);
@@ -1085,7 +1202,7 @@ k_rebuild_rows(RB r) {
           },
           [&](int q) { return r.txi[(int64_t)q * n + k]; },
           [&](int ln, int off) {
-            const int64_t bw = region + ln;
+            const int bw = region + ln;
             if (bw >= n) return;
             if (lds.row_cnt[ln] >= 0) {
               const int sw = r.seg[bw];
