@@ -445,7 +445,9 @@ typedef struct jdem_batch {
   const float* cutoff;
   const float* skin;
   int32_t tile_width; /* particles per workgroup of the step kernel: 256
-                       * (also for 0) or 128 */
+                       * (also for 0) or 128.  In 2D, and in 3D from 80000
+                       * particles on; below that the four waves of a
+                       * workgroup share 64 spheres, whatever stands here. */
   int32_t spec_min_gap; /* launch mode 2: see above; 0 = 2 steps */
 } jdem_batch;
 

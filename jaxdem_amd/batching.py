@@ -85,6 +85,11 @@ def _shift(t: torch.Tensor, off: int) -> torch.Tensor:
     return torch.where(t >= 0, t + off, t)
 
 
+# Below this many spheres the 3D step kernel shares 64 of them among the four
+# waves of a workgroup and has no tile width (kWsSplit of csrc/jdem_resident.hip).
+SPLIT_SPHERES = 80000
+
+
 @dataclass
 class Batch:
     """A packed batch; ``systems`` keeps each system's own parameters."""
@@ -100,7 +105,8 @@ class Batch:
     # gated chain after every step with captured graphs for long calls, 1 the
     # chain step by step, 2 speculative chunks with one host read per chunk
     launch_mode: int = 0
-    # particles per workgroup of the step kernel (256 or 128)
+    # particles per workgroup of the step kernel (256 or 128); without effect
+    # on 3D batches of fewer than SPLIT_SPHERES
     tile_width: int = 256
     # launch mode 2 runs the rest of a call as mode 1 once two rebuilds in a
     # row come this many steps or fewer apart (0: 2)
@@ -414,11 +420,17 @@ def tune_launch(batch: Batch, tiles: Sequence[int] = (256, 128), modes: Sequence
                 probe_steps: int = 200, warm_steps: int = 20) -> tuple:
     """Tile width of the step kernel, then launch mode (how rebuild decisions
     reach the kernels), probed on ``batch`` itself: neither changes a bit of
-    the result, so the batch is not repacked.  Sets the best values on
-    ``batch`` and returns ({"tile_width", "launch_mode"}, [(knob, value,
+    the result, so the batch is not repacked.  A 3D batch of fewer than
+    SPLIT_SPHERES keeps its tile width, which the kernel does not use there.
+    Sets the best values on ``batch`` and returns ({"tile_width", "launch_mode"}, [(knob, value,
     particle-steps/s, rebuilds), ...])."""
     table = []
-    for knob, values in (("tile_width", tiles), ("launch_mode", modes)):
+    knobs = [("tile_width", tiles), ("launch_mode", modes)]
+    if batch.state.dim == 3 and batch.n_particles < SPLIT_SPHERES:
+        knobs = knobs[1:]
+        if batch.tile_width not in tiles:
+            batch.tile_width = int(tiles[0])
+    for knob, values in knobs:
         best_v, best_r = getattr(batch, knob), -1.0
         for v in values:
             setattr(batch, knob, int(v))
