@@ -86,34 +86,20 @@ constexpr int RS_ITEMS = 16;
 constexpr int RS_TILE = kBlock * RS_ITEMS;
 constexpr int RS_WAVES = kBlock / 64;
 
-// n_dev (when set) holds the key count on the device, n is then an upper
-// bound that sized the launch; gate (when set) skips the sort while 0.
 __global__ void __launch_bounds__(kBlock) k_radix_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
-                                                        uint32_t* __restrict__ hist, int ntiles,
-                                                        const int64_t* __restrict__ n_dev,
-                                                        const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  if (n_dev) n = *n_dev;
+                                                        uint32_t* __restrict__ hist, int ntiles) {
   __shared__ uint32_t bins[256];
   const int tid = threadIdx.x;
-  // one tile per workgroup, or (a grid smaller than the tiles) several in turn
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t base = (int64_t)tile * RS_TILE;
-    if (base >= n) {  // a tile past the keys counts nothing
-      hist[(int64_t)tid * ntiles + tile] = 0u;
-      continue;
-    }
-    bins[tid] = 0;
-    __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+  bins[tid] = 0;
+  __syncthreads();
 #pragma unroll 4
-    for (int it = 0; it < RS_ITEMS; ++it) {
-      int64_t idx = base + (int64_t)it * kBlock + tid;
-      if (idx < n) atomicAdd(&bins[(keys[idx] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[(int64_t)tid * ntiles + tile] = bins[tid];
-    __syncthreads();  // the next tile clears bins
+  for (int it = 0; it < RS_ITEMS; ++it) {
+    int64_t idx = base + (int64_t)it * kBlock + tid;
+    if (idx < n) atomicAdd(&bins[(keys[idx] >> shift) & 255u], 1u);
   }
+  __syncthreads();
+  hist[(int64_t)tid * ntiles + blockIdx.x] = bins[tid];
 }
 
 // Parallel exclusive scan of `total` uint32 values in three launches:
@@ -172,9 +158,7 @@ __global__ void __launch_bounds__(1024) k_scan_sums(uint32_t* __restrict__ sums,
 }
 
 __global__ void __launch_bounds__(kBlock) k_scan_apply(uint32_t* __restrict__ data, int64_t total,
-                                                        const uint32_t* __restrict__ sums,
-                                                        const int32_t* __restrict__ gate = nullptr) {
-  if (gate && *gate == 0) return;
+                                                        const uint32_t* __restrict__ sums) {
   __shared__ uint32_t tile[SC_CHUNK];
   __shared__ uint32_t tsum[kBlock];
   const int tid = threadIdx.x;
@@ -214,9 +198,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(uint32_t* __restrict__ da
 
 // Exclusive scan of `total` uint32 values in one block of 1024 threads
 // (kept for totals small enough that one launch is cheaper).
-__global__ void __launch_bounds__(1024) k_scan_exclusive(uint32_t* __restrict__ data, int64_t total,
-                                                          const int32_t* __restrict__ gate = nullptr) {
-  if (gate && *gate == 0) return;
+__global__ void __launch_bounds__(1024) k_scan_exclusive(uint32_t* __restrict__ data, int64_t total) {
   __shared__ uint32_t part[1024];
   const int tid = threadIdx.x;
   const int64_t chunk = (total + 1023) / 1024;
@@ -245,20 +227,15 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(const uint32_t* __rest
                                                            const int32_t* __restrict__ vin,
                                                            uint32_t* __restrict__ kout, int32_t* __restrict__ vout,
                                                            int64_t n, int shift, const uint32_t* __restrict__ offs,
-                                                           int ntiles, const int64_t* __restrict__ n_dev,
-                                                           const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
-  if (n_dev) n = *n_dev;
+                                                           int ntiles) {
   __shared__ uint32_t run[256];
   __shared__ uint32_t wcnt[RS_WAVES][256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const uint64_t lt = (1ull << lane) - 1ull;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-  const int64_t base = (int64_t)tile * RS_TILE;
-  if (base >= n) break;  // tiles past the keys move nothing (and later tiles lie further past)
-  run[tid] = offs[(int64_t)tid * ntiles + tile];
+  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+  run[tid] = offs[(int64_t)tid * ntiles + blockIdx.x];
   for (int it = 0; it < RS_ITEMS; ++it) {
 #pragma unroll
     for (int w = 0; w < RS_WAVES; ++w) wcnt[w][tid] = 0;
@@ -293,7 +270,6 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(const uint32_t* __rest
     run[tid] += add;
     __syncthreads();
   }
-  }
 }
 
 size_t radix_hist_words(int64_t n) {
@@ -304,7 +280,7 @@ size_t radix_hist_words(int64_t n) {
 }
 
 hipError_t radix_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n, int nbits, uint32_t** keys_out,
-                           int32_t** vals_out, hipStream_t s, const int64_t* n_dev, const int32_t* gate) {
+                           int32_t** vals_out, hipStream_t s) {
   const int ntiles = (int)((n + RS_TILE - 1) / RS_TILE);
   const int64_t total = (int64_t)ntiles * 256;
   const int nchunks = (int)((total + SC_CHUNK - 1) / SC_CHUNK);
@@ -319,20 +295,17 @@ hipError_t radix_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t 
   for (int p = 0; p < passes; ++p) {
     const int shift = 8 * p;
     if (n > 0) {
-      // with the count on the device the launch is capped and the tiles are
-      // walked in turn: an idle (gated or empty) sort dispatches few workgroups
-      const int grid = n_dev ? std::min(ntiles, kCappedGrid) : ntiles;
-      hipLaunchKernelGGL(k_radix_hist, dim3(grid), dim3(kBlock), 0, s, kcur, n, shift, hist, ntiles, n_dev, gate);
+      hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(kBlock), 0, s, kcur, n, shift, hist, ntiles);
       if (nchunks <= 1) {
-        hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, hist, total, gate);
+        hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, hist, total);
       } else {
         uint32_t* sums = hist + total;
-        hipLaunchKernelGGL(k_scan_totals, dim3(nchunks), dim3(kBlock), 0, s, hist, total, sums, gate);
-        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nchunks, gate);
-        hipLaunchKernelGGL(k_scan_apply, dim3(nchunks), dim3(kBlock), 0, s, hist, total, sums, gate);
+        hipLaunchKernelGGL(k_scan_totals, dim3(nchunks), dim3(kBlock), 0, s, hist, total, sums);
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nchunks);
+        hipLaunchKernelGGL(k_scan_apply, dim3(nchunks), dim3(kBlock), 0, s, hist, total, sums);
       }
-      hipLaunchKernelGGL(k_radix_scatter, dim3(grid), dim3(kBlock), 0, s, kcur, vcur, kb[out], vb[out], n, shift,
-                         hist, ntiles, n_dev, gate);
+      hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(kBlock), 0, s, kcur, vcur, kb[out], vb[out], n, shift,
+                         hist, ntiles);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -346,7 +319,7 @@ hipError_t radix_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t 
 }
 
 hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int nbits, uint32_t** keys_out,
-                            int32_t** vals_out, hipStream_t s, const int64_t* n_dev, const int32_t* gate) {
+                            int32_t** vals_out, hipStream_t s) {
   const size_t nn = (size_t)(n > 0 ? n : 1);
   if (!ensure(ctx, ctx->keys[0], sizeof(uint32_t) * nn) || !ensure(ctx, ctx->keys[1], sizeof(uint32_t) * nn) ||
       !ensure(ctx, ctx->vals[0], sizeof(int32_t) * nn) || !ensure(ctx, ctx->vals[1], sizeof(int32_t) * nn) ||
@@ -359,7 +332,7 @@ hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, i
   sb.v1 = (int32_t*)ctx->vals[1].p;
   sb.hist = (uint32_t*)ctx->hist.p;
   sb.cur = nullptr;
-  return radix_sort_bufs(sb, keys_in, n, nbits, keys_out, vals_out, s, n_dev, gate);
+  return radix_sort_bufs(sb, keys_in, n, nbits, keys_out, vals_out, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -378,9 +351,7 @@ hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, i
 // were ten (45 -> 25 us of a 100 k-particle cell-list step).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kBlock) k_cs_count(const uint32_t* __restrict__ keys, int64_t n,
-                                                      int32_t* __restrict__ cnt, int32_t* __restrict__ arr,
-                                                      const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                      int32_t* __restrict__ cnt, int32_t* __restrict__ arr) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   arr[i] = atomicAdd(&cnt[keys[i]], 1);
@@ -461,9 +432,7 @@ __global__ void __launch_bounds__(kBlock) k_cs_scan(int32_t* __restrict__ cnt, i
 
 __global__ void __launch_bounds__(kBlock) k_cs_place(const uint32_t* __restrict__ keys, int64_t n,
                                                       const int32_t* __restrict__ starts,
-                                                      const int32_t* __restrict__ arr, uint2* __restrict__ pairs,
-                                                      const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                      const int32_t* __restrict__ arr, uint2* __restrict__ pairs) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t k = keys[i];
@@ -476,9 +445,7 @@ __global__ void __launch_bounds__(kBlock) k_cs_rank(const uint2* __restrict__ pa
                                                      const int32_t* __restrict__ starts, uint32_t* __restrict__ sk,
                                                      int32_t* __restrict__ perm, const Real* __restrict__ pos,
                                                      const Real* __restrict__ rad, int dim,
-                                                     Real4<Real>* __restrict__ spos,
-                                                     const int32_t* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                     Real4<Real>* __restrict__ spos) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const uint2 me = pairs[j];
@@ -532,14 +499,13 @@ hipError_t cs_starts(const CellSort& cs, int64_t n_cells, int32_t* starts, hipSt
 }
 template <class Real>
 hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells, int32_t* starts,
-                     const Real* pos, const Real* rad, int dim, Real4<Real>* spos, hipStream_t s,
-                     const int32_t* gate) {
-  const hipError_t e = cs_starts(cs, n_cells, starts, s, gate);
+                     const Real* pos, const Real* rad, int dim, Real4<Real>* spos, hipStream_t s) {
+  const hipError_t e = cs_starts(cs, n_cells, starts, s, nullptr);
   if (e != hipSuccess) return e;
   if (n > 0) {
-    hipLaunchKernelGGL(k_cs_place, dim3(nblocks(n)), dim3(kBlock), 0, s, keys, n, starts, cs.arr, cs.pairs, gate);
+    hipLaunchKernelGGL(k_cs_place, dim3(nblocks(n)), dim3(kBlock), 0, s, keys, n, starts, cs.arr, cs.pairs);
     hipLaunchKernelGGL((k_cs_rank<Real>), dim3(nblocks(n)), dim3(kBlock), 0, s, cs.pairs, n, starts, cs.sk, cs.perm,
-                       pos, rad, dim, spos, gate);
+                       pos, rad, dim, spos);
   }
   return hipGetLastError();
 }
@@ -548,7 +514,7 @@ hipError_t cs_finish(const CellSort& cs, const uint32_t* keys, int64_t n, int64_
 // sorted keys there.  sb.k0 holds 2 n words, sb.v1 the arrival numbers until
 // the rank pass writes the ids there.
 hipError_t cell_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
-                          int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate) {
+                          int32_t** vals_out, int32_t* starts, hipStream_t s) {
   CellSort cs;
   cs.cnt = sb.cur;
   cs.arr = sb.v1;
@@ -558,10 +524,10 @@ hipError_t cell_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n
   cs.perm = sb.v1;
   hipError_t e = launch_fill_i32(cs.cnt, n_cells, 0, s);
   if (e != hipSuccess) return e;
-  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr, gate);
+  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr);
   *keys_out = cs.sk;
   *vals_out = cs.perm;
-  return cs_finish<float>(cs, keys_in, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s, gate);
+  return cs_finish<float>(cs, keys_in, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s);
 }
 
 // ---- counting sort with device-side counts (batch rebuilds) --------------
@@ -694,8 +660,8 @@ hipError_t cell_sort_begin(jdem_ctx* ctx, int64_t n, int64_t n_cells, CellSort* 
 template <class Real>
 hipError_t cell_sort_end_run(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                              int32_t* starts, const Real* pos, const Real* rad, int dim, Real4<Real>* spos,
-                             hipStream_t s, const int32_t* gate) {
-  const hipError_t e = cs_finish<Real>(cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, gate);
+                             hipStream_t s) {
+  const hipError_t e = cs_finish<Real>(cs, keys, n, n_cells, starts, pos, rad, dim, spos, s);
   ctx->cscnt_clear = e == hipSuccess;
   return e;
 }
@@ -706,28 +672,28 @@ hipError_t cell_sort_starts(jdem_ctx* ctx, const CellSort& cs, int64_t n_cells, 
   return e;
 }
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
-                         int32_t* starts, hipStream_t s, const int32_t* gate) {
-  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s, gate);
+                         int32_t* starts, hipStream_t s) {
+  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, nullptr, nullptr, 0, nullptr, s);
 }
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                          int32_t* starts, const float* pos, const float* rad, int dim, float4* spos, hipStream_t s) {
-  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, nullptr);
+  return cell_sort_end_run<float>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s);
 }
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                          int32_t* starts, const double* pos, const double* rad, int dim, Double4* spos,
                          hipStream_t s) {
-  return cell_sort_end_run<double>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s, nullptr);
+  return cell_sort_end_run<double>(ctx, cs, keys, n, n_cells, starts, pos, rad, dim, spos, s);
 }
 
 hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
-                           int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate) {
+                           int32_t** vals_out, int32_t* starts, hipStream_t s) {
   CellSort cs;
   const hipError_t e = cell_sort_begin(ctx, n, n_cells, &cs, s);
   if (e != hipSuccess) return e;
-  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr, gate);
+  if (n > 0) hipLaunchKernelGGL(k_cs_count, dim3(nblocks(n)), dim3(kBlock), 0, s, keys_in, n, cs.cnt, cs.arr);
   *keys_out = cs.sk;
   *vals_out = cs.perm;
-  return cell_sort_end(ctx, cs, keys_in, n, n_cells, starts, s, gate);
+  return cell_sort_end(ctx, cs, keys_in, n, n_cells, starts, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -93,7 +93,6 @@ struct jdem_ctx {
   // host bytes it was made from
   jdem::Buf route;
   std::vector<char> route_host;
-  // per-cell counts / starts of the batch rebuild's counting sort
   // clumps: members per clump (CSR), lab positions, levers, member totals
   jdem::Buf cl_start, cl_members, plab, ppr, ftot, ttot, crefl;
   // the precision form's Verlet list
@@ -275,41 +274,36 @@ size_t radix_hist_words(int64_t n);
 // uint32 words of SortBufs::hist that a counting sort over n_cells uses
 size_t cell_sort_sum_words(int64_t n_cells);
 // The sorts below on caller-given buffers (no allocation).
-// With n_dev the key count is read on the device (n bounds it and sizes the
-// launches); with gate every kernel returns at once while *gate == 0.
 hipError_t radix_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n, int nbits, uint32_t** keys_out,
-                           int32_t** vals_out, hipStream_t s, const int64_t* n_dev = nullptr,
-                           const int32_t* gate = nullptr);
+                           int32_t** vals_out, hipStream_t s);
 hipError_t cell_sort_bufs(const SortBufs& sb, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
-                          int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
+                          int32_t** vals_out, int32_t* starts, hipStream_t s);
 // Sort (keys, iota) by key; results in (keys_out, vals_out).  nbits = key bits.
 hipError_t radix_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int nbits, uint32_t** keys_out,
-                            int32_t** vals_out, hipStream_t s, const int64_t* n_dev = nullptr,
-                            const int32_t* gate = nullptr);
+                            int32_t** vals_out, hipStream_t s);
 // The same result as radix_sort_pairs for keys < n_cells, by counting:
 // per-cell counts, their exclusive scan (written to starts[0..n_cells],
 // starts[n_cells] = n), placement by arrival number, then each element's rank
-// among its cell's ids.  Cost grows with n + n_cells.  With gate, every kernel
-// of the sort returns at once while *gate == 0 (a device word), leaving the
-// previous sort's outputs in place.
+// among its cell's ids.  Cost grows with n + n_cells.
 // cell_sort_begin hands out the buffers (counts clear); a kernel of the caller
 // then writes each key, adds 1 to its cell's count and keeps the value the
 // atomic returned; cell_sort_end runs the remaining passes on those keys (and,
 // with spos, gathers the sorted (x, r)).
 hipError_t cell_sort_begin(jdem_ctx* ctx, int64_t n, int64_t n_cells, CellSort* cs, hipStream_t s);
 // cell_sort_starts only scans the counts into starts: the caller places its
-// elements itself.
+// elements itself.  Its kernels return at once while *gate == 0 (a device word),
+// leaving the previous starts in place.
 hipError_t cell_sort_starts(jdem_ctx* ctx, const CellSort& cs, int64_t n_cells, int32_t* starts, hipStream_t s,
                             const int32_t* gate);
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
-                         int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
+                         int32_t* starts, hipStream_t s);
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                          int32_t* starts, const float* pos, const float* rad, int dim, float4* spos, hipStream_t s);
 hipError_t cell_sort_end(jdem_ctx* ctx, const CellSort& cs, const uint32_t* keys, int64_t n, int64_t n_cells,
                          int32_t* starts, const double* pos, const double* rad, int dim, Double4* spos,
                          hipStream_t s);
 hipError_t cell_sort_pairs(jdem_ctx* ctx, const uint32_t* keys_in, int64_t n, int64_t n_cells, uint32_t** keys_out,
-                           int32_t** vals_out, int32_t* starts, hipStream_t s, const int32_t* gate = nullptr);
+                           int32_t** vals_out, int32_t* starts, hipStream_t s);
 // The counting sort of a batch rebuild, between cell_sort_begin and the
 // caller's rank pass: the first *n_dev of the keys (n bounds it), every key
 // below *c_dev (n_cells bounds it), starts of *c_dev + 1 entries, (key, id) at
@@ -335,9 +329,11 @@ inline int nbits_for_cells(int64_t n_cells) {
 int noalloc_init(int device);
 // whether cell_sort_pairs is the cheaper sort for n keys below n_cells
 inline bool use_cell_sort(int64_t n, int64_t n_cells) { return n > 0 && n_cells <= 4 * n + 65536; }
-// The same question where memory may be allocated: a cell costs 12 bytes of
-// traffic, the radix sort five launches per eight key bits, so the
-// counting sort stays ahead on grids far sparser than the particles.
+// The same question where memory may be allocated: a cell costs 16 bytes of
+// traffic against 4 with the radix sort, whose launches are two to five per
+// eight key bits, so the counting sort stays ahead on grids far sparser than the
+// particles (10^6 disks on 27 10^6 cells, five steps: 0.95 ms, 2.2 with the
+// radix sort and the cell ranges).
 inline bool use_cell_sort_sparse(int64_t n, int64_t n_cells) { return n > 0 && n_cells <= 32 * n + (1 << 20); }
 hipError_t launch_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 hipError_t launch_cell_ranges(const uint32_t* skeys, int64_t n, int32_t* cstart, int32_t* cend, hipStream_t s);
@@ -651,13 +647,10 @@ hipError_t ws_launch_permute(int64_t n, const int32_t* new_orig, const int32_t* 
                              const float4* V, const float4* W, const float4* Q, const float4* I, float4* P2,
                              float4* V2, float4* W2, float4* Q2, float4* I2, int32_t* orig2, int32_t* src,
                              int32_t* inv, hipStream_t s, float4* old2 = nullptr, int dim = 3);
-// batch rebuilds: per-system mode from the flags (and bump the build counts),
-// and the flags of never-built systems
-// With gate set, *events counts the calls that find *gate != 0 (rebuilds).
+// batch rebuilds, at the start of a call: the flags of never-built systems
+// (and *gate, when one is set)
 hipError_t ws_launch_seg_init_flags(int n_seg, const int32_t* n_build, int32_t* seg_flag, hipStream_t s,
                                    int32_t* gate = nullptr);
-// *gate = 0 (the end of a gated rebuild); *word = 0 when *gate is set
-
 hipError_t ws_launch_cell_starts(const uint32_t* skeys, int64_t n, int64_t n_cells, int32_t* starts, hipStream_t s);
 hipError_t ws_launch_nlist(const NLW& a, int dim, bool naive, hipStream_t s);
 hipError_t ws_launch_step(const WS& a, int dim, int law, hipStream_t s);

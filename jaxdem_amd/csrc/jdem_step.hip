@@ -1,9 +1,10 @@
 // jdem_step.hip -- (b) neighbour traversal with the pair laws and (c) the
 // fused integration of one DEM time step on gfx950.
 //
-// One thread owns one particle i and accumulates F_i and T_i in registers
-// over its candidates in the reference's traversal order -- no atomics, so
-// results are deterministic run to run.  The same kernel then applies
+// The candidates of particle i are walked by a group of lanes or, in large
+// systems, by one, a neighbour-list row always by one; F_i and T_i are summed
+// in the reference's traversal order either way -- no atomics, so results are
+// deterministic run to run.  The same kernel then applies
 // ForceManager, step_after_force of step k, and domain.apply +
 // step_before_force of step k+1 (system.py:60-82), writing positions and
 // velocities to the other half of a ping-pong pair because neighbours of
