@@ -819,8 +819,8 @@ __global__ void __launch_bounds__(kBlock) k_prec_force(PrecArgs a) {
 // (c_i - c_j) h is still exact in float32.  Partners are summed in the
 // list's order (the stencil order of the build).  The list is slot-major, so
 // a wavefront reads each of its slots in one piece; four entries and their
-// spheres are loaded before any is used.  2^18 spheres: 54 -> 25 us with the
-// partials of the reductions that were kernels of their own.
+// spheres are loaded before any is used.  2^18 spheres: 54 -> 19 us, now with
+// the partials of the reductions that were kernels of their own.
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_prec_vforce(PrecArgs a) {
   if (a.stop && *a.stop) return;

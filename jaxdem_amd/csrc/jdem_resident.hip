@@ -1681,7 +1681,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ws_wave
 // four, us: spring-friction, bidisperse 17 / 9.6 at 10 k, 17.6 / 10.8 at 37 k,
 // 18.5 / 13.3 at 70 k, 19.3 / 16.8 at 100 k, 24 / 26 at 200 k; log-normal radii
 // 19 / 12, 21 / 14, 21 / 18, 24 / 27.  Rows of disks are short: 8 / 7 below
-// 20 k, 8 / 8 at 37 k, 9.3 / 12.5 at 100 k, so one wave takes them all.
+// 20 k, 8 / 8 at 37 k, 9.3 / 12.5 at 100 k, so one wave takes them all.  Batches
+// of eight systems of unequal size: bidisperse 22 / 12 at 10 k, 21 / 14 at 37 k,
+// 19 / 15 at 79 k; log-normal 30 / 15, 30 / 17, 32 / 26.
 constexpr int64_t kWsSplit = 80000;
 
 template <int D, int LAW, int MW>
