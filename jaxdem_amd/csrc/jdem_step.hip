@@ -111,9 +111,9 @@ JD bool visit(const StepArgsT<Real>& a, const Side<D, Real>& me, int64_t i, int3
 // One lane per particle instead is a serial chain of dependent loads (27 cell
 // bounds, then the candidates one by one), and below ~10^5 particles there
 // are not even enough wavefronts to hide it.  Measured: the step kernel of
-// 1000 spheres with the naive collider 145 -> 17 us (a step of 30 k 5.1 -> 0.9
-// ms, of 64 as before), of 16 k spheres with the
-// cell list 61 -> 12 us, its energy kernel 58 -> 10 us.
+// 1000 spheres with the naive collider 145 -> 17 us (a step of 64 39 -> 23 us, of
+// 30 k 5.1 -> 0.9 ms), of 16 k spheres with the cell list 61 -> 12 us, its energy
+// kernel 58 -> 10 us.
 //
 // G: a 3D stencil holds about 40 candidates (27 cells of about 1.4), so 16
 // lanes take it in three rounds; a 2D one holds about 13, two rounds of 8.
