@@ -497,7 +497,8 @@ int build_cells(jdem_ctx* ctx, const Real* pos, const Real* rad, int64_t n, int 
 int ensure_flags(jdem_ctx* ctx) {
   ENSURE(ctx, ctx->flags, 64);
   if (!ctx->host_flags) {
-    if (hipHostMalloc((void**)&ctx->host_flags, 64, hipHostMallocDefault) != hipSuccess) {
+    // the words of flags, then room for a minimisation's state
+    if (hipHostMalloc((void**)&ctx->host_flags, 512, hipHostMallocDefault) != hipSuccess) {
       ctx->host_flags = nullptr;
       return fail(ctx, JDEM_ENOMEM, "pinned flag allocation failed");
     }
@@ -1994,12 +1995,10 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
 
   const bool listed = sys->collider_kind == JDEM_COLLIDER_NEIGHBOR_LIST && N > 0;
   bool stopped = false;  // seen by the list's check
-  if (listed) {
-    rc = ensure_flags(ctx);
-    if (rc) return rc;
-    f.stop_word = (int32_t*)ctx->flags.p + 8;
-    HIPCHK(ctx, launch_fill_i32(f.stop_word, 1, 0, st));
-  }
+  rc = ensure_flags(ctx);
+  if (rc) return rc;
+  f.stop_word = listed ? (int32_t*)ctx->flags.p + 8 : nullptr;
+  if (listed) HIPCHK(ctx, launch_fill_i32(f.stop_word, 1, 0, st));
 
   // eval_step (routines.py:228-245) and the next update's decision
   auto eval = [&]() -> int {
@@ -2039,8 +2038,12 @@ int jdem_minimize(jdem_ctx* ctx, jdem_system* sys, const jdem_fire* fire, int64_
   // a first chunk of four).  With a list every iteration sees the stop itself
   // (1558 us for the same call when it did not).
   for (int64_t done = 0;;) {
-    HIPCHK(ctx, hipMemcpyAsync(&h, dev, sizeof(h), hipMemcpyDeviceToHost, st));
+    // to pinned memory: a copy to the stack takes three times as long
+    static_assert(64 + sizeof(Dev) <= 512, "the pinned words hold the state");
+    void* host = ctx->host_flags + 16;
+    HIPCHK(ctx, hipMemcpyAsync(host, dev, sizeof(h), hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
+    std::memcpy(&h, host, sizeof(h));
     if (h.ls.stop) break;
     const int64_t first = std::min<int64_t>(4, std::max<int64_t>(1, done));
     const int64_t todo = std::min(max_steps - done, std::min<int64_t>(32, std::max<int64_t>(first, done / 4)));
