@@ -15,7 +15,7 @@
 // recomputes the forces of the final positions.  So the host reads the loop's
 // state once per chunk of iterations: with a read per iteration and a kernel
 // for each of these terms an iteration of 16 k spheres was 21 launches and
-// 130 us, bounded by them; now 10 and 66 us.  The chunks grow with the steps
+// 130 us, bounded by them; now 10 and 60 us.  The chunks grow with the steps
 // done (1, 1, 2, 4, then a quarter of them up to 32), so the evaluations past a
 // stop stay below half of those needed.  A neighbour list is checked by the
 // host before every evaluation anyway; the stop word comes with that read, and
